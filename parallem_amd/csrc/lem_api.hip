@@ -218,6 +218,8 @@ static void free_all(lemhip_ctx *c)
     if (c->hflags) (void)hipHostFree(c->hflags);
     if (c->stage) (void)hipHostFree(c->stage);
     if (c->hint) (void)hipHostFree(c->hint);
+    for (hipEvent_t e : c->dl_ev)
+        if (e) (void)hipEventDestroy(e);
     for (GraphSeg &g : c->gseg) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (g.graph) (void)hipGraphDestroy(g.graph);
@@ -612,6 +614,85 @@ static int rect_copy(lemhip_ctx *c, void *buf, void *base, int plane, size_t es,
     return LEMHIP_OK;
 }
 
+// Rows r0.. of rectangle D of a field, as the host receives them: row-major,
+// `ne` values per cell (8 for Slopes, direction-minor), widened to double, or
+// to int for codes and the mask (nodata cells carry -9999 in the reference's
+// fd/SFD, newflow.cu:74-78).
+// Bound by HBM (a cell's element read, its host element written).  Packing on
+// the device makes every download one contiguous copy: rows of an odd pitch
+// went through the strided copy's slow path (the directions of a 1201^2 DEM:
+// 18.8 ms, now 0.5 ms), and the conversions ran on one host thread.
+template <typename S, typename O>
+__global__ void __launch_bounds__(256) k_pack(int W, DemDesc D, int r0, long n, const S *__restrict__ src, long plane,
+                                              int ne, const uint8_t *__restrict__ mask, O *__restrict__ out)
+{
+    for (long k = blockIdx.x * (long)blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
+        const int row = (int)(k / D.w), col = (int)(k % D.w);
+        const long i = (long)(D.y0 + r0 + row) * W + D.x0 + col;
+        if constexpr (sizeof(O) == sizeof(int)) {
+            out[k] = !mask || mask[i] ? (O)src[i] : (O)-9999;
+        } else if constexpr (sizeof(S) == sizeof(float2) && !__is_same(S, double)) {
+            const float2 v = src[i];
+            out[k] = (double)v.x + (double)v.y;
+        } else {
+            for (int d = 0; d < ne; d++) out[ne * k + d] = (O)src[d * plane + i];
+        }
+    }
+}
+
+// Device staging to caller memory, on DL_THREADS threads, each taking every DL_THREADS-th chunk through its own two pinned
+// chunks: the next chunk's transfer overlaps the copy into the caller's pages
+// (one thread's page faults and copy took 10 of the 12.2 ms of a 134 MB field
+// and the transfer 2.5; now 4.0 ms, 12.1 ms for 459 MB; 1 to 4 MB chunks are
+// alike, 8 threads slower: 4.6 ms).  The pinned staging stays at 16 MB however
+// large the DEM.
+#define DL_CHUNK ((size_t)2 << 20)
+#define DL_DIRECT ((size_t)4 << 20)
+#define DL_THREADS 4
+static_assert(2 * DL_THREADS <= sizeof(lemhip_ctx::dl_ev) / sizeof(hipEvent_t), "one event per pinned chunk");
+static int copy_out(lemhip_ctx *c, const char *dev, char *host, size_t bytes)
+{
+    LEM_TRY(stage_reserve(c, 2 * (size_t)DL_THREADS * DL_CHUNK));
+    for (hipEvent_t &e : c->dl_ev)
+        if (!e) LEM_CHECK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    const size_t nch = (bytes + DL_CHUNK - 1) / DL_CHUNK, nt = std::min(nch, (size_t)DL_THREADS);
+    auto part = [=](size_t t) -> hipError_t {
+        hipError_t e = hipSetDevice(c->dev);
+        auto fetch = [&](size_t k, size_t buf) {   // chunk k into this thread's pinned chunk
+            if (e != hipSuccess || k >= nch) return;
+            const size_t off = k * DL_CHUNK, len = std::min((size_t)DL_CHUNK, bytes - off);
+            e = hipMemcpyAsync((char *)c->stage + buf * DL_CHUNK, dev + off, len, hipMemcpyDeviceToHost, c->s);
+            if (e == hipSuccess) e = hipEventRecord(c->dl_ev[buf], c->s);
+        };
+        fetch(t, 2 * t);
+        for (size_t k = t, j = 0; k < nch && e == hipSuccess; k += nt, j ^= 1) {
+            fetch(k + nt, 2 * t + (j ^ 1));
+            if (e == hipSuccess) e = hipEventSynchronize(c->dl_ev[2 * t + j]);
+            const size_t off = k * DL_CHUNK;
+            if (e == hipSuccess)
+                memcpy(host + off, (char *)c->stage + (2 * t + j) * DL_CHUNK, std::min((size_t)DL_CHUNK, bytes - off));
+        }
+        return e;
+    };
+    hipError_t rc[DL_THREADS] = {};
+    std::thread th[DL_THREADS];
+    bool inl[DL_THREADS] = {true};   // parts left to this thread: its own, and any no thread could be made for
+    for (size_t t = 1; t < nt; t++) {
+        try {
+            th[t] = std::thread([&, t] { rc[t] = part(t); });
+        } catch (...) {
+            inl[t] = true;
+        }
+    }
+    for (size_t t = 0; t < nt; t++)
+        if (inl[t]) rc[t] = part(t);
+    for (std::thread &t : th)
+        if (t.joinable()) t.join();
+    LEM_CHECK(c, hipStreamSynchronize(c->s));   // no transfer is left writing the pinned chunks
+    for (hipError_t e : rc) LEM_CHECK(c, e);
+    return LEMHIP_OK;
+}
+
 static int slot_download(lemhip_ctx *c, int slot, int field, void *host)
 {
     int kind = -1;
@@ -620,45 +701,45 @@ static int slot_download(lemhip_ctx *c, int slot, int field, void *host)
     DemDesc D;
     LEM_TRY(slot_rect(c, slot, 2, &D));
     LEM_CHECK(c, hipSetDevice(c->dev));
-    long n = (long)D.w * D.h;
-    size_t es = kind_elem(c, kind);
-    int planes = kind == 4 ? 8 : 1;
-    size_t bytes = planes * n * es + (kind == 2 ? n : 0);
-    LEM_TRY(stage_reserve(c, bytes));
-    for (int q = 0; q < planes; q++) LEM_TRY(rect_copy(c, c->stage, src, q, es, D, true));
-    uint8_t *mstage = (uint8_t *)c->stage + planes * n * es;
-    if (kind == 2) LEM_TRY(rect_copy(c, mstage, c->mask, 0, 1, D, true));
-    LEM_CHECK(c, hipStreamSynchronize(c->s));
-    if (kind == 1 || (kind == 0 && c->prec == LEMHIP_FP64) || (kind == 5 && c->prec == LEMHIP_FP64)) {
-        memcpy(host, c->stage, n * 8);
-    } else if (kind == 0) {
-        const float *s = (const float *)c->stage;
-        double *d = (double *)host;
-        for (long i = 0; i < n; i++) d[i] = s[i];
-    } else if (kind == 5) {
-        const float *s = (const float *)c->stage;
-        double *d = (double *)host;
-        for (long i = 0; i < n; i++) d[i] = (double)s[2 * i] + (double)s[2 * i + 1];
-    } else if (kind == 3) {
-        const uint8_t *s = (const uint8_t *)c->stage;
-        int *d = (int *)host;
-        for (long i = 0; i < n; i++) d[i] = s[i];
-    } else if (kind == 2) {
-        // nodata cells carry -9999 in the reference's fd/SFD (newflow.cu:74-78)
-        const uint8_t *s = (const uint8_t *)c->stage;
-        int *d = (int *)host;
-        for (long i = 0; i < n; i++) d[i] = mstage[i] ? (int)s[i] : -9999;
-    } else if (kind == 4) {
-        double *d = (double *)host;
-        if (c->prec == LEMHIP_FP64) {
-            const double *s = (const double *)c->stage;
-            for (int k = 0; k < 8; k++)
-                for (long i = 0; i < n; i++) d[8 * i + k] = s[k * n + i];
-        } else {
-            const float *s = (const float *)c->stage;
-            for (int k = 0; k < 8; k++)
-                for (long i = 0; i < n; i++) d[8 * i + k] = s[k * n + i];
+    const bool whole = kind == 2 || kind == 3, f64 = c->prec == LEMHIP_FP64;
+    const int ne = kind == 4 ? 8 : 1;
+    const size_t cell = whole ? sizeof(int) : ne * sizeof(double);
+    // up to DL_DIRECT bytes are packed straight into pinned host memory (a copy
+    // behind the kernel makes a 96^2 field's 17 us 28, a 512^2 one's 125 us 140).
+    // Otherwise the staging
+    // that initialised the slot holds 8 bytes per cell of its DEM, and Slopes
+    // go in bands of rows.
+    const size_t total = cell * D.w * D.h;
+    const bool direct = total <= DL_DIRECT;
+    int band = D.h;
+    if (direct) {
+        LEM_TRY(stage_reserve(c, total));
+    } else {
+        LEM_TRY(dstage_reserve(c, (size_t)D.w * D.h * 8));
+        band = (int)std::max((size_t)1, std::min((size_t)D.h, c->dstage_bytes / (cell * D.w)));
+        LEM_TRY(dstage_reserve(c, cell * D.w * band));
+    }
+    for (int r0 = 0; r0 < D.h; r0 += band) {
+        const int rows = std::min(band, D.h - r0);
+        const long n = (long)D.w * rows;
+        const int g = grid1d(n);
+        void *to = direct ? c->stage : c->dstage;
+        int *oi = (int *)to;
+        double *od = (double *)to;
+        if (whole) k_pack<uint8_t, int><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const uint8_t *)src, 0, 1,
+                                                            kind == 2 ? c->mask : nullptr, oi);
+        else if (kind == 5 && !f64) k_pack<float2, double><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const float2 *)src, 0,
+                                                                              1, nullptr, od);
+        else if (kind == 1 || f64) k_pack<double, double><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const double *)src,
+                                                                             c->NP, ne, nullptr, od);
+        else k_pack<float, double><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const float *)src, c->NP, ne, nullptr, od);
+        LEM_LAUNCHED(c);
+        if (!direct) {
+            LEM_TRY(copy_out(c, (const char *)c->dstage, (char *)host + (size_t)D.w * r0 * cell, n * cell));
+            continue;
         }
+        LEM_CHECK(c, hipStreamSynchronize(c->s));
+        memcpy(host, c->stage, total);
     }
     return LEMHIP_OK;
 }

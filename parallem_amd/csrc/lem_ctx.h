@@ -164,6 +164,7 @@ struct lemhip_ctx {
     LemScalars *hscal = nullptr;  // pinned host mirror
     void *stage = nullptr;        // pinned host staging for upload/download
     size_t stage_bytes = 0;
+    hipEvent_t dl_ev[16] = {};    // one per pinned chunk of a large download
     int *hint = nullptr;          // pinned host ints for small readbacks
 
     // counters known on the host after each phase
