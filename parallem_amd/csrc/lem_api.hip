@@ -204,7 +204,7 @@ static void free_all(lemhip_ctx *c)
                     c->z2, c->pl_tiles, c->pl_ctl, c->cub_tmp,
                     c->hkeys, c->hvals, c->elo, c->ehi, c->ew, c->rmm, c->seen, c->status, c->comp, c->cmax,
                     c->dmask, c->dag_list[0], c->dag_list[1], c->dag_list[2], c->dag_wake,
-                    c->dag_ctl, c->partials, c->scal, c->demid, c->ddesc, c->dsc, c->slot_flags, c->labdem,
+                    c->dag_ctl, c->res_ex, c->res_list, c->res_pos, c->res_ctl, c->partials, c->scal, c->demid, c->ddesc, c->dsc, c->slot_flags, c->labdem,
                     c->dstage, c->tcache, c->fx_shift, c->fx_tag_cell, c->fx_tag_sum, c->cs_rec};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
@@ -312,6 +312,13 @@ static int alloc_ctx(lemhip_ctx *c, const lem_params *p, int W, int H, int preci
     LEM_TRY(A((void **)&c->dag_wake, ntiles * 4));
     LEM_CHECK(c, hipMemset(c->dag_wake, 0, ntiles * 4));
     LEM_TRY(A(&c->dag_ctl, 512));
+    const long rt = ((W + LEM_RES_T - 1) / LEM_RES_T) * (long)((H + LEM_RES_T - 1) / LEM_RES_T);
+    c->res_cap = (int)std::min(rt, (long)LEM_RES_PER_CU * c->ncu);
+    LEM_TRY(A((void **)&c->res_ex, c->res_cap * LEM_RES_EDGE * 8L));
+    LEM_TRY(A((void **)&c->res_list, c->res_cap * 4L));
+    LEM_TRY(A((void **)&c->res_pos, rt * 4));
+    LEM_TRY(A(&c->res_ctl, LEM_RES_CTL));
+    LEM_CHECK(c, hipMemset(c->res_ctl, 0, LEM_RES_CTL));
     LEM_TRY(A((void **)&c->partials, 3L * SLOT_KB * (LEM_MAX_SLOTS + 1) * 8));
     LEM_TRY(A((void **)&c->fx_shift, sizeof(int) * (LEM_MAX_SLOTS + 1)));
     // tagged cells of the integer flow accumulation: one path per DEM (longer

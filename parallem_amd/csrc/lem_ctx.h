@@ -27,6 +27,12 @@ struct ProfSlot {
 #define PTW 48
 #define PTH 24
 
+// resident tiles of the dependency engine: side, edge entries, control block
+#define LEM_RES_T 32
+#define LEM_RES_EDGE 128
+#define LEM_RES_CTL 4352
+#define LEM_RES_PER_CU 7     // at most this many fit a compute unit's LDS
+
 // per-cell status of the dependency engine
 enum : uint8_t { ST_PENDING = 0, ST_DONE = 1, ST_DEAD = 2, ST_RING_WAIT = 3 };
 
@@ -131,6 +137,11 @@ struct lemhip_ctx {
     int *dag_list[3] = {nullptr, nullptr, nullptr};   // rotating lists of woken tiles
     int *dag_wake = nullptr;                          // per tile: last round it was queued for, DAG_TILE_DONE when finished
     void *dag_ctl = nullptr;
+    // resident tiles of the engine (the last launch of a pass)
+    unsigned long long *res_ex = nullptr;             // edge values per listed tile
+    int *res_list = nullptr, *res_pos = nullptr;      // listed tiles; each tile's place in the list
+    void *res_ctl = nullptr;
+    int res_cap = 0;                                  // tiles the buffers hold
     int dag_round = 0;
     int dag_rounds_last = 0;
     int plat_k = 8;             // plateau rounds per launch (4, 8 or 16)

@@ -12,6 +12,7 @@
 // it was written in an earlier launch (kernel boundary = visibility point).
 #include "lem_ctx.h"
 #include <string.h>
+#include <type_traits>
 
 #define DAG_TILE_DONE 0x7FFFFFFF   // wake stamp of a tile with no pending cell
 // status word: DAG_PENDING, r >= 0 done in round r (0 = before the first
@@ -130,6 +131,29 @@ __device__ __forceinline__ float2 fa_final(float w, float2 a) { return ff_add(ma
 //        the order E..NE of the reference (absent donors add nothing)
 //   finish(L, p, i, fin, upd)  HBM writes of a cell completed in this
 //        round, after the walks (coalesced, off the chains)
+//   word(L, p) / put(L, p, w)  the value a receiver in another tile reads, as
+//        one 64-bit word that is never EX_PENDING or EX_DEAD, and back into LDS
+#define EX_PENDING (~0ULL)
+#define EX_DEAD (~0ULL - 1)
+// a NaN with one of the two reserved payloads is handed on with another one
+__device__ __forceinline__ unsigned long long ex_word(double v)
+{
+    const unsigned long long w = (unsigned long long)__double_as_longlong(v);
+    return w >= EX_DEAD ? 0x7FF8000000000000ULL : w;
+}
+__device__ __forceinline__ unsigned long long ex_word(float2 v)
+{
+    const unsigned long long w = ((unsigned long long)__float_as_uint(v.y) << 32) | __float_as_uint(v.x);
+    return w >= EX_DEAD ? 0x7FC000007FC00000ULL : w;
+}
+__device__ __forceinline__ unsigned long long ex_word(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ void ex_value(unsigned long long w, double *v) { *v = __longlong_as_double((long long)w); }
+__device__ __forceinline__ void ex_value(unsigned long long w, float2 *v)
+{
+    *v = make_float2(__uint_as_float((unsigned)w), __uint_as_float((unsigned)(w >> 32)));
+}
+__device__ __forceinline__ void ex_value(unsigned long long w, float *v) { *v = __uint_as_float((unsigned)w); }
+
 template <typename T, int TW, int TH>
 struct FaCell {
     using FS = typename FaStore<T>::type;
@@ -139,6 +163,7 @@ struct FaCell {
     static constexpr int kWaves = 6;   // waves per SIMD the register budget is cut for
     const T *w;
     FS *fa;
+    template <int A, int B> FaCell<T, A, B> tiled() const { return {w, fa}; }
     struct Lds {
         FS val[NP];
         T w[NP];
@@ -162,20 +187,34 @@ struct FaCell {
     __device__ __forceinline__ void store_halo(Lds &L, int p, const HReg &r) const { L.val[p] = r; }
     // fa = w + max(0, sum of donor fa in the order E..NE) (mfd_simple.cu:71-168;
     // prop = 1 for every mask donor, runoffweight.cu:126-134, so fa*prop == fa)
+    // MANY: all eight neighbours read at once (cells of multiple flow
+    // directions have 3.5 donors on average)
+    template <bool MANY>
     __device__ __forceinline__ void compute(Lds &L, int p, unsigned bits, bool) const
     {
-        // one read per donor (chain cells mostly have one or two donors, and
-        // a compensated add costs more than the read)
         const T wv = L.w[p];
         FS accum{};
-        while (bits) {
-            const int k = __ffs(bits) - 1;
-            bits &= bits - 1;
-            fa_acc(accum, L.val[p + koff<TW>(k)]);
+        if constexpr (MANY) {
+            FS v8[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) v8[k] = L.val[p + poff<TW>(cpull(k))];
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+                if ((bits >> k) & 1u) fa_acc(accum, v8[k]);
+        } else {
+            // one read per donor (chain cells mostly have one or two donors, and
+            // a compensated add costs more than the read)
+            while (bits) {
+                const int k = __ffs(bits) - 1;
+                bits &= bits - 1;
+                fa_acc(accum, L.val[p + koff<TW>(k)]);
+            }
         }
         fa_clamp(accum);
         L.val[p] = fa_final(wv, accum);
     }
+    __device__ __forceinline__ unsigned long long word(const Lds &L, int p) const { return ex_word(L.val[p]); }
+    __device__ __forceinline__ void put(Lds &L, int p, unsigned long long w) const { ex_value(w, &L.val[p]); }
     __device__ __forceinline__ void finish(const Lds &L, int p, long i, const Fin &, bool) const { fa[i] = L.val[p]; }
 };
 
@@ -198,6 +237,10 @@ struct SedCell {
     const T *ero, *inci, *geli, *dps;
     T *depo, *stone, *fines;
     double *soilT;
+    template <int A, int B> SedCell<T, A, B> tiled() const
+    {
+        return {ero, inci, geli, dps, depo, stone, fines, soilT};
+    }
     struct Lds {
         T stone[NP];
         T a[NP], b[NP];
@@ -240,6 +283,7 @@ struct SedCell {
     // the reference sums all eight terms with zeros for absent donors; adding
     // only the donors' terms from +0 gives the same value up to the sign of a
     // zero sum, which the clamp below erases
+    template <bool MANY>
     __device__ __forceinline__ void compute(Lds &L, int p, unsigned bits, bool upd) const
     {
         if (!upd) return;
@@ -259,6 +303,8 @@ struct SedCell {
         else if (st > (T)99.9) st = (T)99.9;
         L.stone[p] = st;
     }
+    __device__ __forceinline__ unsigned long long word(const Lds &L, int p) const { return ex_word(L.stone[p]); }
+    __device__ __forceinline__ void put(Lds &L, int p, unsigned long long w) const { ex_value(w, &L.stone[p]); }
     __device__ __forceinline__ void finish(const Lds &L, int p, long i, const Fin &f, bool upd) const
     {
         depo[i] = f.dp;
@@ -691,7 +737,7 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_round(int W, int H, i
                     int rp0 = f ? cur + koff<TW>(__ffs(f) - 1) : cur;
                     uint32_t ns = ST_DEAD;
                     if (!dead) {
-                        cell.compute(lds, cur, (word >> 8) & 0xFFu, (word & W_UPD) != 0);
+                        cell.template compute<false>(lds, cur, (word >> 8) & 0xFFu, (word & W_UPD) != 0);
                         ns = ST_DONE;
                     }
                     wd[cur] = (word & ~(3u << W_STSH)) | (ns << W_STSH);
@@ -781,6 +827,422 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_round(int W, int H, i
     if (threadIdx.x == 0 && wg_prog) ctl->flag = 1;
 }
 
+// ---------------------------------------------------------- resident tiles
+//
+// Once the unfinished tiles fit the chip's LDS together, one launch finishes
+// the pass: each workgroup keeps one 32 x 32 tile in LDS until its last cell
+// is resolved, and tiles exchange the values of their edge cells while they
+// run.  Bound by the longest dependency path: its cells one after another
+// (0.6 us each under single flow directions, 0.8 to 1.2 under multiple) plus
+// a few us per tile crossing, instead of one launch per crossing, each as long
+// as its slowest visit (12-60 us).  Flow accumulation, launch rounds alone
+// against this: 512^2 FP64 0.56 -> 0.26 ms, under multiple directions
+// 5.7 -> 0.95 ms; 1133 x 739 FP32, multiple directions 19.2 -> 3.1 ms;
+// 4096^2 FP64 4.8 -> 3.4 ms (32 launch rounds, then 1511 resident tiles).
+//
+// Exchange: an entry per edge cell of every listed tile (top row, bottom row,
+// left column, right column; corners twice), EX_PENDING until the cell
+// resolves, then its value or EX_DEAD.  Entries are single 64-bit words
+// stored and polled with relaxed device-scope atomics: a word that is not
+// EX_PENDING is the final value by itself, so no ordering between different
+// addresses (and no fence between XCDs) is needed.
+//
+// End: a tile leaves when nothing is left to poll.  Cells on a cycle never
+// resolve, so a tile also leaves when it has waited RES_IDLE ticks in which no
+// tile at all made progress (every tile that resolves cells adds to one of 64
+// beat counters).  Leaving early, or a tile waiting for one that has not
+// started, costs time only: the host lists what is left and launches again
+// until a launch resolves nothing.
+#define RES_T 32
+#define RES_EDGE 128
+#define RES_BEATS 64
+#define RES_IDLE 3000          // 100 MHz ticks: 30 us
+struct ResCtl {    // LEM_RES_CTL bytes
+    int n;         // listed tiles
+    int left;      // cells still pending in them after the launch
+    int prog;      // some cell was resolved
+    int pad[13];
+    int beat[RES_BEATS * 16];   // one line each
+};
+static_assert(sizeof(ResCtl) <= LEM_RES_CTL && RES_EDGE == LEM_RES_EDGE && RES_T == LEM_RES_T, "resident buffers");
+
+// Tiles with a pending cell, in list; pos[tile]: its place there, or -1.  The
+// exchange entries of the first `cap` listed tiles are cleared.
+#define RES_LIST_TILES 4
+__global__ void __launch_bounds__(256) k_res_list(int W, int H, const int *__restrict__ st, int cap, int *list,
+                                                  int *pos, unsigned long long *ex, ResCtl *ctl)
+{
+    __shared__ int s_pend[RES_LIST_TILES], s_base;
+    const int ntx = (W + RES_T - 1) / RES_T, ntiles = ntx * ((H + RES_T - 1) / RES_T);
+    const int t0 = blockIdx.x * RES_LIST_TILES;
+    if (threadIdx.x < RES_LIST_TILES) s_pend[threadIdx.x] = 0;
+    int v[RES_LIST_TILES][4];
+#pragma unroll
+    for (int j = 0; j < RES_LIST_TILES; j++) {
+        const int t = t0 + j, tx0 = (t % ntx) * RES_T, ty0 = (t / ntx) * RES_T;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int li = threadIdx.x + q * 256;
+            const int r = ty0 + li / RES_T, c = tx0 + li % RES_T;
+            v[j][q] = t < ntiles && r < H && c < W ? st[(long)r * W + c] : 0;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RES_LIST_TILES; j++) {
+        const bool p = v[j][0] == DAG_PENDING || v[j][1] == DAG_PENDING || v[j][2] == DAG_PENDING ||
+                       v[j][3] == DAG_PENDING;
+        if (__any(p) && (threadIdx.x & 63) == 0) s_pend[j] = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int tot = 0;
+        for (int j = 0; j < RES_LIST_TILES; j++) tot += s_pend[j];
+        s_base = tot ? atomicAdd(&ctl->n, tot) : 0;
+    }
+    __syncthreads();
+    int at = s_base;
+    for (int j = 0; j < RES_LIST_TILES && t0 + j < ntiles; j++) {
+        if (threadIdx.x == 0) pos[t0 + j] = s_pend[j] ? at : -1;
+        if (!s_pend[j]) continue;
+        if (threadIdx.x == 0 && at < cap) list[at] = t0 + j;
+        if (at < cap && threadIdx.x < RES_EDGE) ex[(long)at * RES_EDGE + threadIdx.x] = EX_PENDING;
+        at++;
+    }
+}
+
+template <class Cell, bool SFD>
+__global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H, int round, Cell cell,
+                                                                    const uint8_t *__restrict__ dm,
+                                                                    const uint8_t *__restrict__ fdv,
+                                                                    int *__restrict__ st,
+                                                                    const int *__restrict__ list,
+                                                                    const int *__restrict__ pos,
+                                                                    unsigned long long *ex, ResCtl *ctl)
+{
+    constexpr int TW = RES_T, TH = RES_T, NC = TW * TH, PER = NC / 256, PW = TW + 2, NP = PW * (TH + 2);
+    constexpr int NH = 2 * PW + 2 * TH, RPER = (NH + 63) / 64;
+    __shared__ uint32_t wd[NP];      // packed words (W_*), padded layout; ring cells: state 3, fd bits
+    __shared__ uint8_t pst[NP];      // states at the start, as in k_dag_round
+    __shared__ typename Cell::Lds lds;
+    __shared__ uint16_t queue[NC];   // ready cells (each enters at most once)
+    __shared__ int qn, s_left, s_prog;
+    __shared__ int s_pos[9];
+    if ((int)blockIdx.x >= ctl->n) return;
+    const int tile = list[blockIdx.x];
+    const int ntx = (W + TW - 1) / TW, nty = (H + TH - 1) / TH;
+    const int tx0 = (tile % ntx) * TW, ty0 = (tile / ntx) * TH;
+    if (threadIdx.x == 0) { qn = 0; s_left = 0; s_prog = 0; }
+    if (threadIdx.x < 9) {
+        const int ty = tile / ntx + (int)threadIdx.x / 3 - 1, tx = tile % ntx + (int)threadIdx.x % 3 - 1;
+        s_pos[threadIdx.x] = ty >= 0 && ty < nty && tx >= 0 && tx < ntx ? pos[ty * ntx + tx] : -1;
+    }
+    // 1. the tile and its ring into LDS (k_dag_round, phase 1)
+    int vs[PER];
+    uint32_t vb[PER], vf[PER];   // 32-bit: byte registers would be packed, with a wait per load
+    typename Cell::Reg vr[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int r = ty0 + li / TW, c = tx0 + li % TW;
+        vs[q] = 0;
+        vb[q] = 0;
+        vf[q] = 0;
+        vr[q] = typename Cell::Reg{};
+        if (r < H && c < W) {
+            const long i = (long)r * W + c;
+            vs[q] = st[i];
+            vb[q] = dm[i];
+            vf[q] = fdv[i];
+            vr[q] = cell.load(i);
+        }
+    }
+    int hv = 0;
+    uint32_t hf = 0;
+    typename Cell::HReg hr = typename Cell::HReg{};
+    static_assert(NH <= 256, "one ring cell per thread");
+    int hp = 0;
+    if (threadIdx.x < NH) {
+        int nr, nc;
+        halo_pos<TW, TH>(threadIdx.x, &nr, &nc);
+        hp = pidx<TW>(nr, nc);
+        const int r = ty0 + nr, c = tx0 + nc;
+        if (r >= 0 && r < H && c >= 0 && c < W) {
+            const long i = (long)r * W + c;
+            hv = st[i];
+            hf = fdv[i];
+            hr = cell.load_halo(i);
+        }
+    }
+    typename Cell::Fin fin[PER];
+    uint32_t xw[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const uint32_t sv = (vs[q] == DAG_PENDING) ? ST_PENDING : (vs[q] >= 0 ? ST_DONE : ST_DEAD);
+        xw[q] = 0;
+        const int p = pidx<TW>(li / TW, li % TW);
+        fin[q] = cell.store(lds, p, vr[q], &xw[q]);
+        wd[p] = (sv << W_STSH) | (vf[q] << 16) | (vb[q] << 8) | W_NEVER;
+        pst[p] = (uint8_t)sv;
+    }
+    if (threadIdx.x < NH) {
+        // final only if resolved in an earlier launch; the rest is polled
+        uint8_t hs;
+        if (hv == DAG_PENDING) hs = ST_RING_WAIT;
+        else if (hv >= 0) hs = (hv < round) ? ST_DONE : ST_RING_WAIT;
+        else hs = ((-hv - 1) < round) ? ST_DEAD : ST_RING_WAIT;
+        pst[hp] = hs;
+        cell.store_halo(lds, hp, hr);
+        wd[hp] = (3u << W_STSH) | (hf << 16) | W_NEVER;
+    }
+    __syncthreads();
+    // 2. counters: donors unresolved in the tile or in its ring
+    uint32_t myw[PER];
+    int seeds = 0, pend0 = 0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        myw[q] = 0;
+        if (vs[q] != DAG_PENDING) continue;
+        pend0 |= 1 << q;
+        const int li = threadIdx.x + q * 256;
+        const int p = pidx<TW>(li / TW, li % TW);
+        const unsigned bits = vb[q];
+        uint32_t s8[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) s8[k] = pst[p + poff<TW>(cpull(k))];
+        int nin = 0;
+        uint32_t seen = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t oh = ((bits >> k) & 1u) << s8[k];
+            nin += (oh & ((1u << ST_PENDING) | (1u << ST_RING_WAIT))) ? 1 : 0;
+            seen |= oh;
+        }
+        const uint32_t base = ((uint32_t)ST_PENDING << W_STSH) | (vf[q] << 16) | (bits << 8) | xw[q];
+        if ((seen >> ST_DEAD) & 1u) { myw[q] = base | W_NEVER | W_DEAD1; seeds |= 1 << q; }
+        else { myw[q] = base | (uint32_t)nin; if (nin == 0) seeds |= 1 << q; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int p = pidx<TW>(li / TW, li % TW);
+        if ((pend0 >> q) & 1) wd[p] = myw[q];
+        const bool sd = (seeds >> q) & 1;
+        const unsigned long long m = __ballot(sd);
+        int base = 0;
+        if ((threadIdx.x & 63) == 0 && m) base = atomicAdd(&qn, __popcll(m));
+        base = __shfl(base, 0);
+        if (sd) queue[base + __popcll(m & ((1ULL << (threadIdx.x & 63)) - 1))] = (uint16_t)p;
+    }
+    __syncthreads();
+    // 3. one wave resolves cells in lockstep: LDS operations of one wave take
+    //    effect in the order issued, so a value written before the counter
+    //    add of the same step is there for whoever the add hands the cell to
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        const unsigned long long below = (1ULL << lane) - 1ULL;
+        unsigned long long *mine = ex + (long)blockIdx.x * RES_EDGE;
+        // ring cells this lane polls: padded index, exchange entry, receivers in the tile
+        int rp[RPER];
+        unsigned rf[RPER];
+        const unsigned long long *rx[RPER];
+        unsigned live = 0;
+#pragma unroll
+        for (int j = 0; j < RPER; j++) {
+            const int h = lane + 64 * j;
+            rp[j] = 0;
+            rf[j] = 0;
+            rx[j] = ex;
+            if (h >= NH) continue;
+            int nr, nc;
+            halo_pos<TW, TH>(h, &nr, &nc);
+            const int p = pidx<TW>(nr, nc);
+            if (pst[p] != ST_RING_WAIT) continue;
+            const unsigned f = (wd[p] >> 16) & 0xFFu;
+            unsigned in = 0;
+            for (int k = 0; k < 8; k++) {
+                const int d = cpull(k), r = nr + cdy(d), c = nc + cdx(d);
+                if (((f >> k) & 1u) && r >= 0 && r < TH && c >= 0 && c < TW) in |= 1u << k;
+            }
+            const int ty = nr < 0 ? 0 : (nr >= TH ? 2 : 1), tx = nc < 0 ? 0 : (nc >= TW ? 2 : 1);
+            const int np = s_pos[ty * 3 + tx];
+            if (!in || np < 0) continue;
+            const int rr = nr & (TH - 1), cc = nc & (TW - 1);   // place in its own tile
+            const int e = ty == 0 ? 32 + cc : (ty == 2 ? cc : (tx == 0 ? 96 + rr : 64 + rr));
+            rp[j] = p;
+            rf[j] = in;
+            rx[j] = ex + (long)np * RES_EDGE + e;
+            live |= 1u << j;
+        }
+        int head = 0, tail = qn;
+        int cur = -1;
+        uint32_t word = 0;
+        bool worked = false;                 // since the last poll
+        unsigned steps = 0;
+        bool idle = false;
+        unsigned long long t_idle = 0;
+        int beat0 = 0;
+        // the receivers of resolved cells, one bit of f per step in every
+        // lane: each lane keeps the first cell handed to it and queues the rest
+        auto hand_over = [&](int from, unsigned f, uint32_t delta, bool &out) {
+            while (__ballot(f != 0)) {
+                const bool on = f != 0;
+                const int r = on ? from + koff<TW>(__ffs(f) - 1) : from;
+                f &= f - 1;
+                uint32_t old = 0;
+                if (on) old = atomicAdd(&wd[r], delta);
+                out |= on && ((old >> W_STSH) & 3u) == 3u;
+                const bool ready = on && (old & W_CNT) == 1u;
+                const bool push = ready && cur >= 0;
+                if (ready && cur < 0) { cur = r; word = old + delta; }
+                const unsigned long long m = __ballot(push);
+                if (push) queue[tail + __popcll(m & below)] = (uint16_t)r;
+                tail += __popcll(m);
+            }
+        };
+        for (;;) {
+            if (head < tail) {
+                const unsigned long long m = __ballot(cur < 0);
+                const int rank = __popcll(m & below);
+                if (cur < 0 && rank < tail - head) {
+                    cur = queue[head + rank];
+                    word = wd[cur];
+                }
+                const int take = __popcll(m);
+                head += take < tail - head ? take : tail - head;
+            }
+            if (__ballot(cur >= 0)) {
+                // a beat every 16 steps, so that others do not leave while this
+                // tile works through a long stretch
+                if ((++steps & 15) == 0 && lane == 0)
+                    __hip_atomic_fetch_add(&ctl->beat[(blockIdx.x % RES_BEATS) * 16], 1, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                worked = true;
+                const bool on = cur >= 0;
+                const int p = cur;
+                const bool dead = on && Cell::kCanDie && ((word >> 24) & 0xFu) != 0;
+                unsigned f = on ? (word >> 16) & 0xFFu : 0u;
+                if (on) {
+                    if (!dead) cell.template compute<!SFD>(lds, p, (word >> 8) & 0xFFu, (word & W_UPD) != 0);
+                    wd[p] = (word & ~(3u << W_STSH)) | ((uint32_t)(dead ? ST_DEAD : ST_DONE) << W_STSH);
+                }
+                asm volatile("" ::: "memory");
+                cur = -1;
+                bool out = false;   // a receiver lies in another tile
+                const uint32_t delta = dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu;
+                if constexpr (SFD) {
+                    hand_over(p, f, delta, out);
+                } else {
+                    // all eight neighbours' adds in flight at once, 0 for those
+                    // that are no receivers; extra ready cells are queued after
+                    unsigned more = 0;
+                    if (on) {
+                        uint32_t old[8];
+#pragma unroll
+                        for (int k = 0; k < 8; k++)
+                            old[k] = atomicAdd(&wd[p + poff<TW>(cpull(k))], ((f >> k) & 1u) ? delta : 0u);
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            const bool rcv = (f >> k) & 1u;
+                            out |= rcv && ((old[k] >> W_STSH) & 3u) == 3u;
+                            if (!rcv || (old[k] & W_CNT) != 1u) continue;
+                            if (cur < 0) { cur = p + poff<TW>(cpull(k)); word = old[k] + delta; }
+                            else more |= 1u << k;
+                        }
+                    }
+                    while (__ballot(more != 0)) {
+                        const unsigned long long m = __ballot(more != 0);
+                        if (more) queue[tail + __popcll(m & below)] = (uint16_t)(p + koff<TW>(__ffs(more) - 1));
+                        more &= more - 1;
+                        tail += __popcll(m);
+                    }
+                }
+                if (out) {
+                    const unsigned long long v = dead ? EX_DEAD : cell.word(lds, p);
+                    const int lr = p / PW - 1, lc = p % PW - 1;
+                    auto put = [&](int e) {
+                        __hip_atomic_store(&mine[e], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    };
+                    if (lr == 0) put(lc);
+                    if (lr == TH - 1) put(32 + lc);
+                    if (lc == 0) put(64 + lr);
+                    if (lc == TW - 1) put(96 + lr);
+                }
+                continue;
+            }
+            if (!__ballot(live != 0)) break;
+            if (worked && lane == 0)
+                __hip_atomic_fetch_add(&ctl->beat[(blockIdx.x % RES_BEATS) * 16], 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            worked = false;
+            unsigned long long v[RPER];
+#pragma unroll
+            for (int j = 0; j < RPER; j++) {
+                v[j] = EX_PENDING;
+                if ((live >> j) & 1u) v[j] = __hip_atomic_load(rx[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            bool got = false;
+#pragma unroll
+            for (int j = 0; j < RPER; j++) {
+                const bool hit = v[j] != EX_PENDING;
+                const bool dead = Cell::kCanDie && v[j] == EX_DEAD;
+                if (hit) {
+                    live &= ~(1u << j);
+                    if (!dead) cell.put(lds, rp[j], v[j]);
+                }
+                asm volatile("" ::: "memory");
+                got |= hit;
+                bool out = false;
+                hand_over(rp[j], hit ? rf[j] : 0u, dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu, out);
+            }
+            if (__ballot(got)) {
+                idle = false;
+                continue;
+            }
+            // nothing new: leave once no tile has made progress for RES_IDLE ticks
+            const unsigned long long now = wall_clock64();
+            if (!idle || now - t_idle > RES_IDLE) {
+                const int b = __hip_atomic_load(&ctl->beat[lane % RES_BEATS * 16], __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+                if (idle && !__ballot(b != beat0)) break;
+                idle = true;
+                beat0 = b;
+                t_idle = now;
+            }
+        }
+    }
+    __syncthreads();
+    // 4. HBM writes of the cells resolved here, and what is left
+    int left = 0;
+    bool prog = false;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        if (!((pend0 >> q) & 1)) continue;
+        const int li = threadIdx.x + q * 256;
+        const int p = pidx<TW>(li / TW, li % TW);
+        const uint32_t wv = wd[p];
+        const uint32_t s2 = (wv >> W_STSH) & 3u;
+        if (s2 == ST_PENDING) { left++; continue; }
+        prog = true;
+        const long i = (long)(ty0 + li / TW) * W + (tx0 + li % TW);
+        if (s2 == ST_DONE) {
+            cell.finish(lds, p, i, fin[q], (wv & W_UPD) != 0);
+            st[i] = round;
+        } else {
+            st[i] = -(round + 1);
+        }
+    }
+    if (left) atomicAdd(&s_left, left);
+    if (prog) s_prog = 1;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_left) atomicAdd(&ctl->left, s_left);
+        if (s_prog) ctl->prog = 1;
+    }
+}
+
 __global__ void k_count_pending(long N, const uint8_t *mask, const int *st, int *out)
 {
     __shared__ int sh[256];
@@ -813,6 +1275,54 @@ __global__ void k_iota(int n, int *a)
     if (i < n) a[i] = i;
 }
 
+// Finishes the pass with resident tiles if the unfinished ones fit the chip
+// (*done = 1, the uncomputed cells in *uncomputed); *left: their number.  All
+// tiles fit: the launch takes the device's count and the host reads nothing
+// before it.
+template <class Cell, bool SFD>
+static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, int *done, int prof_slot)
+{
+    *done = 0;
+    const int ntiles = ((c->W + RES_T - 1) / RES_T) * ((c->H + RES_T - 1) / RES_T);
+    int bpc = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_dag_resident<Cell, SFD>, 256, 0) != hipSuccess || bpc < 1)
+        return LEMHIP_OK;
+    const int cap = bpc * c->ncu < c->res_cap ? bpc * c->ncu : c->res_cap;
+    int *st = reinterpret_cast<int *>(c->scan_tmp);
+    ResCtl *ctl = reinterpret_cast<ResCtl *>(c->res_ctl);
+    for (;;) {
+        LEM_CHECK(c, hipMemsetAsync(ctl, 0, 4 * sizeof(int), c->s));
+        k_res_list<<<(ntiles + RES_LIST_TILES - 1) / RES_LIST_TILES, 256, 0, c->s>>>(c->W, c->H, st, cap, c->res_list,
+                                                                                    c->res_pos, c->res_ex, ctl);
+        LEM_LAUNCHED(c);
+        int n = ntiles;
+        if (n > cap) {
+            LEM_CHECK(c, hipMemcpyAsync(&c->hint[40], &ctl->n, sizeof(int), hipMemcpyDeviceToHost, c->s));
+            LEM_CHECK(c, hipStreamSynchronize(c->s));
+            n = c->hint[40];
+            if (n > cap) return LEMHIP_OK;
+        }
+        ++*round;
+        prof_begin(c, prof_slot);
+        if (n > 0)
+            k_dag_resident<Cell, SFD><<<n, 256, 0, c->s>>>(c->W, c->H, *round, cell, c->dmask, c->fd, st,
+                                                           c->res_list, c->res_pos, c->res_ex, ctl);
+        prof_end(c, prof_slot, 1);
+        LEM_CHECK(c, hipMemsetAsync(&c->scal->flag, 0, sizeof(int), c->s));
+        k_count_pending<<<grid1d_dag(c->N), 256, 0, c->s>>>(c->N, c->mask, st, &c->scal->flag);
+        LEM_LAUNCHED(c);
+        LEM_CHECK(c, hipMemcpyAsync(&c->hint[40], ctl, 3 * sizeof(int), hipMemcpyDeviceToHost, c->s));
+        LEM_CHECK(c, hipMemcpyAsync(&c->hint[3], &c->scal->flag, sizeof(int), hipMemcpyDeviceToHost, c->s));
+        LEM_CHECK(c, hipStreamSynchronize(c->s));
+        // every launch that resolved a cell is followed by another unless
+        // nothing is left: at most one launch per cell
+        if (c->hint[41] == 0 || c->hint[42] == 0) break;
+    }
+    *uncomputed = c->hint[3];
+    *done = 1;
+    return LEMHIP_OK;
+}
+
 // first_rounds > 0: only that many rounds (the first visits every tile),
 // with no wait for the device; *uncomputed is not set
 template <int TW, int TH, class Cell, bool SFD>
@@ -824,6 +1334,17 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
     DagCtl *ctl = reinterpret_cast<DagCtl *>(c->dag_ctl);
     int r = c->dag_round;
     if (r > (1 << 29)) r = 0;   // status words hold round numbers
+    // few enough tiles for the chip: no launch rounds at all
+    constexpr int RT = RES_T;
+    const auto rcell = cell.template tiled<RT, RT>();
+    int done = 0;
+    if (first_rounds == 0 && ((c->W + RT - 1) / RT) * ((c->H + RT - 1) / RT) <= c->res_cap) {
+        const int r0 = r;
+        LEM_TRY((run_resident<std::remove_const_t<decltype(rcell)>, SFD>(c, rcell, &r, uncomputed, &done, prof_slot)));
+        c->dag_rounds_last = r - r0;
+        c->dag_round = r;
+        if (done) return LEMHIP_OK;
+    }
     // wake stamps start below every round number of the pass
     LEM_CHECK(c, hipMemsetAsync(c->dag_wake, 0, sizeof(int) * ntiles, c->s));
     // the first round visits every tile
@@ -866,6 +1387,12 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
         LEM_CHECK(c, hipMemcpyAsync(&c->hint[20], &ctl->flag, sizeof(int), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipStreamSynchronize(c->s));
         if (!c->hint[20]) break;
+        LEM_TRY((run_resident<std::remove_const_t<decltype(rcell)>, SFD>(c, rcell, &r, uncomputed, &done, prof_slot)));
+        if (done) {
+            c->dag_rounds_last = r - c->dag_round;
+            c->dag_round = r;
+            return LEMHIP_OK;
+        }
         guard += 1;  // batches that made progress; each completes at least one cell
         if (guard > c->N + 2) { c->err = "dependency rounds did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
