@@ -144,7 +144,8 @@ struct lemhip_ctx {
     int res_cap = 0;                                  // tiles the buffers hold
     int dag_round = 0;
     int dag_rounds_last = 0;
-    int plat_k = 8;             // plateau rounds per launch (4, 8 or 16)
+    int plat_k = 8;             // plateau rounds per launch (4, 8 or 16; 8: 16 once few tiles move)
+    int plat_grid[2][2] = {};   // workgroups of the plateau kernels (plat_grids)
     // lemhip_autotune sets both; each tuner clears its own flag once it has run
     bool tune_dag_pending = false;    // the next pass on the engine times tile shapes and batches
     bool tune_plat_pending = false;   // the next plateau pass on a raised surface times rounds per launch

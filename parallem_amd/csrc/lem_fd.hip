@@ -402,10 +402,12 @@ __global__ void k_plat_first_list(int ntiles, const int *tile_has, int *list, Pl
     }
 }
 
-// threads per plateau workgroup: a launch near the end of the pass visits a
-// few tiles, each in K synchronised rounds over its region, so the rounds
-// are spread over many threads
-#define PLAT_NT 512
+// threads per plateau workgroup: a launch near the end of the pass (16 rounds)
+// visits a few tiles, so its rounds are spread over all the waves a workgroup
+// can have (512^2 DEM, pass on the filled surface: 0.19 ms against 0.22 with
+// 512 threads); with many tiles moving 512 threads hold more tiles at once
+// (4096^2: 1.97 ms, 2.22 with 1024)
+#define PLAT_NT(K) ((K) == 16 ? 1024 : 512)
 
 // Distances live in two buffers per tile: tver[tile] = 2 * (launch that last
 // wrote the tile) + (buffer it wrote).  A launch reads every tile from the
@@ -441,9 +443,23 @@ __device__ __forceinline__ void plat_flush(int *qbuf, int *qn, int *next, int *c
 
 // MARKS: the pass records slope marks (the first pass, on the dem; the pass
 // on the raised surface keeps only directions and distances)
+//
+// A visit is bound by the latency of its K rounds: 12.4 of a tail visit's
+// 17 us when every cell was evaluated in every round.  In a round only the
+// cells next to a change of the round before can change: a front a few cells
+// wide.  The region is therefore cut into 8 x 8 blocks, one wave evaluates a
+// block at a time, and a block is evaluated only when it or the adjacent edge
+// of a neighbour block changed in the last round (a front of any orientation
+// meets about a quarter of the blocks); a wave reads the stamps of all its
+// blocks at once, a cell its neighbours, and one flag tells whether the last
+// round changed anything.  5.6 us of 11 for 8 rounds, and the first launch over
+// a 4096^2 DEM 245 -> 182 us; the pass 3.05 -> 1.97 ms, on 1201^2 0.93 -> 0.57.
+// Blocks are dealt to the waves so that a row or column of them falls on
+// different waves; the LDS pitch is an odd number of 8-cell groups, so a
+// block's rows lie in different banks.
 template <int K, typename TS, bool MARKS>
-__global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch, int r0, const int *__restrict__ act,
-                                                    int *__restrict__ next, float *__restrict__ sp0,
+__global__ void __launch_bounds__(PLAT_NT(K), K == 16 ? 4 : 6) k_plat_block(int W, int H, int launch, int r0,
+                                                    int kn, const int *__restrict__ act, int *__restrict__ next, float *__restrict__ sp0,
                                                     float *__restrict__ sp1, int *__restrict__ tver,
                                                     const uint8_t *__restrict__ eqb,
                                                     uint8_t *__restrict__ fd, uint8_t *__restrict__ SFD,
@@ -452,21 +468,44 @@ __global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch
                                                     PlatCtl *ctl)
 {
     constexpr int RW = PTW + 2 * K, RH = PTH + 2 * K, RN = RW * RH, NI = PTW * PTH;
-    constexpr int PER = (RN + PLAT_NT - 1) / PLAT_NT, PERI = (NI + PLAT_NT - 1) / PLAT_NT;
-    static_assert(PER <= 32, "region too large for the per-thread cell mask");
-    __shared__ float A[RN], B[RN];
-    __shared__ uint8_t E[RN];
+    constexpr int NT = PLAT_NT(K), PER = (RN + NT - 1) / NT, PERI = (NI + NT - 1) / NT;
+    constexpr int NBX = RW / 8, NBY = RH / 8, NB = NBX * NBY, NW = NT / 64, BPW = (NB + NW - 1) / NW;
+    constexpr int P = (NBX & 1) ? RW : RW + 8, LN = P * RH;   // LDS pitch
+    constexpr int G = P + 1;                                  // guard: every cell's neighbours can be read
+    constexpr int SX = NBX + 2;                               // pitch of the block stamps (a ring of unused ones)
+    static_assert(RW % 8 == 0 && RH % 8 == 0 && (NW & (NW - 1)) == 0, "8 x 8 blocks dealt to the waves");
+    __shared__ uint32_t bufA[LN + 2 * G], bufB[LN + 2 * G];   // distances as bits: none is negative, so they order as unsigned
+    // equal-height bits, and above them the distance from the region's edge: a
+    // cell is current after round k when that is at least k (0: never changes)
+    __shared__ uint16_t E[LN];
     __shared__ uint8_t code[NI], marks[NI];
+    __shared__ uint8_t stamp[2][SX * (NBY + 2)];   // by round parity: the last round the block is due in
+    __shared__ int s_any[K + 1];   // some cell changed in that round
     __shared__ int last;
-    __shared__ int s_qmask;   // 3x3 tiles within K cells of a cell that changed in round K
-    __shared__ int s_buf[9];
+    __shared__ int s_qmask;   // 3x3 tiles within kn cells of a cell that changed in round K
+    __shared__ int s_buf[9], s_has[9];
     __shared__ int qbuf[PLAT_QCAP];   // tiles queued for the next launch, not yet appended
     __shared__ int qn;
     int wg_last = 0;                  // thread 0: the last round with a change in this workgroup's visits
+    uint32_t *const A = bufA + G, *const B = bufB + G;
     if (threadIdx.x == 0) qn = 0;
     const int n = ctl->cnt[launch % 3];
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl->cnt[(launch + 2) % 3] = 0;
     const int ntx = (W + PTW - 1) / PTW, nty = (H + PTH - 1) / PTH;
+    // the cell of a block this lane evaluates, and (lanes 0-8) the neighbour
+    // block it stamps with the cells of a block that are adjacent to it
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int ly = lane >> 3, lx = lane & 7;
+    const int wy = lane / 3 - 1, wx = lane % 3 - 1;
+    unsigned long long adj = ~0ULL;
+    if (wy < 0) adj &= 0xFFULL;
+    if (wy > 0) adj &= 0xFFULL << 56;
+    if (wx < 0) adj &= 0x0101010101010101ULL;
+    if (wx > 0) adj &= 0x8080808080808080ULL;
+    if (lane >= 9) adj = 0;
+    // block `lane` of this wave's (lanes below BPW): its stamp
+    const int myb = lane * NW + ((wave - 3 * lane) & (NW - 1));
+    const int mys = lane < BPW && myb < NB ? (myb / NBX + 1) * SX + myb % NBX + 1 : -1;
     // the next visit's tile is read during this one (the first together with
     // the count: the grid never exceeds the list's capacity, and an entry
     // past the count is never used)
@@ -477,6 +516,8 @@ __global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch
         const int tx0 = (tile % ntx) * PTW, ty0 = (tile / ntx) * PTH;
         __syncthreads();
         if (threadIdx.x == 0) { last = 0; s_qmask = 0; }
+        if (threadIdx.x < 2 * SX * (NBY + 2)) stamp[0][threadIdx.x] = 0;   // both parities
+        if (threadIdx.x <= K) s_any[threadIdx.x] = 0;
         // load the region from both distance buffers, and in the same wait
         // which buffer holds each of the 3x3 tiles as of the last launch: the
         // region's loads do not wait for that choice (a visit of the first
@@ -486,7 +527,7 @@ __global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch
         int part[PER];   // 3x3 tile of the region cell, -1 off the grid
 #pragma unroll
         for (int q = 0; q < PER; q++) {
-            int idx = threadIdx.x + q * PLAT_NT;
+            int idx = threadIdx.x + q * NT;
             int gy = ty0 - K + idx / RW, gx = tx0 - K + idx % RW;
             v0[q] = 0.f;
             v1[q] = 0.f;
@@ -503,87 +544,117 @@ __global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch
         }
         if (threadIdx.x < 9) {
             int ty = tile / ntx + (int)threadIdx.x / 3 - 1, tx = tile % ntx + (int)threadIdx.x % 3 - 1;
-            s_buf[threadIdx.x] = (ty >= 0 && ty < nty && tx >= 0 && tx < ntx) ? plat_buf_as_of(tver[ty * ntx + tx], launch) : 0;
+            const bool in = ty >= 0 && ty < nty && tx >= 0 && tx < ntx;
+            const int tv = in ? tver[ty * ntx + tx] : 0;
+            s_has[threadIdx.x] = in ? tile_has[ty * ntx + tx] : 0;
+            s_buf[threadIdx.x] = in ? plat_buf_as_of(tv, launch) : 0;
         }
         __syncthreads();
         // both LDS buffers hold every cell, so cells that cannot change (no
         // candidate, or no equal-height neighbour) are never rewritten
-        unsigned own = 0;
-        float v[PER];
-#pragma unroll
-        for (int q = 0; q < PER; q++) v[q] = part[q] < 0 ? 0.f : (s_buf[part[q]] ? v1[q] : v0[q]);
 #pragma unroll
         for (int q = 0; q < PER; q++) {
-            int idx = threadIdx.x + q * PLAT_NT;
+            const int idx = threadIdx.x + q * NT;
+            const float v = part[q] < 0 ? 0.f : (s_buf[part[q]] ? v1[q] : v0[q]);
             if (idx < RN) {
-                A[idx] = v[q];
-                B[idx] = v[q];
-                E[idx] = e[q];
-                if (v[q] != 0.f && e[q] != 0) own |= 1u << q;
+                const int rr = idx / RW, cc = idx % RW, li = rr * P + cc;
+                const int dy = rr < RH - 1 - rr ? rr : RH - 1 - rr, dx = cc < RW - 1 - cc ? cc : RW - 1 - cc;
+                A[li] = __float_as_uint(v);
+                B[li] = __float_as_uint(v);
+                E[li] = v != 0.f && e[q] != 0 ? (uint16_t)(e[q] | ((dy < dx ? dy : dx) << 8)) : 0;
             }
         }
 #pragma unroll
         for (int q = 0; q < PERI; q++) {
-            int li = threadIdx.x + q * PLAT_NT;
+            int li = threadIdx.x + q * NT;
             if (li < NI) { code[li] = 0; marks[li] = 0; }
         }
         __syncthreads();
-        float *cur = A, *nxt = B;
+        uint32_t *cur = A, *nxt = B;
         int moved = 0;   // last round in which one of this thread's tile cells changed
-        unsigned qm = 0;  // 3x3 tiles within K cells of this thread's cells that changed in round K
+        unsigned qm = 0;  // 3x3 tiles within kn cells of this thread's cells that changed in round K
         // A round in which no cell of its window changes leaves every later
         // round unchanged too (round k+1 reads only round k values of a window
-        // that contains its own), so the launch stops there.
+        // that contains its own), so the launch stops there.  A block not due
+        // in round k did not change in round k-1, so both buffers hold it.
         for (int k = 1; k <= K; k++) {
+            // the blocks due of this wave, one bit each, and whether the last
+            // round changed anything: one LDS wait
+            unsigned due = (1u << BPW) - 1;
+            if (k > 1) {
+                const int st = mys >= 0 ? stamp[k & 1][mys] : 0;
+                const int any = s_any[k - 1];
+                if (!any) break;
+                due = (unsigned)__ballot(st == k);
+            }
             bool changed = false;
+            while (due) {
+                const int j = __ffs(due) - 1;
+                due &= due - 1;
+                const int blk = j * NW + ((wave - 3 * j) & (NW - 1)), by = blk / NBX, bx = blk - by * NBX;
+                if (NB % NW && blk >= NB) continue;
+                // every read of the cell in flight at once (lanes whose cell
+                // is not current read within the guard and discard)
+                const int b = (by * 8 + ly) * P + bx * 8 + lx;
+                const uint32_t ee = E[b], md0 = cur[b];
+                uint32_t c[8];
 #pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int idx = threadIdx.x + q * PLAT_NT;
-                const int rr = idx / RW, cc = idx % RW;
-                const bool act = ((own >> q) & 1) && rr >= k && rr < RH - k && cc >= k && cc < RW - k;
-                if (!act) continue;
-                // the scan N..NW without branches
-                const int b = idx;
-                float md = cur[b];
-                const unsigned ee = E[b];   // read per round: keeps 8 lane masks per cell out of the registers
-                unsigned cd = 0, mk = 0;
+                for (int d = 0; d < 8; d++) c[d] = cur[b + cdy(d) * P + cdx(d)];
+                const int dep = (int)(ee >> 8);
+                // the scan N..NW takes the smallest distance below the cell's
+                // own, the first direction that has it; directions without an
+                // equal-height neighbour count as beyond every distance
+                uint32_t m = ~0u;
 #pragma unroll
                 for (int d = 0; d < 8; d++) {
-                    const float dc = (d & 1) ? 1.41f : 1.0f;
-                    const float dis = cur[b + cdy(d) * RW + cdx(d)] + dc;
-                    const bool take = ((ee >> d) & 1u) && (md > dis);
-                    md = take ? dis : md;
-                    cd = take ? (1u << ((d + 6) & 7)) : cd;   // fd code of direction d
-                    if (MARKS) mk |= take ? (1u << d) : 0u;
+                    const float dis = __uint_as_float(c[d]) + ((d & 1) ? 1.41f : 1.0f);
+                    c[d] = __float_as_uint(dis) | (uint32_t)((int)(~ee << (31 - d)) >> 31);
+                    m = c[d] < m ? c[d] : m;
                 }
-                nxt[idx] = md;
-                changed |= cd != 0;
-                if (cd && rr >= K && rr < K + PTH && cc >= K && cc < K + PTW) {
-                    int li = (rr - K) * PTW + (cc - K);
-                    code[li] = (uint8_t)cd;
-                    if (MARKS) marks[li] |= (uint8_t)mk;
+                const bool on = dep >= k, ch = on && m < md0;
+                if (on) nxt[b] = ch ? m : md0;
+                const unsigned long long M = __ballot(ch);
+                if (!M) continue;
+                changed = true;
+                if (M & adj) stamp[(k + 1) & 1][(by + 1) * SX + bx + 1 + wy * SX + wx] = (uint8_t)(k + 1);
+                if (ch && dep >= K) {   // a changed cell of the tile
+                    unsigned cd = 0;
+#pragma unroll
+                    for (int d = 7; d >= 0; d--) cd = c[d] == m ? (1u << ((d + 6) & 7)) : cd;   // fd code of direction d
+                    const int ty = by * 8 + ly - K, tx = bx * 8 + lx - K;
+                    code[ty * PTW + tx] = (uint8_t)cd;
+                    if (MARKS) {
+                        uint32_t md = md0;
+                        unsigned mk = 0;
+#pragma unroll
+                        for (int d = 0; d < 8; d++) {
+                            const bool take = c[d] < md;
+                            md = take ? c[d] : md;
+                            mk |= take ? (1u << d) : 0u;
+                        }
+                        marks[ty * PTW + tx] |= (uint8_t)mk;
+                    }
                     moved = k;
                     if (k == K) {
-                        const int ly = rr - K, lx = cc - K;
-                        const unsigned rows = 2u | (ly < K ? 1u : 0u) | (ly >= PTH - K ? 4u : 0u);
-                        const unsigned cols = 2u | (lx < K ? 1u : 0u) | (lx >= PTW - K ? 4u : 0u);
+                        const unsigned rows = 2u | (ty < kn ? 1u : 0u) | (ty >= PTH - kn ? 4u : 0u);
+                        const unsigned cols = 2u | (tx < kn ? 1u : 0u) | (tx >= PTW - kn ? 4u : 0u);
 #pragma unroll
                         for (int ny = 0; ny < 3; ny++)
                             if ((rows >> ny) & 1u) qm |= cols << (3 * ny);
                     }
                 }
             }
-            const int any = __syncthreads_or(changed);
-            float *t = cur; cur = nxt; nxt = t;
-            if (!any) break;
+            if (changed) s_any[k] = 1;
+            __syncthreads();
+            uint32_t *t = cur; cur = nxt; nxt = t;
         }
         if (moved) atomicMax(&last, moved);
         if (qm) atomicOr(&s_qmask, (int)qm);
         __syncthreads();
         // still moving at the end of the launch: this tile and the neighbours
-        // within K cells of a cell that changed in the last round go on (a
+        // within kn cells of a cell that changed in the last round go on (a
         // cell changing in round K + j lies within j cells of one that changed
-        // in round K), gathered in LDS and appended to the next list with one
+        // in round K, and the next launch takes at most kn rounds), gathered in LDS and appended to the next list with one
         // atomic per full buffer (workgroups adding to one counter serialise).
         // Before the write-back: the wait for the atomic's returned value
         // would otherwise also wait for those stores
@@ -591,7 +662,7 @@ __global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch
             int ty = tile / ntx + (int)threadIdx.x / 3 - 1, tx = tile % ntx + (int)threadIdx.x % 3 - 1;
             if (ty >= 0 && ty < nty && tx >= 0 && tx < ntx) {
                 const int t2 = ty * ntx + tx;
-                if (tile_has[t2] && atomicExch(&tstamp[t2], launch + 1) != launch + 1) qbuf[atomicAdd(&qn, 1)] = t2;
+                if (s_has[threadIdx.x] && atomicExch(&tstamp[t2], launch + 1) != launch + 1) qbuf[atomicAdd(&qn, 1)] = t2;
             }
         }
         // write back the tile: distances (into its other buffer), directions of
@@ -599,11 +670,11 @@ __global__ void __launch_bounds__(PLAT_NT) k_plat_block(int W, int H, int launch
         float *sp_out = s_buf[4] ? sp0 : sp1;
 #pragma unroll
         for (int q = 0; q < PERI; q++) {
-            int li = threadIdx.x + q * PLAT_NT;
+            int li = threadIdx.x + q * NT;
             int gy = ty0 + li / PTW, gx = tx0 + li % PTW;
             if (li >= NI || gy >= H || gx >= W) continue;
             long i = (long)gy * W + gx;
-            sp_out[i] = cur[(li / PTW + K) * RW + (li % PTW + K)];
+            sp_out[i] = __uint_as_float(cur[(li / PTW + K) * P + (li % PTW + K)]);
             uint8_t cd = code[li];
             if (cd) { fd[i] = cd; SFD[i] = cd; }
             if (MARKS && marks[li]) {
@@ -1303,6 +1374,22 @@ static int read_flag(lemhip_ctx *c, int *v)
     return LEMHIP_OK;
 }
 
+// workgroups the chip holds of each plateau kernel a context uses: fewer than
+// 16 rounds per launch and 16, without and with slope marks
+template <typename TS>
+static int plat_grids(lemhip_ctx *c)
+{
+    const void *f[2][2] = {{(const void *)k_plat_block<8, TS, false>, (const void *)k_plat_block<8, TS, true>},
+                           {(const void *)k_plat_block<16, TS, false>, (const void *)k_plat_block<16, TS, true>}};
+    for (int q = 0; q < 2; q++)
+        for (int m = 0; m < 2; m++) {
+            int bpc = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, f[q][m], q ? PLAT_NT(16) : PLAT_NT(8), 0) != hipSuccess || bpc < 1) bpc = 1;
+            c->plat_grid[q][m] = bpc * c->ncu;
+        }
+    return LEMHIP_OK;
+}
+
 // FlowDirs + plateau routing on surface zs; slopes == nullptr for pass 2.
 // Leaves the candidate list in c->cand and its length in *ncand_out; returns
 // the number of rounds that changed something in *rounds.
@@ -1345,46 +1432,54 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
     k_sp_seedmark<<<grid1d(n, 256, 1 << 30), 256, 0, c->s>>>(W, H, c->cand, n, sp_in, eqb, ntx, nty, tile_has);
     k_plat_first_list<<<grid1d(ntiles, 256, 1024), 256, 0, c->s>>>(ntiles, tile_has, L[launch % 3], ctl, launch % 3);
     LEM_LAUNCHED(c);
-    int bpc = 0;
-    hipError_t oe = hipSuccess;
-    switch (c->plat_k) {
-    case 4: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_plat_block<4, TS, false>, PLAT_NT, 0); break;
-    case 16: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_plat_block<16, TS, false>, PLAT_NT, 0); break;
-    default: oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_plat_block<8, TS, false>, PLAT_NT, 0); break;
+    // Eight rounds per launch while many tiles move (with 16 throughout, the
+    // wider halo makes the pass 2.9 instead of 2.0 ms on 4096^2), 16 once they
+    // are no more than the compute units, where a launch costs about 9 us
+    // whatever it does (8 throughout: 2.17 ms on 4096^2, 0.68 instead of 0.57
+    // on 1201^2).  The last launch of a
+    // batch queues the tiles a launch of 16 rounds could reach.
+    const bool widen = c->plat_k == 8;
+    int K = widen && ntiles <= c->ncu ? 16 : c->plat_k;
+    int G[2] = {c->plat_grid[0][slopes ? 1 : 0], c->plat_grid[1][slopes ? 1 : 0]};   // of K < 16 and K = 16
+    if (!G[0]) {
+        LEM_TRY(plat_grids<TS>(c));
+        for (int q = 0; q < 2; q++) G[q] = c->plat_grid[q][slopes ? 1 : 0];
     }
-    if (oe != hipSuccess || bpc < 1) bpc = 1;
-    int G = bpc * c->ncu;
-    if (G > ntiles) G = ntiles;
-    const int BATCH = 16;   // launches between host checks (an empty launch costs less than a read)
     int r = 0;  // rounds done in this pass
     long guard = 0;
-    for (;;) {
+    // launches between host checks (an empty launch costs less than a read);
+    // the first pass seldom has a flat to drain
+    for (int batch = slopes ? 4 : 128 / K;; batch = 128 / K) {
         prof_begin(c, PROF_PLAT_K);
-        for (int q = 0; q < BATCH; q++) {
+        for (int q = 0; q < batch; q++) {
             const int *a_cur = L[launch % 3];
             int *a_next = L[(launch + 1) % 3];
-            switch (c->plat_k) {
+            const int grid = G[K == 16] < ntiles ? G[K == 16] : ntiles;
+            const int kn = q == batch - 1 && widen ? 16 : K;
+            switch (K) {
 #define PLAT_LAUNCH(K)                                                                                           \
     if (slopes)                                                                                                  \
-        k_plat_block<K, TS, true><<<G, PLAT_NT, 0, c->s>>>(W, H, launch, r, a_cur, a_next, sp_in, sp_out, tver, eqb, \
-                                                           c->fd, c->SFD, slopes, c->NP, tile_has, tstamp, ctl);      \
+        k_plat_block<K, TS, true><<<grid, PLAT_NT(K), 0, c->s>>>(W, H, launch, r, kn, a_cur, a_next, sp_in, sp_out, tver, \
+                                                              eqb, c->fd, c->SFD, slopes, c->NP, tile_has, tstamp, ctl); \
     else                                                                                                         \
-        k_plat_block<K, TS, false><<<G, PLAT_NT, 0, c->s>>>(W, H, launch, r, a_cur, a_next, sp_in, sp_out, tver, eqb, \
-                                                            c->fd, c->SFD, slopes, c->NP, tile_has, tstamp, ctl)
+        k_plat_block<K, TS, false><<<grid, PLAT_NT(K), 0, c->s>>>(W, H, launch, r, kn, a_cur, a_next, sp_in, sp_out, tver, \
+                                                               eqb, c->fd, c->SFD, slopes, c->NP, tile_has, tstamp, ctl)
             case 4: PLAT_LAUNCH(4); break;
             case 16: PLAT_LAUNCH(16); break;
             default: PLAT_LAUNCH(8); break;
 #undef PLAT_LAUNCH
             }
             ++launch;
-            r += c->plat_k;
+            r += K;
         }
-        prof_end(c, PROF_PLAT_K, BATCH);
+        prof_end(c, PROF_PLAT_K, batch);
         LEM_LAUNCHED(c);
         LEM_CHECK(c, hipMemcpyAsync(&c->hint[24], ctl, 3 * sizeof(int), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipMemcpyAsync(&c->hint[27], &ctl->last_change, sizeof(int), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipStreamSynchronize(c->s));
-        if (c->hint[24 + launch % 3] == 0) break;   // nothing queued for the next launch
+        const int moving = c->hint[24 + launch % 3];
+        if (moving == 0) break;   // nothing queued for the next launch
+        if (widen && moving <= c->ncu) K = 16;
         // every launch with a moving tile changes at least one cell, and a
         // cell's distance only decreases through a finite set of path lengths
         if (++guard > (long)n + 2) { c->err = "plateau routing did not converge"; return LEMHIP_E_NOT_CONVERGED; }
