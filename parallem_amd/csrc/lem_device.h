@@ -97,7 +97,7 @@ struct LemScalars {
     int fa_uncomputed, sed_uncomputed;
     int ncand;            // plateau candidates (mask cells without a downhill neighbour)
     int flag;             // generic change flag for host-driven loops
-    int hash_overflow;
+    int cut;              // some sink label has no path to label 0
     int w_bad;            // a mask cell's runoff weight is negative or not finite
     unsigned long long lowest_enc;
 };

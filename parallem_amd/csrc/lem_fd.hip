@@ -148,9 +148,9 @@ __device__ __forceinline__ void compact_chunks_ordered(long n, int *count, int *
     }
 }
 
-static inline int grid_chunks(long n, int cap = 8192)
+static inline int grid_chunks(long n, int cap = 8192, int items = COMPACT_ITEMS)
 {
-    long g = (n + 256L * COMPACT_ITEMS - 1) / (256L * COMPACT_ITEMS);
+    long g = (n + 256L * items - 1) / (256L * items);
     if (g > cap) g = cap;
     if (g < 1) g = 1;
     return (int)g;
@@ -819,51 +819,32 @@ __global__ void __launch_bounds__(256) k_merge_list(const int *cand, int n, cons
     }
 }
 
-// cells still pointing at another cell after the first jumps
-__global__ void __launch_bounds__(256) k_jump_list(long N, const uint8_t *mask, const int *ws, int *list, int *count)
+// identify_watershedMFD (newflow.cu:469-487): pointer jumping; in-place reads
+// of already-jumped targets only shorten chains
+__global__ void k_jump(long N, const uint8_t *mask, int *ws)
 {
-    __shared__ int s_wave[4];
-    __shared__ int s_base;
-    compact_chunks<COMPACT_ITEMS>(N, count, s_wave, &s_base, [&](long i) { return mask[i] && ws[i] < 0; },
-                                  [&](long i, int at) { list[at] = (int)i; });
-}
-
-// One lane per wave raises a progress flag (every lane writing the same word
-// serialises those writes).
-__device__ __forceinline__ void wave_flag(bool f, int *flag)
-{
-    const unsigned long long m = __ballot(f);
-    if (m && (int)(threadIdx.x & 63) == __ffsll((long long)m) - 1) *flag = 1;
-}
-
-__global__ void k_jump_some(int n, const int *list, int *ws, int *flag)
-{
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        int i = list[k];
-        int v = ws[i];
-        bool more = false;
-        if (v < 0) {
-            int t = ws[-v - 1];
-            ws[i] = t;
-            more = t < 0;
-        }
-        wave_flag(more, flag);
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
+        const int v = ws[i];
+        if (v < 0 && mask[i]) ws[i] = ws[-v - 1];
     }
 }
 
-// identify_watershedMFD (newflow.cu:469-487): pointer jumping; in-place reads
-// of already-jumped targets only shorten chains
-__global__ void k_jump(long N, const uint8_t *mask, int *ws, int *flag)
+// The rest in one launch: every cell still pointing walks to its label.  The
+// cells ahead of it walk at the same time and leave their labels, so a chain
+// of n links ends after about sqrt(2 n) of them.  (A list of the cells still
+// pointing and launches over it until none was left cost two host reads and
+// nine launches more: 0.12 ms of a 512^2 DEM's step.)  A walk longer than any
+// chain raises the error flag.
+__global__ void k_jump_walk(long N, const uint8_t *mask, int *ws, int *err)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
         int v = ws[i];
-        bool more = false;
-        if (v < 0 && mask[i]) {
-            int t = ws[-v - 1];
-            ws[i] = t;
-            more = t < 0;
-        }
-        wave_flag(more, flag);
+        if (v >= 0 || !mask[i]) continue;
+        long hops = 0;
+        do v = __hip_atomic_load(&ws[-v - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        while (v < 0 && ++hops <= N);
+        if (v < 0) *err = 1;
+        ws[i] = v;
     }
 }
 
@@ -1068,14 +1049,17 @@ __global__ void k_minimax_relax(int ne, const uint32_t *elo, const uint32_t *ehi
 //
 // Per phase (bw/be: the chosen weight and edge per component, double-buffered
 // by phase parity; nxt: the component each root joins):
+// st[0], st[1]: label 0's running maximum and its component (st[2], st[3] in
+// odd phases)
 __global__ void k_bv_init(long n, uint32_t *comp, unsigned long long *mv, unsigned long long *bw0,
-                          unsigned long long *bw1, uint32_t *be0, uint32_t *be1)
+                          unsigned long long *bw1, uint32_t *be0, uint32_t *be1, unsigned long long *st)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         comp[i] = (uint32_t)i;
         mv[i] = 0ULL;
         bw0[i] = bw1[i] = ~0ULL;
         be0[i] = be1[i] = ~0u;
+        if (i == 0) st[0] = st[1] = 0ULL;
     }
 }
 
@@ -1137,49 +1121,45 @@ __global__ void k_bv_min_e(int ne, const uint32_t *__restrict__ lo, const uint32
     if (wk == bw[cb]) atomicMin(&be[cb], (uint32_t)k);
 }
 
-// a component with a chosen edge points at the component across it (every
-// other label at itself)
+// A component with a chosen edge points at the component across it (every
+// other label at itself).  Two components that chose the same edge would
+// point at each other (under a strict order no longer cycle forms): the
+// smaller is the root.  The edge counter of this phase's compaction is cleared.
 __global__ void k_bv_hook(long n, const uint32_t *__restrict__ lo, const uint32_t *__restrict__ hi,
-                          const uint32_t *__restrict__ comp, const uint32_t *__restrict__ be, uint32_t *nxt)
+                          const uint32_t *__restrict__ comp, const uint32_t *__restrict__ be, uint32_t *nxt, int *kept)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        if (i == 0) *kept = 0;
         const uint32_t e = be[i];
         uint32_t t = (uint32_t)i;
         if (e != ~0u) {
             const uint32_t a = comp[lo[e]], b = comp[hi[e]];
-            t = a == (uint32_t)i ? b : a;
+            const uint32_t o = a == (uint32_t)i ? b : a;
+            if (be[o] != e || o < (uint32_t)i) t = o;
         }
         nxt[i] = t;
     }
 }
 
-// Two components that chose the same edge point at each other (under a
-// strict order no longer cycle forms); the smaller becomes the root.  Only
-// the smaller writes, and the entry it reads is the larger's, which the
-// larger never writes here.
-__global__ void k_bv_break(long n, const uint32_t *__restrict__ be, uint32_t *nxt)
-{
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        if (be[i] == ~0u) continue;
-        const uint32_t o = nxt[i];
-        if (o > (uint32_t)i && nxt[o] == (uint32_t)i) nxt[i] = (uint32_t)i;
-    }
-}
-
-// pointer jumping towards the roots of the joined components (a fixed
-// number of passes; the readers below walk what is left)
+// pointer jumping towards the roots of the joined components, four links a
+// launch (a fixed number of launches; the readers below walk what is left)
 __global__ void k_bv_jump(long n, uint32_t *nxt)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const uint32_t t = nxt[i];
-        const uint32_t tt = nxt[t];
-        if (tt != t) nxt[i] = tt;
+        const uint32_t t0 = nxt[i];
+        uint32_t t = t0;
+        for (int q = 0; q < 4; q++) {
+            const uint32_t u = nxt[t];
+            if (u == t) break;
+            t = u;
+        }
+        if (t != t0) nxt[i] = t;
     }
 }
 
 // The root of x's joined component: the pointers form trees whose roots
 // point at themselves (the only cycles Borůvka's choices make under a
-// strict order are pairs, and k_bv_break turns those into roots), and after
+// strict order are pairs, and k_bv_hook turns those into roots), and after
 // the jumping passes few links are left.  A walk longer than any tree could
 // be raises the error flag instead of running on.
 #define BV_WALK_MAX (1u << 20)
@@ -1194,26 +1174,32 @@ __device__ __forceinline__ uint32_t bv_root(const uint32_t *nxt, uint32_t x, int
     return x;
 }
 
-// label 0's running maximum and its new component: st[0], st[1]
-__global__ void k_bv_root0(const uint32_t *comp, const unsigned long long *bw, const uint32_t *be,
-                           const uint32_t *nxt, unsigned long long *st, int *err)
-{
-    const uint32_t c0 = comp[0];
-    if (be[c0] != ~0u && bw[c0] > st[0]) st[0] = bw[c0];
-    st[1] = bv_root(nxt, nxt[c0], err);
-}
-
 // every label: its running maximum, its new component, and its spill height
-// if that component is label 0's; the other parity's entries are reset for
-// the next phase (each label its own)
+// if that component is label 0's (whose own maximum and root each block finds
+// by itself: st as of this phase, stn for the next); the other parity's
+// entries are reset for the next phase (each label its own)
 __global__ void k_bv_labels(long n, uint32_t *comp, const unsigned long long *__restrict__ bw,
                             const uint32_t *__restrict__ be, const uint32_t *__restrict__ nxt,
                             unsigned long long *mv, unsigned long long *r, const unsigned long long *st,
-                            unsigned long long *bwn, uint32_t *ben, int *err)
+                            unsigned long long *stn, unsigned long long *bwn, uint32_t *ben, int *err)
 {
     const unsigned long long INF = ord_enc(lm_inf()), NEG = ord_enc(-lm_inf());
-    const unsigned long long m0 = st[0];
-    const uint32_t root0 = (uint32_t)st[1];
+    __shared__ unsigned long long s_m0;
+    __shared__ uint32_t s_root0;
+    if (threadIdx.x == 0) {
+        const uint32_t c0 = (uint32_t)st[1];
+        unsigned long long m = st[0];
+        if (be[c0] != ~0u && bw[c0] > m) m = bw[c0];
+        s_m0 = m;
+        s_root0 = bv_root(nxt, nxt[c0], err);
+        if (blockIdx.x == 0) {
+            stn[0] = m;
+            stn[1] = s_root0;
+        }
+    }
+    __syncthreads();
+    const unsigned long long m0 = s_m0;
+    const uint32_t root0 = s_root0;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         const uint32_t c = comp[i];
         unsigned long long m = mv[i];
@@ -1230,7 +1216,10 @@ __global__ void k_bv_labels(long n, uint32_t *comp, const unsigned long long *__
     }
 }
 
-// edges between different components, in order
+// edges between different components, in order (chunks of 4 rows on short
+// lists: with 16, the 27 K edges of a 512^2 DEM ran in 7 workgroups, 14.6 us a
+// phase; on long ones fewer workgroups add to the one counter)
+template <int ITEMS>
 __global__ void __launch_bounds__(256) k_bv_keep(int ne, const uint32_t *elo, const uint32_t *ehi,
                                                  const unsigned long long *ew, const uint32_t *comp, uint32_t *lo2,
                                                  uint32_t *hi2, unsigned long long *w2, int *count)
@@ -1238,7 +1227,7 @@ __global__ void __launch_bounds__(256) k_bv_keep(int ne, const uint32_t *elo, co
     __shared__ int s_wave[4];
     __shared__ int s_base;
     const unsigned long long INF = ord_enc(lm_inf());
-    compact_chunks_ordered<COMPACT_ITEMS>(
+    compact_chunks_ordered<ITEMS>(
         ne, count, s_wave, &s_base, [&](long k) { return ew[k] < INF && comp[elo[k]] != comp[ehi[k]]; },
         [&](long k, int at) { lo2[at] = elo[k]; hi2[at] = ehi[k]; w2[at] = ew[k]; });
 }
@@ -1392,9 +1381,12 @@ static int plat_grids(lemhip_ctx *c)
 
 // FlowDirs + plateau routing on surface zs; slopes == nullptr for pass 2.
 // Leaves the candidate list in c->cand and its length in *ncand_out; returns
-// the number of rounds that changed something in *rounds.
+// the number of rounds that changed something in *rounds.  cut (pass 2): set,
+// and the pass left before its plateau rounds, when labels turn out to be cut
+// off from label 0.
 template <typename TS>
-static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, int *ncand_out, int *rounds)
+static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, int *ncand_out, int *rounds,
+                                   bool *cut = nullptr)
 {
     long N = c->N;
     int W = c->W, H = c->H;
@@ -1407,11 +1399,14 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
                                           c->cand, &c->scal->ncand);
     prof_end(c, PROF_FLOWDIRS);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemcpyAsync(&c->hscal->ncand, &c->scal->ncand, sizeof(int), hipMemcpyDeviceToHost, c->s));
-    LEM_CHECK(c, hipStreamSynchronize(c->s));
+    LEM_TRY(read_scalars(c));
     int n = c->hscal->ncand;
     *ncand_out = n;
     *rounds = 0;
+    if (cut) {
+        *cut = c->hscal->cut != 0;
+        if (*cut) return LEMHIP_OK;
+    }
     if (n == 0) return LEMHIP_OK;
     prof_begin(c, PROF_PLATEAU);
     const int ntx = (W + PTW - 1) / PTW, nty = (H + PTH - 1) / PTH, ntiles = ntx * nty;
@@ -1569,6 +1564,7 @@ static int cutoff_components(lemhip_ctx *c, int nlab, int ne)
     return LEMHIP_OK;
 }
 
+#define BV_KEEP_SHORT (1 << 20)
 // Spill heights of the labels into c->rmm (initialised: label 0 -inf, the
 // rest +inf) by Borůvka phases over the label-sorted edge list.
 static int spill_heights(lemhip_ctx *c, int nlab, int ne)
@@ -1582,9 +1578,8 @@ static int spill_heights(lemhip_ctx *c, int nlab, int ne)
     unsigned long long *mv = c->hvals, *bw[2] = {c->cmax, c->hvals + n}, *st = c->hvals + 2 * n;
     uint32_t *be[2] = {reinterpret_cast<uint32_t *>(c->hkeys), reinterpret_cast<uint32_t *>(c->hkeys) + n};
     uint32_t *nxt = reinterpret_cast<uint32_t *>(c->hkeys) + 2 * n;
-    k_bv_init<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, mv, bw[0], bw[1], be[0], be[1]);
+    k_bv_init<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, mv, bw[0], bw[1], be[0], be[1], st);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemsetAsync(st, 0, 2 * sizeof(unsigned long long), c->s));
     const uint32_t *lo = c->elo, *hi = c->ehi;
     const unsigned long long *w = c->ew;
     int na = ne, buf = 0;
@@ -1593,25 +1588,24 @@ static int spill_heights(lemhip_ctx *c, int nlab, int ne)
     for (int ph = 0; na > 0; ph++) {
         const int p = ph & 1;
         const int ge = grid1d(na, 256, 1 << 30);
+        uint32_t *lo2 = c->elo2[buf], *hi2 = c->ehi2[buf];
+        unsigned long long *w2 = c->ew2[buf];
         prof_begin(c, PROF_MM_K);
         k_bv_min_w<<<ge, 256, 0, c->s>>>(na, lo, hi, w, c->comp, bw[p]);
         k_bv_min_e<<<ge, 256, 0, c->s>>>(na, lo, hi, w, c->comp, bw[p], be[p]);
-        k_bv_hook<<<grid1d(n), 256, 0, c->s>>>(n, lo, hi, c->comp, be[p], nxt);
-        k_bv_break<<<grid1d(n), 256, 0, c->s>>>(n, be[p], nxt);
-        // five jumping passes leave chains at most 1/32 as long; the root and
-        // label kernels walk the rest (no host read per phase for the jumps)
-        for (int q = 0; q < 5; q++) k_bv_jump<<<grid1d(n), 256, 0, c->s>>>(n, nxt);
-        prof_end(c, PROF_MM_K, 9);
-        LEM_LAUNCHED(c);
-        uint32_t *lo2 = c->elo2[buf], *hi2 = c->ehi2[buf];
-        unsigned long long *w2 = c->ew2[buf];
-        LEM_CHECK(c, hipMemsetAsync(&c->scal->nedges, 0, sizeof(int), c->s));
-        prof_begin(c, PROF_MM_K);
-        k_bv_root0<<<1, 1, 0, c->s>>>(c->comp, bw[p], be[p], nxt, st, &c->scal->flag);
-        k_bv_labels<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, bw[p], be[p], nxt, mv, c->rmm, st, bw[p ^ 1],
-                                                  be[p ^ 1], &c->scal->flag);
-        k_bv_keep<<<grid_chunks(na), 256, 0, c->s>>>(na, lo, hi, w, c->comp, lo2, hi2, w2, &c->scal->nedges);
-        prof_end(c, PROF_MM_K, 3);
+        k_bv_hook<<<grid1d(n), 256, 0, c->s>>>(n, lo, hi, c->comp, be[p], nxt, &c->scal->nedges);
+        // two launches of four links leave short chains; the label kernel
+        // walks the rest (no host read per phase for the jumps)
+        for (int q = 0; q < 2; q++) k_bv_jump<<<grid1d(n), 256, 0, c->s>>>(n, nxt);
+        k_bv_labels<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, bw[p], be[p], nxt, mv, c->rmm, st + 2 * p,
+                                                  st + 2 * (p ^ 1), bw[p ^ 1], be[p ^ 1], &c->scal->flag);
+        if (na <= BV_KEEP_SHORT)
+            k_bv_keep<4><<<grid_chunks(na, 8192, 4), 256, 0, c->s>>>(na, lo, hi, w, c->comp, lo2, hi2, w2,
+                                                                     &c->scal->nedges);
+        else
+            k_bv_keep<COMPACT_ITEMS><<<grid_chunks(na), 256, 0, c->s>>>(na, lo, hi, w, c->comp, lo2, hi2, w2,
+                                                                        &c->scal->nedges);
+        prof_end(c, PROF_MM_K, 7);
         LEM_LAUNCHED(c);
         LEM_TRY(read_scalars(c));
         if (c->hscal->flag) { c->err = "spill-height component pointers form a cycle"; return LEMHIP_E_NOT_CONVERGED; }
@@ -1626,6 +1620,14 @@ static int spill_heights(lemhip_ctx *c, int nlab, int ne)
     }
     return LEMHIP_OK;
 }
+
+static int raise_surface(lemhip_ctx *c)
+{
+    k_raise<<<grid1d(c->N), 256, 0, c->s>>>(c->N, c->mask, c->ws, c->rmm, c->dem, c->demid, c->dsc, c->z2);
+    LEM_LAUNCHED(c);
+    return LEMHIP_OK;
+}
+
 
 // floodingDriver (routeflow.cu:202-676) up to the raised surface in c->z2
 static int flooding(lemhip_ctx *c, int ncand1)
@@ -1649,57 +1651,35 @@ static int flooding(lemhip_ctx *c, int ncand1)
     LEM_CHECK(c, hipMemcpyAsync(&c->hint[0], c->scan_tmp + (N - 1), sizeof(int), hipMemcpyDeviceToHost, c->s));
     LEM_CHECK(c, hipMemcpyAsync(&c->hint[1], prefix + (N - 1), sizeof(int), hipMemcpyDeviceToHost, c->s));
     k_init_ws<<<grid2d(W, H), 256, 0, c->s>>>(W, H, c->mask, c->SFD, prefix, c->demid, c->ddesc, c->ws, c->labdem);
-    LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipStreamSynchronize(c->s));
-    int nlab = c->hint[0] + c->hint[1];
-    c->h_nlab = nlab;
     // sink merge over the sinks that have an equal-height neighbour (list in the
     // prefix buffer, free after k_init_ws)
-    {
-        int *mlist = reinterpret_cast<int *>(c->z2);
-        LEM_CHECK(c, hipMemsetAsync(&c->scal->ncand, 0, sizeof(int), c->s));
-        k_merge_list<<<grid1d(ncand1, 256, 4096), 256, 0, c->s>>>(c->cand, ncand1, c->SFD, c->dmask, mlist,
-                                                                 &c->scal->ncand);
-        LEM_LAUNCHED(c);
-        LEM_TRY(read_scalars(c));
-        int nm = c->hscal->ncand;
-        for (int it = 0; nm > 0; it += 4) {
-            LEM_TRY(clear_flag(c));
-            for (int q = 0; q < 4; q++)
-                k_sink_merge<<<grid1d(nm, 256, 1 << 30), 256, 0, c->s>>>(W, H, mlist, nm, c->SFD, c->dem, c->ws,
-                                                                         &c->scal->flag);
-            LEM_LAUNCHED(c);
-            int f = 0;
-            LEM_TRY(read_flag(c, &f));
-            if (!f) break;
-            if (it / 4 > nm + 2) { c->err = "sink merge did not converge"; return LEMHIP_E_NOT_CONVERGED; }
-        }
-    }
-    // pointer jumping: four passes over every cell, then only the cells still pointing
-    for (int it = 0;; it += 4) {
+    int *mlist = reinterpret_cast<int *>(c->z2);
+    LEM_CHECK(c, hipMemcpyAsync(&c->hint[1], prefix + (N - 1), sizeof(int), hipMemcpyDeviceToHost, c->s));
+    LEM_CHECK(c, hipMemsetAsync(&c->scal->ncand, 0, sizeof(int), c->s));
+    k_merge_list<<<grid1d(ncand1, 256, 4096), 256, 0, c->s>>>(c->cand, ncand1, c->SFD, c->dmask, mlist,
+                                                             &c->scal->ncand);
+    LEM_LAUNCHED(c);
+    LEM_TRY(read_scalars(c));
+    const int nlab = c->hint[0] + c->hint[1];
+    c->h_nlab = nlab;
+    const int nm = c->hscal->ncand;
+    for (int it = 0; nm > 0; it += 4) {
         LEM_TRY(clear_flag(c));
-        for (int q = 0; q < 4; q++) k_jump<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag);
+        for (int q = 0; q < 4; q++)
+            k_sink_merge<<<grid1d(nm, 256, 1 << 30), 256, 0, c->s>>>(W, H, mlist, nm, c->SFD, c->dem, c->ws,
+                                                                     &c->scal->flag);
         LEM_LAUNCHED(c);
         int f = 0;
         LEM_TRY(read_flag(c, &f));
         if (!f) break;
-        int *jlist = c->scan_tmp;
-        LEM_CHECK(c, hipMemsetAsync(&c->scal->ncand, 0, sizeof(int), c->s));
-        k_jump_list<<<grid_chunks(N), 256, 0, c->s>>>(N, c->mask, c->ws, jlist, &c->scal->ncand);
-        LEM_LAUNCHED(c);
-        LEM_TRY(read_scalars(c));
-        int nj = c->hscal->ncand;
-        for (int it2 = 0; nj > 0; it2 += 4) {
-            LEM_TRY(clear_flag(c));
-            for (int q = 0; q < 4; q++)
-                k_jump_some<<<grid1d(nj, 256, 8192), 256, 0, c->s>>>(nj, jlist, c->ws, &c->scal->flag);
-            LEM_LAUNCHED(c);
-            LEM_TRY(read_flag(c, &f));
-            if (!f) break;
-            if (it2 > 128) { c->err = "watershed pointer jumping did not converge"; return LEMHIP_E_NOT_CONVERGED; }
-        }
-        break;
+        if (it / 4 > nm + 2) { c->err = "sink merge did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
+    // watershed labels: one jump over every cell, then each walks the rest
+    // (none to four jumps first: within 2 % on every size)
+    LEM_TRY(clear_flag(c));
+    k_jump<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws);
+    k_jump_walk<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag);
+    LEM_LAUNCHED(c);
     // edges: block-distinct pairs appended, sorted by pair, reduced to the
     // minimum weight per pair; the list comes out sorted by label (the
     // Borůvka phases read neighbouring labels' components from the same
@@ -1718,6 +1698,7 @@ static int flooding(lemhip_ctx *c, int ncand1)
                                             &c->scal->nedges, B);
         LEM_LAUNCHED(c);
         LEM_TRY(read_scalars(c));
+        if (c->hscal->flag) { c->err = "watershed pointer jumping did not converge"; return LEMHIP_E_NOT_CONVERGED; }
         np = c->hscal->nedges;
         if (np <= c->hcap) break;
         want = np + np / 4;
@@ -1758,15 +1739,11 @@ static int flooding(lemhip_ctx *c, int ncand1)
     c->h_nedges = ne;
 
     LEM_TRY(spill_heights(c, nlab, ne));
-    LEM_TRY(clear_flag(c));
-    if (ne > 0) k_fb_unreached<<<grid1d(ne, 256, 1 << 30), 256, 0, c->s>>>(ne, c->elo, c->ehi, c->rmm, &c->scal->flag);
-    LEM_LAUNCHED(c);
-    int cut = 0;
-    LEM_TRY(read_flag(c, &cut));
-    if (cut) LEM_TRY(cutoff_components(c, nlab, ne));
-    k_raise<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, c->rmm, c->dem, c->demid, c->dsc, c->z2);
-    LEM_LAUNCHED(c);
-    return LEMHIP_OK;
+    // labels cut off from label 0 (NaN heights only) raise scal->cut, read with
+    // the next pass's candidate count: the surface is raised before it is known
+    LEM_CHECK(c, hipMemsetAsync(&c->scal->cut, 0, sizeof(int), c->s));
+    if (ne > 0) k_fb_unreached<<<grid1d(ne, 256, 1 << 30), 256, 0, c->s>>>(ne, c->elo, c->ehi, c->rmm, &c->scal->cut);
+    return raise_surface(c);
 }
 
 // Times the plateau pass with every rounds-per-launch candidate on the same
@@ -1844,8 +1821,14 @@ static int fd_phase_t(lemhip_ctx *c, int iter)
         k_slots_sinkcount_fin<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->ddesc, c->nslot, c->dsc);
         prof_end(c, PROF_FLOOD);
         int n2 = 0, r2 = 0;
+        bool cut = false;
+        LEM_TRY(directions_and_plateaus<TS>(c, c->z2, (TS *)nullptr, &n2, &r2, &cut));
+        if (cut) {
+            LEM_TRY(cutoff_components(c, c->h_nlab, c->h_nedges));
+            LEM_TRY(raise_surface(c));
+        }
         if (c->tune_plat_pending) LEM_TRY(tune_plateau<TS>(c, c->z2, (TS *)nullptr));
-        LEM_TRY(directions_and_plateaus<TS>(c, c->z2, (TS *)nullptr, &n2, &r2));
+        if (cut) LEM_TRY(directions_and_plateaus<TS>(c, c->z2, (TS *)nullptr, &n2, &r2));
         c->h_rounds2 = r2;
     }
     k_merge<<<grid1d(N), 256, 0, c->s>>>(N, c->p.flowdirectiontype, c->mask, c->fd, c->SFD);
