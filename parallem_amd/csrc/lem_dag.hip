@@ -55,6 +55,9 @@ __device__ __forceinline__ float2 ff_add(float2 a, float2 b)
 #define W_DEAD1 (1u << 24)
 #define W_STSH 28
 #define W_UPD (1u << 30)
+// resident tiles under single flow directions: bits 16-23 hold the receiver's
+// signed offset in the padded layout (0: none in the tile), and
+#define W_OUT (1u << 31)   // the receiver lies in another tile
 
 // ------------------------------------------------------------ cell bodies
 //
@@ -129,6 +132,9 @@ __device__ __forceinline__ float2 fa_final(float w, float2 a) { return ff_add(ma
 //   compute(L, p, bits, upd)  the chain part, LDS only; the donors are the
 //        set bits of the pull-order mask, summed lowest bit first, which is
 //        the order E..NE of the reference (absent donors add nothing)
+//   fetch(L, p), result(in, bits), set(L, p, v, upd)  compute in parts: the
+//        LDS reads, the arithmetic, the LDS write
+//   final(r)            the Fin of store alone
 //   finish(L, p, i, fin, upd)  HBM writes of a cell completed in this
 //        round, after the walks (coalesced, off the chains)
 //   word(L, p) / put(L, p, w)  the value a receiver in another tile reads, as
@@ -184,35 +190,47 @@ struct FaCell {
         L.val[p] = r.v;
         return Fin{};
     }
+    __device__ __forceinline__ Fin final(const Reg &) const { return Fin{}; }
     __device__ __forceinline__ void store_halo(Lds &L, int p, const HReg &r) const { L.val[p] = r; }
     // fa = w + max(0, sum of donor fa in the order E..NE) (mfd_simple.cu:71-168;
     // prop = 1 for every mask donor, runoffweight.cu:126-134, so fa*prop == fa)
-    // MANY: all eight neighbours read at once (cells of multiple flow
-    // directions have 3.5 donors on average)
-    template <bool MANY>
     __device__ __forceinline__ void compute(Lds &L, int p, unsigned bits, bool) const
     {
+        // one read per donor (chain cells mostly have one or two donors, and
+        // a compensated add costs more than the read)
         const T wv = L.w[p];
         FS accum{};
-        if constexpr (MANY) {
-            FS v8[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) v8[k] = L.val[p + poff<TW>(cpull(k))];
-#pragma unroll
-            for (int k = 0; k < 8; k++)
-                if ((bits >> k) & 1u) fa_acc(accum, v8[k]);
-        } else {
-            // one read per donor (chain cells mostly have one or two donors, and
-            // a compensated add costs more than the read)
-            while (bits) {
-                const int k = __ffs(bits) - 1;
-                bits &= bits - 1;
-                fa_acc(accum, L.val[p + koff<TW>(k)]);
-            }
+        while (bits) {
+            const int k = __ffs(bits) - 1;
+            bits &= bits - 1;
+            fa_acc(accum, L.val[p + koff<TW>(k)]);
         }
         fa_clamp(accum);
         L.val[p] = fa_final(wv, accum);
     }
+    // the same in two parts: every LDS read of cell p, and the result from them
+    struct In {
+        T w;
+        FS v8[8];
+    };
+    __device__ __forceinline__ In fetch(const Lds &L, int p) const
+    {
+        In n;
+        n.w = L.w[p];
+#pragma unroll
+        for (int k = 0; k < 8; k++) n.v8[k] = L.val[p + poff<TW>(cpull(k))];
+        return n;
+    }
+    __device__ __forceinline__ FS result(const In &n, unsigned bits) const
+    {
+        FS accum{};
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if ((bits >> k) & 1u) fa_acc(accum, n.v8[k]);
+        fa_clamp(accum);
+        return fa_final(n.w, accum);
+    }
+    __device__ __forceinline__ void set(Lds &L, int p, FS v, bool) const { L.val[p] = v; }
     __device__ __forceinline__ unsigned long long word(const Lds &L, int p) const { return ex_word(L.val[p]); }
     __device__ __forceinline__ void put(Lds &L, int p, unsigned long long w) const { ex_value(w, &L.val[p]); }
     __device__ __forceinline__ void finish(const Lds &L, int p, long i, const Fin &, bool) const { fa[i] = L.val[p]; }
@@ -271,10 +289,15 @@ struct SedCell {
         }
         L.a[p] = a;
         L.b[p] = b;
+        return final(r);
+    }
+    __device__ __forceinline__ Fin final(const Reg &r) const
+    {
+        const double sedthick = r.sT + (double)r.dp;
         double toterosion;
         if (sizeof(T) == 8) toterosion = (double)r.e + (double)r.in + (double)r.g;
         else toterosion = (double)(r.e + r.in + r.g);
-        Fin f{r.dp, sT};
+        Fin f{r.dp, r.sT};
         if (toterosion >= sedthick) f.sTn = 0.0;
         if (sedthick > toterosion) f.sTn = sedthick - toterosion;
         return f;
@@ -283,25 +306,41 @@ struct SedCell {
     // the reference sums all eight terms with zeros for absent donors; adding
     // only the donors' terms from +0 gives the same value up to the sign of a
     // zero sum, which the clamp below erases
-    template <bool MANY>
     __device__ __forceinline__ void compute(Lds &L, int p, unsigned bits, bool upd) const
     {
-        if (!upd) return;
-        const T one = (T)1;
-        const T a = L.a[p], b = L.b[p];
-        // all eight neighbours in flight at once (the padded layout keeps the
-        // reads inside the array), then the donors' terms in order
+        if (upd) L.stone[p] = result(fetch(L, p), bits);
+    }
+    struct In {
+        T a, b;
         T v8[8];
+    };
+    // all eight neighbours in flight at once (the padded layout keeps the
+    // reads inside the array)
+    __device__ __forceinline__ In fetch(const Lds &L, int p) const
+    {
+        In n;
+        n.a = L.a[p];
+        n.b = L.b[p];
 #pragma unroll
-        for (int k = 0; k < 8; k++) v8[k] = L.stone[p + poff<TW>(cpull(k))];
+        for (int k = 0; k < 8; k++) n.v8[k] = L.stone[p + poff<TW>(cpull(k))];
+        return n;
+    }
+    // the donors' terms in order
+    __device__ __forceinline__ T result(const In &n, unsigned bits) const
+    {
+        const T one = (T)1;
         T propStonefrom = (T)0;
 #pragma unroll
         for (int k = 0; k < 8; k++)
-            if (bits & (1u << k)) propStonefrom = propStonefrom + one * v8[k];
-        T st = a + b * propStonefrom;
+            if (bits & (1u << k)) propStonefrom = propStonefrom + one * n.v8[k];
+        T st = n.a + n.b * propStonefrom;
         if (st < (T)0.01) st = (T)0.01;
         else if (st > (T)99.9) st = (T)99.9;
-        L.stone[p] = st;
+        return st;
+    }
+    __device__ __forceinline__ void set(Lds &L, int p, T v, bool upd) const
+    {
+        if (upd) L.stone[p] = v;
     }
     __device__ __forceinline__ unsigned long long word(const Lds &L, int p) const { return ex_word(L.stone[p]); }
     __device__ __forceinline__ void put(Lds &L, int p, unsigned long long w) const { ex_value(w, &L.stone[p]); }
@@ -316,6 +355,69 @@ struct SedCell {
         soilT[i] = f.sTn;
     }
 };
+
+// bits 16-31 of a tile cell's word: receiver bits, or the single receiver
+template <int TW, int TH, bool SFD>
+__device__ __forceinline__ uint32_t receiver_bits(uint32_t f, int li)
+{
+    if (!SFD || !f) return f << 16;
+    static_assert(TW + 3 <= 127, "offsets fit a signed byte");
+    const int d = cpull(__ffs(f) - 1), r = li / TW + kDY[d], c = li % TW + kDX[d];
+    const bool in = r >= 0 && r < TH && c >= 0 && c < TW;
+    return in ? (uint32_t)((kDY[d] * (TW + 2) + kDX[d]) & 0xFF) << 16 : W_OUT;
+}
+
+// Follows chains under single flow directions, one wave in lockstep: LDS
+// operations of one wave take effect in the order issued, so a value written
+// before the counter add of the same step is there for whoever the add hands
+// the cell to.  The receiver is known before the result: the add that may hand
+// it over and every read of it are issued together, one wait per link; a lane
+// that was not the last to arrive drops what it read.  A link is bound by its
+// instructions (about 8 cycles each for a wave alone) and that wait: 0.37 us,
+// 0.6 with the reads after the add's return and the queue tests in every link.
+// Steps until no lane has a cell or `steps` links; cur < 0: no cell.
+template <int TW, class Cell, class Out>
+__device__ __forceinline__ void follow_chains(const Cell &cell, typename Cell::Lds &lds, uint32_t *wd, int &cur,
+                                              uint32_t &word, typename Cell::In &in, int steps, Out out_of_tile)
+{
+    for (int q = 0; q < steps; q++) {
+        const bool on = cur >= 0;
+        const int p = cur;
+        const bool dead = on && Cell::kCanDie && ((word >> 24) & 0xFu) != 0;
+        const bool out = on && (word & W_OUT);
+        if (on) {
+            const bool upd = (word & W_UPD) != 0;
+            if (!dead) cell.set(lds, p, cell.result(in, (word >> 8) & 0xFFu), upd);
+            wd[p] = ((uint32_t)(dead ? ST_DEAD : ST_DONE) << W_STSH) | W_NEVER | (word & W_UPD);
+            asm volatile("" ::: "memory");
+            const int off = (int)(int8_t)(uint8_t)(word >> 16);
+            const uint32_t delta = dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu;
+            const uint32_t old = atomicAdd(&wd[p + off], off ? delta : 0u);
+            in = cell.fetch(lds, p + off);
+            cur = off && (old & W_CNT) == 1u ? p + off : -1;
+            word = old + delta;
+        }
+        if (__ballot(out)) out_of_tile(out, p, dead);
+        if (!__ballot(cur >= 0)) break;
+    }
+}
+
+// lanes without a cell take one each from queue[head, tail)
+template <class Cell, class Q>
+__device__ __forceinline__ void take_cells(const Cell &cell, const typename Cell::Lds &lds, const uint32_t *wd,
+                                           const Q *queue, int &head, int tail, int &cur, uint32_t &word,
+                                           typename Cell::In &in)
+{
+    if (head >= tail) return;
+    const unsigned long long m = __ballot(cur < 0);
+    const int n = __popcll(m), rank = __popcll(m & ((1ULL << (threadIdx.x & 63)) - 1ULL));
+    if (cur < 0 && rank < tail - head) {
+        cur = queue[head + rank];
+        word = wd[cur];
+        in = cell.fetch(lds, cur);
+    }
+    head += n < tail - head ? n : tail - head;
+}
 
 // ------------------------------------------------------------ prep kernels
 
@@ -737,7 +839,7 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_round(int W, int H, i
                     int rp0 = f ? cur + koff<TW>(__ffs(f) - 1) : cur;
                     uint32_t ns = ST_DEAD;
                     if (!dead) {
-                        cell.template compute<false>(lds, cur, (word >> 8) & 0xFFu, (word & W_UPD) != 0);
+                        cell.compute(lds, cur, (word >> 8) & 0xFFu, (word & W_UPD) != 0);
                         ns = ST_DONE;
                     }
                     wd[cur] = (word & ~(3u << W_STSH)) | (ns << W_STSH);
@@ -833,12 +935,12 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_round(int W, int H, i
 // the pass: each workgroup keeps one 32 x 32 tile in LDS until its last cell
 // is resolved, and tiles exchange the values of their edge cells while they
 // run.  Bound by the longest dependency path: its cells one after another
-// (0.6 us each under single flow directions, 0.8 to 1.2 under multiple) plus
-// a few us per tile crossing, instead of one launch per crossing, each as long
-// as its slowest visit (12-60 us).  Flow accumulation, launch rounds alone
-// against this: 512^2 FP64 0.56 -> 0.26 ms, under multiple directions
-// 5.7 -> 0.95 ms; 1133 x 739 FP32, multiple directions 19.2 -> 3.1 ms;
-// 4096^2 FP64 4.8 -> 3.4 ms (32 launch rounds, then 1511 resident tiles).
+// (0.37 us each under single flow directions, 0.75 to 1.35 under multiple)
+// plus about 2 us per tile crossing, instead of one launch per crossing, each
+// as long as its slowest visit (12-60 us).  Flow accumulation, launch rounds
+// alone against this: 512^2 FP64 0.56 -> 0.17 ms, under multiple directions
+// 5.7 -> 0.72 ms; 1133 x 739 FP32, multiple directions 19.2 -> 2.5 ms;
+// 4096^2 FP64 4.8 -> 2.8 ms (32 launch rounds, then 1511 resident tiles).
 //
 // Exchange: an entry per edge cell of every listed tile (top row, bottom row,
 // left column, right column; corners twice), EX_PENDING until the cell
@@ -857,6 +959,7 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_round(int W, int H, i
 #define RES_EDGE 128
 #define RES_BEATS 64
 #define RES_IDLE 3000          // 100 MHz ticks: 30 us
+#define RES_LIMIT 50000000     // no tile waits longer than this after its start (0.5 s)
 struct ResCtl {    // LEM_RES_CTL bytes
     int n;         // listed tiles
     int left;      // cells still pending in them after the launch
@@ -911,6 +1014,13 @@ __global__ void __launch_bounds__(256) k_res_list(int W, int H, const int *__res
     }
 }
 
+// queue entry of cell p: padded index, bit 11 a dead donor, bit 12 the stone
+// update applies, bits 16-23 donors, bits 24-31 receivers
+__device__ __forceinline__ uint32_t res_entry(uint32_t word, int p)
+{
+    return ((word & 0x00FFFF00u) << 8) | (uint32_t)p | ((word >> 24) & 0xFu ? 0x800u : 0u) | (word & W_UPD ? 0x1000u : 0u);
+}
+
 template <class Cell, bool SFD>
 __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H, int round, Cell cell,
                                                                     const uint8_t *__restrict__ dm,
@@ -925,7 +1035,10 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
     __shared__ uint32_t wd[NP];      // packed words (W_*), padded layout; ring cells: state 3, fd bits
     __shared__ uint8_t pst[NP];      // states at the start, as in k_dag_round
     __shared__ typename Cell::Lds lds;
-    __shared__ uint16_t queue[NC];   // ready cells (each enters at most once)
+    // ready cells (each enters at most once): the padded index, and under
+    // multiple directions in one word with what a step needs of the cell
+    using Q = typename std::conditional<SFD, uint16_t, uint32_t>::type;
+    __shared__ Q queue[NC];
     __shared__ int qn, s_left, s_prog;
     __shared__ int s_pos[9];
     if ((int)blockIdx.x >= ctl->n) return;
@@ -974,7 +1087,6 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
             hr = cell.load_halo(i);
         }
     }
-    typename Cell::Fin fin[PER];
     uint32_t xw[PER];
 #pragma unroll
     for (int q = 0; q < PER; q++) {
@@ -982,7 +1094,7 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
         const uint32_t sv = (vs[q] == DAG_PENDING) ? ST_PENDING : (vs[q] >= 0 ? ST_DONE : ST_DEAD);
         xw[q] = 0;
         const int p = pidx<TW>(li / TW, li % TW);
-        fin[q] = cell.store(lds, p, vr[q], &xw[q]);
+        (void)cell.store(lds, p, vr[q], &xw[q]);
         wd[p] = (sv << W_STSH) | (vf[q] << 16) | (vb[q] << 8) | W_NEVER;
         pst[p] = (uint8_t)sv;
     }
@@ -1019,7 +1131,8 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
             nin += (oh & ((1u << ST_PENDING) | (1u << ST_RING_WAIT))) ? 1 : 0;
             seen |= oh;
         }
-        const uint32_t base = ((uint32_t)ST_PENDING << W_STSH) | (vf[q] << 16) | (bits << 8) | xw[q];
+        const uint32_t base = ((uint32_t)ST_PENDING << W_STSH) | receiver_bits<TW, TH, SFD>(vf[q], li) | (bits << 8) |
+                              xw[q];
         if ((seen >> ST_DEAD) & 1u) { myw[q] = base | W_NEVER | W_DEAD1; seeds |= 1 << q; }
         else { myw[q] = base | (uint32_t)nin; if (nin == 0) seeds |= 1 << q; }
     }
@@ -1034,37 +1147,36 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
         int base = 0;
         if ((threadIdx.x & 63) == 0 && m) base = atomicAdd(&qn, __popcll(m));
         base = __shfl(base, 0);
-        if (sd) queue[base + __popcll(m & ((1ULL << (threadIdx.x & 63)) - 1))] = (uint16_t)p;
+        if (sd) queue[base + __popcll(m & ((1ULL << (threadIdx.x & 63)) - 1))] = SFD ? (Q)p : (Q)res_entry(myw[q], p);
     }
     __syncthreads();
-    // 3. one wave resolves cells in lockstep: LDS operations of one wave take
-    //    effect in the order issued, so a value written before the counter
-    //    add of the same step is there for whoever the add hands the cell to
+    // 3. one wave resolves cells in lockstep (follow_chains) and polls the ring
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
         const unsigned long long below = (1ULL << lane) - 1ULL;
         unsigned long long *mine = ex + (long)blockIdx.x * RES_EDGE;
-        // ring cells this lane polls: padded index, exchange entry, receivers in the tile
-        int rp[RPER];
-        unsigned rf[RPER];
-        const unsigned long long *rx[RPER];
+        // ring cells this lane polls: padded index, exchange entry, receivers in
+        // the tile (direction bits; the padded index of the only one under
+        // single directions)
+        int rp[RPER], rf[RPER];
+        int rx[RPER];
         unsigned live = 0;
 #pragma unroll
         for (int j = 0; j < RPER; j++) {
             const int h = lane + 64 * j;
             rp[j] = 0;
             rf[j] = 0;
-            rx[j] = ex;
+            rx[j] = 0;
             if (h >= NH) continue;
             int nr, nc;
             halo_pos<TW, TH>(h, &nr, &nc);
             const int p = pidx<TW>(nr, nc);
             if (pst[p] != ST_RING_WAIT) continue;
             const unsigned f = (wd[p] >> 16) & 0xFFu;
-            unsigned in = 0;
+            int in = 0;
             for (int k = 0; k < 8; k++) {
                 const int d = cpull(k), r = nr + cdy(d), c = nc + cdx(d);
-                if (((f >> k) & 1u) && r >= 0 && r < TH && c >= 0 && c < TW) in |= 1u << k;
+                if (((f >> k) & 1u) && r >= 0 && r < TH && c >= 0 && c < TW) in = SFD ? pidx<TW>(r, c) : in | (1 << k);
             }
             const int ty = nr < 0 ? 0 : (nr >= TH ? 2 : 1), tx = nc < 0 ? 0 : (nc >= TW ? 2 : 1);
             const int np = s_pos[ty * 3 + tx];
@@ -1073,143 +1185,177 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
             const int e = ty == 0 ? 32 + cc : (ty == 2 ? cc : (tx == 0 ? 96 + rr : 64 + rr));
             rp[j] = p;
             rf[j] = in;
-            rx[j] = ex + (long)np * RES_EDGE + e;
+            rx[j] = np * RES_EDGE + e;
             live |= 1u << j;
         }
-        int head = 0, tail = qn;
-        int cur = -1;
-        uint32_t word = 0;
-        bool worked = false;                 // since the last poll
-        unsigned steps = 0;
+        // queue[head, tail): ready cells; both the same in every lane
+        int head = 0, tail = __builtin_amdgcn_readfirstlane(qn);
+        auto push = [&](bool ready, uint32_t entry) {
+            const unsigned long long m = __ballot(ready);
+            if (!m) return;
+            if (ready) queue[tail + __popcll(m & below)] = (Q)entry;
+            tail += __popcll(m);
+        };
+        auto beat = [&]() {
+            if (lane == 0)
+                __hip_atomic_fetch_add(&ctl->beat[(blockIdx.x % RES_BEATS) * 16], 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        };
+        auto publish = [&](int p, unsigned long long v, bool row0, bool row1, bool col0, bool col1) {
+            const int lr = p / PW - 1, lc = p % PW - 1;
+            auto put = [&](int e) { __hip_atomic_store(&mine[e], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+            if (row0 && lr == 0) put(lc);
+            if (row1 && lr == TH - 1) put(32 + lc);
+            if (col0 && lc == 0) put(64 + lr);
+            if (col1 && lc == TW - 1) put(96 + lr);
+        };
+        // Polls the ring once: arrived(j, delta) for each lane's cells that
+        // resolved.  Returns 0 when the tile should leave, 1 when nothing is
+        // new, 2 otherwise.
         bool idle = false;
         unsigned long long t_idle = 0;
         int beat0 = 0;
-        // the receivers of resolved cells, one bit of f per step in every
-        // lane: each lane keeps the first cell handed to it and queues the rest
-        auto hand_over = [&](int from, unsigned f, uint32_t delta, bool &out) {
-            while (__ballot(f != 0)) {
-                const bool on = f != 0;
-                const int r = on ? from + koff<TW>(__ffs(f) - 1) : from;
-                f &= f - 1;
-                uint32_t old = 0;
-                if (on) old = atomicAdd(&wd[r], delta);
-                out |= on && ((old >> W_STSH) & 3u) == 3u;
-                const bool ready = on && (old & W_CNT) == 1u;
-                const bool push = ready && cur >= 0;
-                if (ready && cur < 0) { cur = r; word = old + delta; }
-                const unsigned long long m = __ballot(push);
-                if (push) queue[tail + __popcll(m & below)] = (uint16_t)r;
-                tail += __popcll(m);
-            }
-        };
-        for (;;) {
-            if (head < tail) {
-                const unsigned long long m = __ballot(cur < 0);
-                const int rank = __popcll(m & below);
-                if (cur < 0 && rank < tail - head) {
-                    cur = queue[head + rank];
-                    word = wd[cur];
-                }
-                const int take = __popcll(m);
-                head += take < tail - head ? take : tail - head;
-            }
-            if (__ballot(cur >= 0)) {
-                // a beat every 16 steps, so that others do not leave while this
-                // tile works through a long stretch
-                if ((++steps & 15) == 0 && lane == 0)
-                    __hip_atomic_fetch_add(&ctl->beat[(blockIdx.x % RES_BEATS) * 16], 1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-                worked = true;
-                const bool on = cur >= 0;
-                const int p = cur;
-                const bool dead = on && Cell::kCanDie && ((word >> 24) & 0xFu) != 0;
-                unsigned f = on ? (word >> 16) & 0xFFu : 0u;
-                if (on) {
-                    if (!dead) cell.template compute<!SFD>(lds, p, (word >> 8) & 0xFFu, (word & W_UPD) != 0);
-                    wd[p] = (word & ~(3u << W_STSH)) | ((uint32_t)(dead ? ST_DEAD : ST_DONE) << W_STSH);
-                }
-                asm volatile("" ::: "memory");
-                cur = -1;
-                bool out = false;   // a receiver lies in another tile
-                const uint32_t delta = dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu;
-                if constexpr (SFD) {
-                    hand_over(p, f, delta, out);
-                } else {
-                    // all eight neighbours' adds in flight at once, 0 for those
-                    // that are no receivers; extra ready cells are queued after
-                    unsigned more = 0;
-                    if (on) {
-                        uint32_t old[8];
-#pragma unroll
-                        for (int k = 0; k < 8; k++)
-                            old[k] = atomicAdd(&wd[p + poff<TW>(cpull(k))], ((f >> k) & 1u) ? delta : 0u);
-#pragma unroll
-                        for (int k = 0; k < 8; k++) {
-                            const bool rcv = (f >> k) & 1u;
-                            out |= rcv && ((old[k] >> W_STSH) & 3u) == 3u;
-                            if (!rcv || (old[k] & W_CNT) != 1u) continue;
-                            if (cur < 0) { cur = p + poff<TW>(cpull(k)); word = old[k] + delta; }
-                            else more |= 1u << k;
-                        }
-                    }
-                    while (__ballot(more != 0)) {
-                        const unsigned long long m = __ballot(more != 0);
-                        if (more) queue[tail + __popcll(m & below)] = (uint16_t)(p + koff<TW>(__ffs(more) - 1));
-                        more &= more - 1;
-                        tail += __popcll(m);
-                    }
-                }
-                if (out) {
-                    const unsigned long long v = dead ? EX_DEAD : cell.word(lds, p);
-                    const int lr = p / PW - 1, lc = p % PW - 1;
-                    auto put = [&](int e) {
-                        __hip_atomic_store(&mine[e], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    };
-                    if (lr == 0) put(lc);
-                    if (lr == TH - 1) put(32 + lc);
-                    if (lc == 0) put(64 + lr);
-                    if (lc == TW - 1) put(96 + lr);
-                }
-                continue;
-            }
-            if (!__ballot(live != 0)) break;
-            if (worked && lane == 0)
-                __hip_atomic_fetch_add(&ctl->beat[(blockIdx.x % RES_BEATS) * 16], 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            worked = false;
+        const unsigned long long t_begin = wall_clock64();
+        auto poll = [&](auto arrived) -> int {
+            if (!__ballot(live != 0)) return 0;
             unsigned long long v[RPER];
 #pragma unroll
             for (int j = 0; j < RPER; j++) {
                 v[j] = EX_PENDING;
-                if ((live >> j) & 1u) v[j] = __hip_atomic_load(rx[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((live >> j) & 1u) v[j] = __hip_atomic_load(&ex[rx[j]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             bool got = false;
 #pragma unroll
             for (int j = 0; j < RPER; j++) {
                 const bool hit = v[j] != EX_PENDING;
+                if (!__ballot(hit)) continue;
+                got = true;
                 const bool dead = Cell::kCanDie && v[j] == EX_DEAD;
                 if (hit) {
                     live &= ~(1u << j);
                     if (!dead) cell.put(lds, rp[j], v[j]);
                 }
                 asm volatile("" ::: "memory");
-                got |= hit;
-                bool out = false;
-                hand_over(rp[j], hit ? rf[j] : 0u, dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu, out);
+                arrived(hit, rp[j], rf[j], dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu);
             }
-            if (__ballot(got)) {
+            if (got) {
                 idle = false;
-                continue;
+                return 2;
             }
-            // nothing new: leave once no tile has made progress for RES_IDLE ticks
+            // leave once no tile has made progress for RES_IDLE ticks
             const unsigned long long now = wall_clock64();
+            if (now - t_begin > RES_LIMIT) return 0;
             if (!idle || now - t_idle > RES_IDLE) {
                 const int b = __hip_atomic_load(&ctl->beat[lane % RES_BEATS * 16], __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_AGENT);
-                if (idle && !__ballot(b != beat0)) break;
+                if (idle && !__ballot(b != beat0)) return 0;
                 idle = true;
                 beat0 = b;
                 t_idle = now;
+            }
+            return 1;
+        };
+        if constexpr (SFD) {
+            int cur = -1;
+            uint32_t word = 0;
+            typename Cell::In in;
+            for (;;) {
+                take_cells(cell, lds, wd, queue, head, tail, cur, word, in);
+                if (!__ballot(cur >= 0)) {
+                    const int got = poll([&](bool hit, int, int r, uint32_t delta) {
+                        uint32_t old = 0;
+                        if (hit) old = atomicAdd(&wd[r], delta);
+                        const bool ready = hit && (old & W_CNT) == 1u;
+                        push(ready && cur >= 0, (uint32_t)r);
+                        if (ready && cur < 0) {
+                            cur = r;
+                            word = old + delta;
+                        }
+                    });
+                    if (got == 0) break;
+                    if (cur >= 0) in = cell.fetch(lds, cur);
+                    continue;
+                }
+                // a beat every 16 links, so that others do not leave while this
+                // tile works through a long stretch
+                follow_chains<TW>(cell, lds, wd, cur, word, in, 16, [&](bool out, int p, bool dead) {
+                    if (out) publish(p, dead ? EX_DEAD : cell.word(lds, p), true, true, true, true);
+                });
+                beat();
+            }
+        } else {
+            // Few cells are ready at a time (3 on average on fBm DEMs), each
+            // with up to eight receivers: eight lanes take a cell together, one
+            // receiver each, and all compute its value.  With 24 or more ready
+            // cells (a tile's first steps) every lane takes one.
+            const int g = lane >> 3, k8 = lane & 7;
+            const int off8 = koff<TW>(k8);
+            unsigned steps = 0;
+            bool worked = false;
+            for (;;) {
+                if (head == tail) {
+                    // a beat only for work done: waiting is no progress
+                    if (worked) beat();
+                    worked = false;
+                    const int got = poll([&](bool hit, int from, int f, uint32_t delta) {
+                        unsigned b = hit ? (unsigned)f : 0u;
+                        while (__ballot(b != 0)) {
+                            const int r = b ? from + koff<TW>(__ffs(b) - 1) : from;
+                            uint32_t old = 0;
+                            if (b) old = atomicAdd(&wd[r], delta);
+                            push(b && (old & W_CNT) == 1u, res_entry(old + delta, r));
+                            b &= b - 1;
+                        }
+                    });
+                    if (got == 0) break;
+                    continue;
+                }
+                worked = true;
+                if ((++steps & 15) == 0) beat();
+                const int n = tail - head;
+                const bool wide = n >= 24;
+                const int at = head + (wide ? lane : g);
+                const bool on = at < tail;
+                head += wide ? (n < 64 ? n : 64) : (n < 8 ? n : 8);
+                uint32_t e = 0;
+                if (on) e = queue[at];
+                const int p = on ? (int)(e & 0x7FFu) : PW + 1;
+                const unsigned bits = (e >> 16) & 0xFFu, f = e >> 24;
+                const bool dead = Cell::kCanDie && (e & 0x800u), upd = (e & 0x1000u) != 0;
+                const uint32_t delta = dead ? (W_DEAD1 - 1u) : 0xFFFFFFFFu;
+                const auto in = cell.fetch(lds, p);
+                if (on && (wide || k8 == 0)) {
+                    if (!dead) cell.set(lds, p, cell.result(in, bits), upd);
+                    wd[p] = ((uint32_t)(dead ? ST_DEAD : ST_DONE) << W_STSH) | W_NEVER | (upd ? W_UPD : 0u);
+                }
+                asm volatile("" ::: "memory");
+                bool out = false;   // a receiver lies in another tile
+                if (!wide) {
+                    const bool rcv = on && ((f >> k8) & 1u);
+                    uint32_t old = 0;
+                    if (rcv) old = atomicAdd(&wd[p + off8], delta);
+                    push(rcv && (old & W_CNT) == 1u, res_entry(old + delta, p + off8));
+                    const unsigned long long m = __ballot(rcv && ((old >> W_STSH) & 3u) == 3u);
+                    if (m) out = (m >> (8 * g)) & 0xFFu;
+                    if (out && k8 < 4)
+                        publish(p, dead ? EX_DEAD : cell.word(lds, p), k8 == 0, k8 == 1, k8 == 2, k8 == 3);
+                } else {
+                    // all eight neighbours' adds in flight at once, 0 for those
+                    // that are no receivers
+                    uint32_t old[8];
+                    if (on) {
+#pragma unroll
+                        for (int k = 0; k < 8; k++)
+                            old[k] = atomicAdd(&wd[p + poff<TW>(cpull(k))], ((f >> k) & 1u) ? delta : 0u);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const bool rcv = on && ((f >> k) & 1u);
+                        out |= rcv && ((old[k] >> W_STSH) & 3u) == 3u;
+                        push(rcv && (old[k] & W_CNT) == 1u, res_entry(old[k] + delta, p + poff<TW>(cpull(k))));
+                    }
+                    if (out) publish(p, dead ? EX_DEAD : cell.word(lds, p), true, true, true, true);
+                }
             }
         }
     }
@@ -1228,7 +1374,8 @@ __global__ void __launch_bounds__(256, Cell::kWaves) k_dag_resident(int W, int H
         prog = true;
         const long i = (long)(ty0 + li / TW) * W + (tx0 + li % TW);
         if (s2 == ST_DONE) {
-            cell.finish(lds, p, i, fin[q], (wv & W_UPD) != 0);
+            // read again rather than held in registers through the walk
+            cell.finish(lds, p, i, cell.final(cell.load(i)), (wv & W_UPD) != 0);
             st[i] = round;
         } else {
             st[i] = -(round + 1);
@@ -1276,11 +1423,12 @@ __global__ void k_iota(int n, int *a)
 }
 
 // Finishes the pass with resident tiles if the unfinished ones fit the chip
-// (*done = 1, the uncomputed cells in *uncomputed); *left: their number.  All
-// tiles fit: the launch takes the device's count and the host reads nothing
-// before it.
+// (*done = 1, the uncomputed cells in *uncomputed).  If all of the grid's tiles
+// do, the launch takes the device's count and the host reads nothing before
+// it.  over: by how many the unfinished tiles are too many, if by less than half.
 template <class Cell, bool SFD>
-static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, int *done, int prof_slot)
+static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, int *done, int prof_slot,
+                        int *over = nullptr)
 {
     *done = 0;
     const int ntiles = ((c->W + RES_T - 1) / RES_T) * ((c->H + RES_T - 1) / RES_T);
@@ -1300,7 +1448,10 @@ static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, i
             LEM_CHECK(c, hipMemcpyAsync(&c->hint[40], &ctl->n, sizeof(int), hipMemcpyDeviceToHost, c->s));
             LEM_CHECK(c, hipStreamSynchronize(c->s));
             n = c->hint[40];
-            if (n > cap) return LEMHIP_OK;
+            if (n > cap) {
+                if (over && n < cap + cap / 2) *over = n - cap;
+                return LEMHIP_OK;
+            }
         }
         ++*round;
         prof_begin(c, prof_slot);
@@ -1354,6 +1505,7 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
     c->hint[16] = ntiles;
     LEM_CHECK(c, hipMemcpyAsync(&ctl->cnt[(r + 1) % 3], &c->hint[16], sizeof(int), hipMemcpyHostToDevice, c->s));
     const int BATCH = c->dag_batch;
+    int batch = BATCH;
     // as many workgroups as the CUs hold at once (the first rounds visit every tile)
     int bpc = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_dag_round<TW, TH, Cell, SFD>, 256, 0) != hipSuccess || bpc < 1)
@@ -1377,17 +1529,20 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
     for (;;) {
         LEM_CHECK(c, hipMemsetAsync(&ctl->flag, 0, sizeof(int), c->s));
         prof_begin(c, prof_slot);
-        for (int q = 0; q < BATCH; q++) {
+        for (int q = 0; q < batch; q++) {
             ++r;
             k_dag_round<TW, TH, Cell, SFD><<<G, 256, 0, c->s>>>(c->W, c->H, r, cell, c->dmask, c->fd, st, L[r % 3],
                                                            L[(r + 1) % 3], c->dag_wake, ctl);
         }
-        prof_end(c, prof_slot, BATCH);
+        prof_end(c, prof_slot, batch);
         LEM_LAUNCHED(c);
         LEM_CHECK(c, hipMemcpyAsync(&c->hint[20], &ctl->flag, sizeof(int), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipStreamSynchronize(c->s));
         if (!c->hint[20]) break;
-        LEM_TRY((run_resident<std::remove_const_t<decltype(rcell)>, SFD>(c, rcell, &r, uncomputed, &done, prof_slot)));
+        int over = 0;
+        LEM_TRY((run_resident<std::remove_const_t<decltype(rcell)>, SFD>(c, rcell, &r, uncomputed, &done, prof_slot, &over)));
+        // not many more tiles than fit: look again soon
+        if (over > 0 && BATCH > 4) batch = 4;
         if (done) {
             c->dag_rounds_last = r - c->dag_round;
             c->dag_round = r;
