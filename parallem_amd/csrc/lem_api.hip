@@ -335,7 +335,7 @@ static int alloc_ctx(lemhip_ctx *c, const lem_params *p, int W, int H, int preci
     LEM_CHECK(c, hipHostMalloc((void **)&c->hscal, sizeof(LemScalars), hipHostMallocDefault));
     LEM_CHECK(c, hipHostMalloc((void **)&c->hdsc, sizeof(DemScal) * (LEM_MAX_SLOTS + 1), hipHostMallocDefault));
     LEM_CHECK(c, hipHostMalloc((void **)&c->hflags, sizeof(int) * (LEM_MAX_SLOTS + 1), hipHostMallocDefault));
-    LEM_CHECK(c, hipHostMalloc((void **)&c->hint, 64 * sizeof(int), hipHostMallocDefault));
+    LEM_CHECK(c, hipHostMalloc((void **)&c->hint, 128 * sizeof(int), hipHostMallocDefault));
     memset(c->hscal, 0, sizeof(LemScalars));
     memset(c->hdsc, 0, sizeof(DemScal) * (LEM_MAX_SLOTS + 1));
     memset(c->hflags, 0, sizeof(int) * (LEM_MAX_SLOTS + 1));

@@ -177,7 +177,7 @@ struct lemhip_ctx {
     void *stage = nullptr;        // pinned host staging for upload/download
     size_t stage_bytes = 0;
     hipEvent_t dl_ev[16] = {};    // one per pinned chunk of a large download
-    int *hint = nullptr;          // pinned host ints for small readbacks
+    int *hint = nullptr;          // pinned host ints for small readbacks (from 64: the plateau control block)
 
     // counters known on the host after each phase
     int h_rounds1 = 0, h_rounds2 = 0, h_nlab = 0, h_nedges = 0, h_sinkcount = 0, h_sinks1 = 0;

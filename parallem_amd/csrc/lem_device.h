@@ -95,9 +95,9 @@ struct LemScalars {
     int nedges;
     int plateau_rounds1, plateau_rounds2;
     int fa_uncomputed, sed_uncomputed;
-    int ncand;            // plateau candidates (mask cells without a downhill neighbour)
+    int ncand;            // sinks with an equal-height neighbour
+    int kept[2];          // edges left after a spill-height phase, by phase parity
     int flag;             // generic change flag for host-driven loops
-    int cut;              // some sink label has no path to label 0
     int w_bad;            // a mask cell's runoff weight is negative or not finite
     unsigned long long lowest_enc;
 };

@@ -386,9 +386,8 @@ static int fx_grid(long n)
 int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
 {
     *fallback = 0;
-    LEM_TRY(lem_read_slots(c));
     LEM_CHECK(c, hipMemcpyAsync(&c->hint[30], &c->scal->w_bad, sizeof(int), hipMemcpyDeviceToHost, c->s));
-    LEM_CHECK(c, hipStreamSynchronize(c->s));
+    LEM_TRY(lem_read_slots(c));
     if (c->hint[30]) { *fallback = 1; return LEMHIP_OK; }
     // per-slot shift: sums stay below 2^61 (the rounding adds at most N/2)
     for (int j = 0; j < c->nslot; j++) {
@@ -448,9 +447,15 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
         int *P = reinterpret_cast<int *>(c->sp0), *tp = reinterpret_cast<int *>(c->sp1);
         k_fx_parent<<<fx_grid(nex), 256, 0, c->s>>>(nex, a.ex_recv, a.xroot, a.exit_id, P);
         LEM_LAUNCHED(c);
-        for (int round = 0;; round++) {
-            LEM_CHECK(c, hipMemsetAsync(&c->scal->nlabels, 0, sizeof(int), c->s));
-            for (int q = 0; q < 2; q++) {
+        // rounds before the first host read: enough to double along a path
+        // that crosses every tile row and column twice (a read leaves the
+        // device idle for about 15 us, a round over a short list takes less);
+        // only a batch's last round reports changes
+        int batch = 2;
+        while ((1 << batch) < 4 * ((c->W + TW - 1) / TW + (c->H + TH - 1) / TH)) batch++;
+        for (int round = 0;; round += batch, batch = 2) {
+            for (int q = 0; q < batch; q++) {
+                if (q == batch - 1) LEM_CHECK(c, hipMemsetAsync(&c->scal->nlabels, 0, sizeof(int), c->s));
                 k_fx_gather<<<fx_grid(nex), 256, 0, c->s>>>(nex, a.ex_val, P, tv, tp);
                 k_fx_scatter<<<fx_grid(nex), 256, 0, c->s>>>(nex, a.ex_val, P, tv, tp, &c->scal->nlabels);
             }
@@ -458,7 +463,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
             LEM_CHECK(c, hipMemcpyAsync(&c->hint[32], &c->scal->nlabels, sizeof(int), hipMemcpyDeviceToHost, c->s));
             LEM_CHECK(c, hipStreamSynchronize(c->s));
             if (!c->hint[32]) break;
-            if (round > 32) { c->err = "exit forest did not converge"; return LEMHIP_E_NOT_CONVERGED; }
+            if (round > 64) { c->err = "exit forest did not converge"; return LEMHIP_E_NOT_CONVERGED; }
         }
     }
     // C: final sums, fa, tagged cells

@@ -218,8 +218,8 @@ template <typename TS>
 __global__ void __launch_bounds__(256) k_flowdirs(int W, int H, int cell_size, const double *__restrict__ z,
                                                   const uint8_t *__restrict__ mask, TS *__restrict__ slopes,
                                                   long plane, uint8_t *__restrict__ fd, uint8_t *__restrict__ SFD,
-                                                  uint8_t *__restrict__ eqb, int *__restrict__ cand,
-                                                  int *__restrict__ ncand)
+                                                  uint8_t *__restrict__ eqb, float *__restrict__ sp,
+                                                  int *__restrict__ cand, int *__restrict__ ncand)
 {
     constexpr int RW = 66, RH = 18, RN = RW * RH, PER = (RN + 255) / 256;
     __shared__ double zs[RN];
@@ -301,8 +301,15 @@ __global__ void __launch_bounds__(256) k_flowdirs(int W, int H, int cell_size, c
                 if ((flat + up) > 7 && up <= 7) { aspect = 0; aspectsfd = 0; }
                 if ((flat < 8) && (flat + up > 7)) { aspect = 0; aspectsfd = 0; }
             }
-            if (inside) { fd[self] = (uint8_t)aspect; SFD[self] = (uint8_t)aspectsfd; eqb[self] = (uint8_t)eq; }
-            if (active && aspect == 0 && aspectsfd == 0) cand_rows |= 1u << (sub * 4 + rg);
+            const bool is_cand = active && aspect == 0 && aspectsfd == 0;
+            if (inside) {
+                fd[self] = (uint8_t)aspect;
+                SFD[self] = (uint8_t)aspectsfd;
+                eqb[self] = (uint8_t)eq;
+                // candidates start at 2e7 (newflow.cu:252), the rest keep 0 and never change
+                sp[self] = is_cand ? 20000000.0f : 0.0f;
+            }
+            if (is_cand) cand_rows |= 1u << (sub * 4 + rg);
         }
     }
     // one append per block for its candidates (their order is not needed)
@@ -330,54 +337,6 @@ __global__ void __launch_bounds__(256) k_flowdirs(int W, int H, int cell_size, c
 // tile width and height: in it or in one of its 8 neighbour tiles); tiles
 // without candidates never change.
 
-__global__ void k_sp_init(long N, float *sp)
-{
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) sp[i] = 0.0f;
-}
-
-// candidates start at 2e7 (newflow.cu:252); non-candidates keep 0 and never change
-__global__ void k_sp_seed(int W, const int *cand, int n, float *sp, int ntx, int *tile_has)
-{
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int i = cand[k];
-    sp[i] = 20000000.0f;
-    int t = ((i / W) / PTH) * ntx + (i % W) / PTW;
-    if (tile_has[t] == 0) tile_has[t] = 1;
-}
-
-// A candidate with an equal-height neighbour at distance 0 (not a
-// candidate, or off the grid, where the plateau rounds read 0) takes its
-// distance in the first round; every other cell changes in round r only if
-// an equal-height neighbour changed in round r-1, i.e. it lies within r-1
-// cells of such a seed.  The first launch's K rounds (K <= tile height) can
-// therefore change only tiles in the 3x3 tile neighbourhood of a seed's
-// tile: those tiles (with candidates) are marked 3, the first list.
-__global__ void k_sp_seedmark(int W, int H, const int *cand, int n, const float *sp, const uint8_t *eqb, int ntx,
-                              int nty, int *tile_has)
-{
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const int i = cand[k];
-    const int y = i / W, x = i % W;
-    const unsigned e = eqb[i];
-    bool seed = false;
-#pragma unroll
-    for (int d = 0; d < 8; d++) {
-        const int yy = y + cdy(d), xx = x + cdx(d);
-        if ((e >> d) & 1u) seed |= yy < 0 || yy >= H || xx < 0 || xx >= W || sp[(long)yy * W + xx] == 0.0f;
-    }
-    if (!seed) return;
-    const int ty = y / PTH, tx = x / PTW;
-    for (int dy = -1; dy <= 1; dy++)
-        for (int dx = -1; dx <= 1; dx++) {
-            const int t2y = ty + dy, t2x = tx + dx;
-            if (t2y < 0 || t2y >= nty || t2x < 0 || t2x >= ntx) continue;
-            const int t2 = t2y * ntx + t2x;
-            if (tile_has[t2] != 0) tile_has[t2] = 3;
-        }
-}
-
 // Launch bookkeeping: launch L visits list L % 3 (count cnt[L % 3]); a tile
 // still moving at its end queues itself and its neighbours with candidates in
 // list (L+1) % 3, each once (stamp[tile] holds the last launch it was queued
@@ -387,8 +346,68 @@ struct PlatCtl {
     int cnt[3];
     int pad0[29];
     int last_change;   // last round (absolute number) in which any cell changed
-    int pad1[31];
+    int ncand;         // plateau candidates (mask cells without a downhill neighbour)
+    int cut;           // some sink label has no path to label 0 (pass 2: known after the surface was raised)
+    int pad1[29];
 };
+
+// everything a pass starts from but its distances
+__global__ void k_plat_init(int ntiles, int *tile_has, int *tver, PlatCtl *ctl)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < ntiles) {
+        tile_has[t] = 0;
+        tver[t] = -2;   // buffer 0, written before any launch
+    }
+    if (t < 3) ctl->cnt[t] = 0;
+    if (t == 3) ctl->last_change = 0;
+    if (t == 4) ctl->ncand = 0;
+}
+
+// the tiles with candidates (their number is read on the device, so the host
+// does not wait for it)
+__global__ void k_sp_seed(int W, const int *cand, const PlatCtl *ctl, int ntx, int *tile_has)
+{
+    const int n = ctl->ncand;
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const int i = cand[k];
+        const int t = ((i / W) / PTH) * ntx + (i % W) / PTW;
+        if (tile_has[t] == 0) tile_has[t] = 1;
+    }
+}
+
+// A candidate with an equal-height neighbour at distance 0 (not a
+// candidate, or off the grid, where the plateau rounds read 0) takes its
+// distance in the first round; every other cell changes in round r only if
+// an equal-height neighbour changed in round r-1, i.e. it lies within r-1
+// cells of such a seed.  The first launch's K rounds (K <= tile height) can
+// therefore change only tiles in the 3x3 tile neighbourhood of a seed's
+// tile: those tiles (with candidates) are marked 3, the first list.
+__global__ void k_sp_seedmark(int W, int H, const int *cand, const PlatCtl *ctl, const float *sp, const uint8_t *eqb,
+                              int ntx, int nty, int *tile_has)
+{
+    const int n = ctl->ncand;
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const int i = cand[k];
+        const int y = i / W, x = i % W;
+        const unsigned e = eqb[i];
+        bool seed = false;
+#pragma unroll
+        for (int d = 0; d < 8; d++) {
+            const int yy = y + cdy(d), xx = x + cdx(d);
+            if ((e >> d) & 1u) seed |= yy < 0 || yy >= H || xx < 0 || xx >= W || sp[(long)yy * W + xx] == 0.0f;
+        }
+        if (!seed) continue;
+        const int ty = y / PTH, tx = x / PTW;
+        for (int dy = -1; dy <= 1; dy++)
+            for (int dx = -1; dx <= 1; dx++) {
+                const int t2y = ty + dy, t2x = tx + dx;
+                if (t2y < 0 || t2y >= nty || t2x < 0 || t2x >= ntx) continue;
+                const int t2 = t2y * ntx + t2x;
+                if (tile_has[t2] != 0) tile_has[t2] = 3;
+            }
+    }
+}
 
 __global__ void k_plat_first_list(int ntiles, const int *tile_has, int *list, PlatCtl *ctl, int slot)
 {
@@ -418,12 +437,6 @@ __device__ __forceinline__ int plat_buf_as_of(int tv, int launch)
 {
     int b = tv & 1;
     return (tv >> 1) == launch ? 1 - b : b;
-}
-
-__global__ void k_plat_tver_init(int ntiles, int *tver)
-{
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < ntiles) tver[t] = -2;   // buffer 0, written before any launch
 }
 
 // Appends a workgroup's queued tiles to the next launch's list with one
@@ -953,12 +966,12 @@ __global__ void __launch_bounds__(256) k_edges_emit(int W, int H, const uint8_t 
 }
 
 // unique pairs (sorted) to the edge list; label flags as in the compaction
-__global__ void k_edges_decode(int ne, const unsigned long long *ukeys, const unsigned long long *uw, int B,
+__global__ void k_edges_decode(const int *cnt, const unsigned long long *ukeys, const unsigned long long *uw, int B,
                                uint32_t *elo, uint32_t *ehi, unsigned long long *ew, uint8_t *seen,
                                const uint8_t *labdem, DemScal *ds)
 {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= ne) return;
+    if (k >= *cnt) return;
     unsigned long long key = ukeys[k];
     uint32_t lo = (uint32_t)(key >> B), hi = (uint32_t)(key & ((1ULL << B) - 1));
     elo[k] = lo;
@@ -1069,13 +1082,13 @@ __global__ void k_bv_init(long n, uint32_t *comp, unsigned long long *mv, unsign
 // (a minimum over edges of one component, in any grouping) and only the
 // run's first lane updates the component, instead of one atomic per lane
 // on the same address; the same for runs on the hi side.
-__global__ void __launch_bounds__(256) k_bv_min_w(int ne, const uint32_t *__restrict__ lo,
+__global__ void __launch_bounds__(256) k_bv_min_w(const int *cnt, const uint32_t *__restrict__ lo,
                                                   const uint32_t *__restrict__ hi,
                                                   const unsigned long long *__restrict__ w,
                                                   const uint32_t *__restrict__ comp, unsigned long long *bw)
 {
     const unsigned long long INF = ord_enc(lm_inf());
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, ne = *cnt;
     const int lane = threadIdx.x & 63;
     bool live = false;
     unsigned long long wk = ~0ULL;
@@ -1107,13 +1120,13 @@ __global__ void __launch_bounds__(256) k_bv_min_w(int ne, const uint32_t *__rest
 }
 
 // the first edge of that weight
-__global__ void k_bv_min_e(int ne, const uint32_t *__restrict__ lo, const uint32_t *__restrict__ hi,
+__global__ void k_bv_min_e(const int *cnt, const uint32_t *__restrict__ lo, const uint32_t *__restrict__ hi,
                            const unsigned long long *__restrict__ w, const uint32_t *__restrict__ comp,
                            const unsigned long long *__restrict__ bw, uint32_t *be)
 {
     const unsigned long long INF = ord_enc(lm_inf());
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= ne) return;
+    if (k >= *cnt) return;
     const unsigned long long wk = w[k];
     const uint32_t ca = comp[lo[k]], cb = comp[hi[k]];
     if (ca == cb || wk >= INF) return;
@@ -1220,7 +1233,7 @@ __global__ void k_bv_labels(long n, uint32_t *comp, const unsigned long long *__
 // lists: with 16, the 27 K edges of a 512^2 DEM ran in 7 workgroups, 14.6 us a
 // phase; on long ones fewer workgroups add to the one counter)
 template <int ITEMS>
-__global__ void __launch_bounds__(256) k_bv_keep(int ne, const uint32_t *elo, const uint32_t *ehi,
+__global__ void __launch_bounds__(256) k_bv_keep(const int *cnt, const uint32_t *elo, const uint32_t *ehi,
                                                  const unsigned long long *ew, const uint32_t *comp, uint32_t *lo2,
                                                  uint32_t *hi2, unsigned long long *w2, int *count)
 {
@@ -1228,7 +1241,7 @@ __global__ void __launch_bounds__(256) k_bv_keep(int ne, const uint32_t *elo, co
     __shared__ int s_base;
     const unsigned long long INF = ord_enc(lm_inf());
     compact_chunks_ordered<ITEMS>(
-        ne, count, s_wave, &s_base, [&](long k) { return ew[k] < INF && comp[elo[k]] != comp[ehi[k]]; },
+        *cnt, count, s_wave, &s_base, [&](long k) { return ew[k] < INF && comp[elo[k]] != comp[ehi[k]]; },
         [&](long k, int at) { lo2[at] = elo[k]; hi2[at] = ehi[k]; w2[at] = ew[k]; });
 }
 
@@ -1381,9 +1394,9 @@ static int plat_grids(lemhip_ctx *c)
 
 // FlowDirs + plateau routing on surface zs; slopes == nullptr for pass 2.
 // Leaves the candidate list in c->cand and its length in *ncand_out; returns
-// the number of rounds that changed something in *rounds.  cut (pass 2): set,
-// and the pass left before its plateau rounds, when labels turn out to be cut
-// off from label 0.
+// the number of rounds that changed something in *rounds, all read after the
+// first launches.  cut (pass 2): set, and the pass left, when labels turn out
+// to be cut off from label 0.
 template <typename TS>
 static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, int *ncand_out, int *rounds,
                                    bool *cut = nullptr)
@@ -1391,24 +1404,6 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
     long N = c->N;
     int W = c->W, H = c->H;
     uint8_t *eqb = c->dmask;   // equal-height neighbour bits; the accumulation passes reuse the buffer later
-    LEM_CHECK(c, hipMemsetAsync(&c->scal->ncand, 0, sizeof(int), c->s));
-    dim3 blk(64, 4);
-    dim3 grd((W + 63) / 64, (H + 63) / 64);
-    prof_begin(c, PROF_FLOWDIRS);
-    k_flowdirs<TS><<<grd, blk, 0, c->s>>>(W, H, (int)c->p.cellsize, zs, c->mask, slopes, c->NP, c->fd, c->SFD, eqb,
-                                          c->cand, &c->scal->ncand);
-    prof_end(c, PROF_FLOWDIRS);
-    LEM_LAUNCHED(c);
-    LEM_TRY(read_scalars(c));
-    int n = c->hscal->ncand;
-    *ncand_out = n;
-    *rounds = 0;
-    if (cut) {
-        *cut = c->hscal->cut != 0;
-        if (*cut) return LEMHIP_OK;
-    }
-    if (n == 0) return LEMHIP_OK;
-    prof_begin(c, PROF_PLATEAU);
     const int ntx = (W + PTW - 1) / PTW, nty = (H + PTH - 1) / PTH, ntiles = ntx * nty;
     int *tile_has = c->pl_tiles, *tstamp = c->pl_tiles + ntiles, *tver = c->pl_tiles + 5 * (long)ntiles;
     int *L[3] = {c->pl_tiles + 2 * (long)ntiles, c->pl_tiles + 3 * (long)ntiles, c->pl_tiles + 4 * (long)ntiles};
@@ -1419,12 +1414,19 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
         LEM_CHECK(c, hipMemsetAsync(tstamp, 0, ntiles * sizeof(int), c->s));
         launch = 0;
     }
-    LEM_CHECK(c, hipMemsetAsync(tile_has, 0, ntiles * sizeof(int), c->s));
-    LEM_CHECK(c, hipMemsetAsync(ctl, 0, sizeof(PlatCtl), c->s));
-    k_sp_init<<<grid1d(N), 256, 0, c->s>>>(N, sp_in);
-    k_plat_tver_init<<<(ntiles + 255) / 256, 256, 0, c->s>>>(ntiles, tver);
-    k_sp_seed<<<grid1d(n, 256, 1 << 30), 256, 0, c->s>>>(W, c->cand, n, sp_in, ntx, tile_has);
-    k_sp_seedmark<<<grid1d(n, 256, 1 << 30), 256, 0, c->s>>>(W, H, c->cand, n, sp_in, eqb, ntx, nty, tile_has);
+    k_plat_init<<<(ntiles + 255) / 256, 256, 0, c->s>>>(ntiles, tile_has, tver, ctl);
+    dim3 blk(64, 4);
+    dim3 grd((W + 63) / 64, (H + 63) / 64);
+    prof_begin(c, PROF_FLOWDIRS);
+    k_flowdirs<TS><<<grd, blk, 0, c->s>>>(W, H, (int)c->p.cellsize, zs, c->mask, slopes, c->NP, c->fd, c->SFD, eqb,
+                                          sp_in, c->cand, &ctl->ncand);
+    prof_end(c, PROF_FLOWDIRS);
+    LEM_LAUNCHED(c);
+    prof_begin(c, PROF_PLATEAU);
+    // about a tenth of the cells or fewer are candidates
+    const int gc = grid1d(N / 16, 256, 8192);
+    k_sp_seed<<<gc, 256, 0, c->s>>>(W, c->cand, ctl, ntx, tile_has);
+    k_sp_seedmark<<<gc, 256, 0, c->s>>>(W, H, c->cand, ctl, sp_in, eqb, ntx, nty, tile_has);
     k_plat_first_list<<<grid1d(ntiles, 256, 1024), 256, 0, c->s>>>(ntiles, tile_has, L[launch % 3], ctl, launch % 3);
     LEM_LAUNCHED(c);
     // Eight rounds per launch while many tiles move (with 16 throughout, the
@@ -1441,6 +1443,7 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
         for (int q = 0; q < 2; q++) G[q] = c->plat_grid[q][slopes ? 1 : 0];
     }
     int r = 0;  // rounds done in this pass
+    int n = 0;
     long guard = 0;
     // launches between host checks (an empty launch costs less than a read);
     // the first pass seldom has a flat to drain
@@ -1469,10 +1472,17 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
         }
         prof_end(c, PROF_PLAT_K, batch);
         LEM_LAUNCHED(c);
-        LEM_CHECK(c, hipMemcpyAsync(&c->hint[24], ctl, 3 * sizeof(int), hipMemcpyDeviceToHost, c->s));
-        LEM_CHECK(c, hipMemcpyAsync(&c->hint[27], &ctl->last_change, sizeof(int), hipMemcpyDeviceToHost, c->s));
+        PlatCtl *h = reinterpret_cast<PlatCtl *>(c->hint + 64);
+        LEM_CHECK(c, hipMemcpyAsync(h, ctl, sizeof(PlatCtl), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipStreamSynchronize(c->s));
-        const int moving = c->hint[24 + launch % 3];
+        n = h->ncand;
+        *ncand_out = n;
+        *rounds = h->last_change;
+        if (cut) {
+            *cut = h->cut != 0;
+            if (*cut) break;   // the surface has to be raised again: this pass is repeated
+        }
+        const int moving = h->cnt[launch % 3];
         if (moving == 0) break;   // nothing queued for the next launch
         if (widen && moving <= c->ncu) K = 16;
         // every launch with a moving tile changes at least one cell, and a
@@ -1480,7 +1490,6 @@ static int directions_and_plateaus(lemhip_ctx *c, const double *zs, TS *slopes, 
         if (++guard > (long)n + 2) { c->err = "plateau routing did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
     c->pl_launch = launch;
-    *rounds = c->hint[27];
     prof_end(c, PROF_PLATEAU, *rounds + 1);
     return LEMHIP_OK;
 }
@@ -1566,14 +1575,20 @@ static int cutoff_components(lemhip_ctx *c, int nlab, int ne)
 
 #define BV_KEEP_SHORT (1 << 20)
 // Spill heights of the labels into c->rmm (initialised: label 0 -inf, the
-// rest +inf) by Borůvka phases over the label-sorted edge list.
-static int spill_heights(lemhip_ctx *c, int nlab, int ne)
+// rest +inf) by Borůvka phases over the label-sorted edge list, whose length
+// is in scal->nedges (at most `bound`, read with the first counts).  Two phases
+// run between host reads: the kernels take the edge counts from the device and
+// their grids from the last count the host knows.  A read leaves the device
+// idle for about 15 us, as long as the phase itself on short lists (a step at
+// 512^2 with seven reads fewer, these among them: 1.80 instead of 1.88 ms).
+static int spill_heights(lemhip_ctx *c, int nlab, int bound)
 {
     const long n = (long)nlab + 1;
-    if (ne <= 0) return LEMHIP_OK;
-    // per-label scratch: running maxima, chosen weights (parity 1) and the two
-    // scalars in the hash value table, chosen edges and roots in the hash key
-    // table (both >= 8 * (nlab + 1) entries of 8 bytes), chosen weights
+    c->h_nedges = 0;
+    if (bound <= 0) return LEMHIP_OK;
+    // per-label scratch: running maxima, chosen weights (parity 1) and label
+    // 0's scalars in the hash value table, chosen edges and roots in the hash
+    // key table (both >= 8 * (nlab + 1) entries of 8 bytes), chosen weights
     // (parity 0) in cmax
     unsigned long long *mv = c->hvals, *bw[2] = {c->cmax, c->hvals + n}, *st = c->hvals + 2 * n;
     uint32_t *be[2] = {reinterpret_cast<uint32_t *>(c->hkeys), reinterpret_cast<uint32_t *>(c->hkeys) + n};
@@ -1582,40 +1597,43 @@ static int spill_heights(lemhip_ctx *c, int nlab, int ne)
     LEM_LAUNCHED(c);
     const uint32_t *lo = c->elo, *hi = c->ehi;
     const unsigned long long *w = c->ew;
-    int na = ne, buf = 0;
+    const int *cnt = &c->scal->nedges;
     LEM_TRY(clear_flag(c));   // raised only by a pointer walk that does not end
     // the profile slot times the kernels only, not the host reads between them
-    for (int ph = 0; na > 0; ph++) {
-        const int p = ph & 1;
-        const int ge = grid1d(na, 256, 1 << 30);
-        uint32_t *lo2 = c->elo2[buf], *hi2 = c->ehi2[buf];
-        unsigned long long *w2 = c->ew2[buf];
-        prof_begin(c, PROF_MM_K);
-        k_bv_min_w<<<ge, 256, 0, c->s>>>(na, lo, hi, w, c->comp, bw[p]);
-        k_bv_min_e<<<ge, 256, 0, c->s>>>(na, lo, hi, w, c->comp, bw[p], be[p]);
-        k_bv_hook<<<grid1d(n), 256, 0, c->s>>>(n, lo, hi, c->comp, be[p], nxt, &c->scal->nedges);
-        // two launches of four links leave short chains; the label kernel
-        // walks the rest (no host read per phase for the jumps)
-        for (int q = 0; q < 2; q++) k_bv_jump<<<grid1d(n), 256, 0, c->s>>>(n, nxt);
-        k_bv_labels<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, bw[p], be[p], nxt, mv, c->rmm, st + 2 * p,
-                                                  st + 2 * (p ^ 1), bw[p ^ 1], be[p ^ 1], &c->scal->flag);
-        if (na <= BV_KEEP_SHORT)
-            k_bv_keep<4><<<grid_chunks(na, 8192, 4), 256, 0, c->s>>>(na, lo, hi, w, c->comp, lo2, hi2, w2,
-                                                                     &c->scal->nedges);
-        else
-            k_bv_keep<COMPACT_ITEMS><<<grid_chunks(na), 256, 0, c->s>>>(na, lo, hi, w, c->comp, lo2, hi2, w2,
-                                                                        &c->scal->nedges);
-        prof_end(c, PROF_MM_K, 7);
-        LEM_LAUNCHED(c);
+    for (int ph = 0, na = bound; na > 0;) {
+        for (int q = 0; q < 2; q++, ph++) {
+            const int p = ph & 1;
+            const int ge = grid1d(na, 256, 1 << 30);
+            uint32_t *lo2 = c->elo2[p], *hi2 = c->ehi2[p];
+            unsigned long long *w2 = c->ew2[p];
+            int *kept = &c->scal->kept[p];
+            prof_begin(c, PROF_MM_K);
+            k_bv_min_w<<<ge, 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, bw[p]);
+            k_bv_min_e<<<ge, 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, bw[p], be[p]);
+            k_bv_hook<<<grid1d(n), 256, 0, c->s>>>(n, lo, hi, c->comp, be[p], nxt, kept);
+            // two launches of four links leave short chains; the label kernel
+            // walks the rest (no host read per phase for the jumps)
+            for (int j = 0; j < 2; j++) k_bv_jump<<<grid1d(n), 256, 0, c->s>>>(n, nxt);
+            k_bv_labels<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, bw[p], be[p], nxt, mv, c->rmm, st + 2 * p,
+                                                      st + 2 * (p ^ 1), bw[p ^ 1], be[p ^ 1], &c->scal->flag);
+            if (na <= BV_KEEP_SHORT)
+                k_bv_keep<4><<<grid_chunks(na, 8192, 4), 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, lo2, hi2, w2, kept);
+            else
+                k_bv_keep<COMPACT_ITEMS><<<grid_chunks(na), 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, lo2, hi2, w2,
+                                                                            kept);
+            prof_end(c, PROF_MM_K, 7);
+            LEM_LAUNCHED(c);
+            lo = lo2; hi = hi2; w = w2;
+            cnt = kept;
+        }
         LEM_TRY(read_scalars(c));
+        c->h_nedges = c->hscal->nedges;
         if (c->hscal->flag) { c->err = "spill-height component pointers form a cycle"; return LEMHIP_E_NOT_CONVERGED; }
-        const int nk = c->hscal->nedges;
+        const int nk = c->hscal->kept[(ph - 1) & 1];
         // every component with an outgoing edge joins another each phase, so
         // the components with edges at least halve
-        if (nk >= na && ph > 0) { c->err = "spill-height phases made no progress"; return LEMHIP_E_NOT_CONVERGED; }
+        if (nk >= na && ph > 2) { c->err = "spill-height phases made no progress"; return LEMHIP_E_NOT_CONVERGED; }
         na = nk;
-        lo = lo2; hi = hi2; w = w2;
-        buf ^= 1;
         if (ph > 64) { c->err = "spill-height phases did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
     return LEMHIP_OK;
@@ -1629,8 +1647,10 @@ static int raise_surface(lemhip_ctx *c)
 }
 
 
-// floodingDriver (routeflow.cu:202-676) up to the raised surface in c->z2
-static int flooding(lemhip_ctx *c, int ncand1)
+// floodingDriver (routeflow.cu:202-676) up to the raised surface in c->z2.
+// *sinks: the sinks pass 1 left, counted per DEM on the device and read with
+// the label count; with none of them nothing is flooded.
+static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
 {
     long N = c->N;
     int W = c->W, H = c->H;
@@ -1654,12 +1674,15 @@ static int flooding(lemhip_ctx *c, int ncand1)
     // sink merge over the sinks that have an equal-height neighbour (list in the
     // prefix buffer, free after k_init_ws)
     int *mlist = reinterpret_cast<int *>(c->z2);
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[1], prefix + (N - 1), sizeof(int), hipMemcpyDeviceToHost, c->s));
     LEM_CHECK(c, hipMemsetAsync(&c->scal->ncand, 0, sizeof(int), c->s));
     k_merge_list<<<grid1d(ncand1, 256, 4096), 256, 0, c->s>>>(c->cand, ncand1, c->SFD, c->dmask, mlist,
                                                              &c->scal->ncand);
     LEM_LAUNCHED(c);
+    LEM_CHECK(c, hipMemcpyAsync(c->hdsc, c->dsc, sizeof(DemScal) * c->nslot, hipMemcpyDeviceToHost, c->s));
     LEM_TRY(read_scalars(c));
+    *sinks = 0;
+    for (int j = 0; j < c->nslot; j++) *sinks += c->hdesc[j].w > 0 ? c->hdsc[j].sinks_pass1 : 0;
+    if (*sinks == 0) return LEMHIP_OK;
     const int nlab = c->hint[0] + c->hint[1];
     c->h_nlab = nlab;
     const int nm = c->hscal->ncand;
@@ -1707,7 +1730,6 @@ static int flooding(lemhip_ctx *c, int ncand1)
     k_minimax_init<<<grid1d(nlab + 1), 256, 0, c->s>>>(nlab + 1, c->rmm, c->seen);
     k_slots_sinkcount_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc);
     LEM_LAUNCHED(c);
-    int ne = 0;
     if (np > 0) {
         unsigned long long *skeys = c->ew2[0], *svals = c->ew2[1];
         size_t need3 = 0, need4 = 0;
@@ -1728,21 +1750,20 @@ static int flooding(lemhip_ctx *c, int ncand1)
         t3 = c->cub_bytes;
         LEM_CHECK(c, hipcub::DeviceReduce::ReduceByKey(c->cub_tmp, t3, skeys, c->hkeys, svals, c->hvals,
                                                         &c->scal->nedges, hipcub::Min(), (int)np, c->s));
-        LEM_TRY(read_scalars(c));
-        ne = c->hscal->nedges;
-        k_edges_decode<<<(ne + 255) / 256, 256, 0, c->s>>>(ne, c->hkeys, c->hvals, B, c->elo, c->ehi, c->ew, c->seen,
-                                                          c->labdem, c->dsc);
+        k_edges_decode<<<((int)np + 255) / 256, 256, 0, c->s>>>(&c->scal->nedges, c->hkeys, c->hvals, B, c->elo, c->ehi,
+                                                                c->ew, c->seen, c->labdem, c->dsc);
         LEM_LAUNCHED(c);
     }
     k_count_labels<<<grid1d(nlab + 1, 256, 1024), 256, 0, c->s>>>(nlab + 1, c->seen, c->labdem, c->nslot, c->dsc);
     LEM_LAUNCHED(c);
-    c->h_nedges = ne;
 
-    LEM_TRY(spill_heights(c, nlab, ne));
-    // labels cut off from label 0 (NaN heights only) raise scal->cut, read with
-    // the next pass's candidate count: the surface is raised before it is known
-    LEM_CHECK(c, hipMemsetAsync(&c->scal->cut, 0, sizeof(int), c->s));
-    if (ne > 0) k_fb_unreached<<<grid1d(ne, 256, 1 << 30), 256, 0, c->s>>>(ne, c->elo, c->ehi, c->rmm, &c->scal->cut);
+    LEM_TRY(spill_heights(c, nlab, (int)np));
+    // labels cut off from label 0 (NaN heights only) raise the flag read with
+    // the next pass's first counts: the surface is raised before it is known
+    int *cut = &reinterpret_cast<PlatCtl *>(c->pl_ctl)->cut;
+    LEM_CHECK(c, hipMemsetAsync(cut, 0, sizeof(int), c->s));
+    const int ne = c->h_nedges;
+    if (ne > 0) k_fb_unreached<<<grid1d(ne, 256, 1 << 30), 256, 0, c->s>>>(ne, c->elo, c->ehi, c->rmm, cut);
     return raise_surface(c);
 }
 
@@ -1804,22 +1825,22 @@ static int fd_phase_t(lemhip_ctx *c, int iter)
         k_count_sinks<<<grid1d(n1, 256, 2048), 256, 0, c->s>>>(c->cand, n1, c->SFD, c->demid, c->nslot, c->dsc);
         LEM_LAUNCHED(c);
     }
-    LEM_TRY(lem_read_slots(c));
-    int sinks = 0;
-    for (int j = 0; j < c->nslot; j++) sinks += c->hdesc[j].w > 0 ? c->hdsc[j].sinks_pass1 : 0;
-
-    c->h_sinks1 = sinks;
     c->h_rounds1 = r1;
     c->h_rounds2 = 0;
     c->h_nlab = 0;
     c->h_nedges = 0;
-    c->h_sinkcount = sinks;
-    if (sinks == 0) k_slots_sinkcount_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc);
-    if (sinks > 0) {
-        prof_begin(c, PROF_FLOOD);
-        LEM_TRY(flooding(c, n1));
+    prof_begin(c, PROF_FLOOD);
+    int sinks = 0;
+    if (n1 > 0) LEM_TRY(flooding(c, n1, &sinks));
+    if (sinks > 0)
         k_slots_sinkcount_fin<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->ddesc, c->nslot, c->dsc);
-        prof_end(c, PROF_FLOOD);
+    prof_end(c, PROF_FLOOD);
+    c->h_sinks1 = sinks;
+    c->h_sinkcount = sinks;
+    if (sinks == 0) {
+        c->h_nlab = 0;
+        k_slots_sinkcount_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc);
+    } else {
         int n2 = 0, r2 = 0;
         bool cut = false;
         LEM_TRY(directions_and_plateaus<TS>(c, c->z2, (TS *)nullptr, &n2, &r2, &cut));
