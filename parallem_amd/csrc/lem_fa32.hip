@@ -14,14 +14,15 @@
 //
 // Two passes over tiles of TW x TH cells with a small global solve between:
 //   A. each tile sums its own subtrees in LDS by pointer doubling (round t
-//      adds every cell's partial sum to its 2^t-th in-tile ancestor), finds
-//      each cell's in-tile root, and lists its exits (cells whose receiver is
-//      in another tile) with their in-tile sums;
+//      adds every cell's partial sum to its 2^t-th in-tile ancestor), which
+//      also finds each cell's in-tile root, lists its exits (cells whose
+//      receiver is in another tile) with their in-tile sums, and leaves every
+//      in-tile sum in the cell's fa entry;
 //   B. the exits form a forest of their own (an exit's parent is the exit
 //      its receiver's in-tile path leads to); the same doubling over that
 //      forest gives every exit its final value;
-//   C. each tile sums its subtrees again with the final values of the exits
-//      that flow into it added at their receivers, and writes fa.
+//   C. each tile adds the final values of the exits that flow into it along
+//      their in-tile paths, and writes fa.
 //
 // Cycles: fd[outlet] = WEST can close a cycle through the outlet (the only
 // possible one: every other link goes strictly downhill or down a plateau's
@@ -33,7 +34,9 @@
 #include "lem_ctx.h"
 
 #define FX_TAG (1ULL << 62)
-#define FX_NONE 0xFFFFu
+#define FX_NONE 0xFFFFu   // no receiver
+#define FX_EXIT 0xFFFEu   // the receiver is in another tile
+#define FX_ROOT 0x8000u   // pass A: the pointer has reached the path's root
 
 // direction index of a single ESRI code, -1 for 0 or a multi-bit code
 __device__ __forceinline__ int fx_dir(uint8_t code)
@@ -70,7 +73,8 @@ struct FxArgs {
     const float *w;
     const DemScal *ds;
     const int *shift;            // per slot
-    // pass A outputs / pass C inputs
+    int nslot;
+    // pass A outputs / pass C inputs (and the in-tile sums, in fa)
     int *exit_id;                // per cell (exits only)
     int *xroot;                  // per cell (tile border cells only): exit its in-tile path leads to, or -1
     unsigned long long *ex_val;  // per exit: in-tile sum (A), final value after the forest solve
@@ -118,178 +122,280 @@ __device__ __forceinline__ int fx_block_append(int *counter, int n, int *s_wave,
 // neighbours in other tiles (or off the grid)
 template <int TW> __device__ __forceinline__ int fx_pad(int lr, int lc) { return (lr + 1) * (TW + 2) + lc + 1; }
 
-template <int TW, int TH, bool FINAL>
-__global__ void __launch_bounds__(256) k_fx_tile(FxArgs a)
+// A tile's directions, mask and links in LDS
+template <int TW, int TH>
+struct FxTile {
+    static constexpr int NC = TW * TH, PER = NC / 256, PW = TW + 2, NP = (TW + 2) * (TH + 2);
+    static constexpr int NPPER = (NP + 255) / 256, NB = 2 * TW + 2 * (TH - 2);
+    static_assert(NC % 256 == 0 && NB <= 256 && NC <= (int)FX_ROOT, "tile shape");
+    unsigned long long x[NC];
+    uint16_t J[NC];   // pointer of the doubling (A); receiver in the tile, FX_EXIT or FX_NONE (C)
+    uint8_t sfd[NP], smk[NP];
+    int outlet[LEM_MAX_SLOTS + 1], shift[LEM_MAX_SLOTS + 1];   // per DEM
+};
+
+template <int TW, int TH> __device__ __forceinline__ void fx_slots(const FxArgs &a, FxTile<TW, TH> &T)
 {
-    constexpr int NC = TW * TH, PER = NC / 256, PW = TW + 2, NP = (TW + 2) * (TH + 2);
-    constexpr int NPPER = (NP + 255) / 256;
-    static_assert(NC % 256 == 0, "tile shape");
-    __shared__ unsigned long long x[NC];
-    __shared__ uint16_t J[NC];
-    __shared__ uint16_t R[FINAL ? 1 : NC];
-    __shared__ uint8_t sfd[NP], smk[NP];
-    __shared__ uint8_t isexit[FINAL ? 1 : NC];
+    for (int s = threadIdx.x; s < a.nslot; s += 256) {
+        T.outlet[s] = a.ds[s].outlet;
+        T.shift[s] = a.shift[s];
+    }
+}
+
+// border cell k of a tile: the first and last row, then the two columns
+template <int TW, int TH>
+__device__ __forceinline__ void fx_border(int k, int &lr, int &lc)
+{
+    if (k < 2 * TW) {
+        lr = k < TW ? 0 : TH - 1;
+        lc = k < TW ? k : k - TW;
+    } else {
+        lr = 1 + ((k - 2 * TW) >> 1);
+        lc = (k & 1) ? TW - 1 : 0;
+    }
+}
+
+// receiver of tile cell (lr, lc), a mask cell
+template <int TW, int TH>
+__device__ __forceinline__ uint16_t fx_link(const FxTile<TW, TH> &T, int lr, int lc, bool is_outlet)
+{
+    const int p = fx_pad<TW>(lr, lc);
+    const int d = fx_dir(T.sfd[p]);
+    if (d < 0 || is_outlet || !T.smk[p + cdy(d) * FxTile<TW, TH>::PW + cdx(d)]) return FX_NONE;
+    const int nr = lr + cdy(d), nc = lc + cdx(d);
+    return nr >= 0 && nr < TH && nc >= 0 && nc < TW ? (uint16_t)(nr * TW + nc) : (uint16_t)FX_EXIT;
+}
+
+// Loads of both passes: directions and mask of the tile and its ring, each
+// cell's slot and val(i) (kept by the caller in registers), with every load in
+// flight before the first use.  Off-grid positions: no mask, no code.
+template <int TW, int TH, typename V, class F>
+__device__ __forceinline__ void fx_load(const FxArgs &a, int tx0, int ty0, FxTile<TW, TH> &T, V *v, int *slot, F &&val)
+{
+    typedef FxTile<TW, TH> FT;
+    const int W = a.W, H = a.H;
+    // offsets from the tile's first cell: 32 bits beside a uniform base (a
+    // 64-bit address per load in flight would take half the registers)
+    const long c0 = (long)ty0 * W + tx0;
+    const uint8_t *fd0 = a.fd + c0, *mask0 = a.mask + c0, *dem0 = a.demid + c0;
+    uint32_t vf[FT::NPPER], vm[FT::NPPER];   // 32-bit: byte registers would be packed, with a wait per load
+#pragma unroll
+    for (int q = 0; q < FT::NPPER; q++) {
+        const int k = threadIdx.x + q * 256;
+        const int ry = k / FT::PW - 1, rx = k % FT::PW - 1;
+        const bool in = k < FT::NP && ty0 + ry >= 0 && ty0 + ry < H && tx0 + rx >= 0 && tx0 + rx < W;
+        const int n = ry * W + rx;
+        vf[q] = in ? fd0[n] : 0;
+        vm[q] = in ? mask0[n] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < FT::PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int r = li / TW, col = li % TW;
+        const int n = ty0 + r < H && tx0 + col < W ? r * W + col : 0;
+        v[q] = val(c0, n);
+        slot[q] = a.demid ? (int)dem0[n] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < FT::NPPER; q++) {
+        const int k = threadIdx.x + q * 256;
+        if (k < FT::NP) {
+            T.sfd[k] = vf[q];
+            T.smk[k] = vm[q];
+        }
+    }
+}
+
+// Pass A.  After round t a cell holds the sum over the cells within 2^(t+1) - 1
+// links upstream in the tile, and its pointer, kept in a register as well, is
+// its 2^(t+1)-th ancestor or, marked FX_ROOT, the root of its path if that is
+// nearer: such a cell has nothing more to add.
+//
+// Both passes are bound by the latency of what a tile waits for (loads, seven
+// rounds here, a path of the tile's height or so there) and hide it with five
+// and seven tiles per compute unit.  One workgroup per tile: in a loop over
+// tiles the compiler keeps every cell's offsets in registers across the loop
+// (155 of them, three tiles per compute unit).  4096^2: 285 -> 176 us here
+// (a second pointer array for the roots and a wait per cell's weight before)
+// and 361 -> 120 us for pass C, which used to repeat the doubling and to look
+// up a border cell's donors one after another.  Walks from the leaves, each
+// link taken once, instead of the doubling: 409 us (one long river keeps the
+// tile's other waves waiting).
+template <int TW, int TH>
+__global__ void __launch_bounds__(256, 5) k_fx_sums(FxArgs a)
+{
+    typedef FxTile<TW, TH> FT;
+    __shared__ FT T;
     __shared__ int s_wave[4], s_base;
     const int W = a.W, H = a.H;
-    const int ntx = (W + TW - 1) / TW, nty = (H + TH - 1) / TH;
-    for (int tile = blockIdx.x; tile < ntx * nty; tile += gridDim.x) {
-        const int tx0 = (tile % ntx) * TW, ty0 = (tile / ntx) * TH;
-        __syncthreads();
-        // directions and mask of the tile and its ring, every load in flight
-        // before the first store (off-grid positions: no mask, no code)
-        {
-            uint32_t vf[NPPER], vm[NPPER];   // 32-bit: byte registers would be packed, with a wait per load
+    const int ntx = (W + TW - 1) / TW;
+    const int tx0 = (int)(blockIdx.x % ntx) * TW, ty0 = (int)(blockIdx.x / ntx) * TH;
+    fx_slots(a, T);
+    float w[FT::PER];
+    int slot[FT::PER];
+    fx_load<TW, TH>(a, tx0, ty0, T, w, slot, [&](long c0, int n) { return (a.w + c0)[n]; });
+    __syncthreads();
+    int nexit = 0;
+    uint32_t exits = 0, cells = 0;   // of this thread's cells
+    uint32_t jr[FT::PER];
 #pragma unroll
-            for (int q = 0; q < NPPER; q++) {
-                const int k = threadIdx.x + q * 256;
-                const int gy = ty0 - 1 + k / PW, gx = tx0 - 1 + k % PW;
-                const bool in = k < NP && gy >= 0 && gy < H && gx >= 0 && gx < W;
-                const long n = (long)gy * W + gx;
-                vf[q] = in ? a.fd[n] : 0;
-                vm[q] = in ? a.mask[n] : 0;
-            }
-#pragma unroll
-            for (int q = 0; q < NPPER; q++) {
-                const int k = threadIdx.x + q * 256;
-                if (k < NP) {
-                    sfd[k] = vf[q];
-                    smk[k] = vm[q];
-                }
-            }
-        }
-        __syncthreads();
-        int nexit = 0;
-        uint32_t exitbits = 0;
-        int slot[PER];
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int li = threadIdx.x + q * 256;
-            const int lr = li / TW, lc = li % TW;
-            const int r = ty0 + lr, col = tx0 + lc;
-            const int p = fx_pad<TW>(lr, lc);
-            slot[q] = 0;
-            unsigned long long v = 0;
-            uint16_t j = FX_NONE;
-            bool ex = false;
-            if (smk[p]) {
-                const long i = (long)r * W + col;
-                const int s = a.demid ? (int)a.demid[i] : 0;
-                slot[q] = s;
-                const int outlet = a.ds[s].outlet;
-                v = fx_quant(a.w[i], a.shift[s]);
-                if (fx_tagged(i, W, a.mask, outlet)) v += FX_TAG;
-                const int d = fx_dir(sfd[p]);
-                if (d >= 0 && i != outlet) {
-                    const int pn = p + cdy(d) * PW + cdx(d);
-                    if (smk[pn]) {
-                        const int nr = lr + cdy(d), nc = lc + cdx(d);
-                        if (nr >= 0 && nr < TH && nc >= 0 && nc < TW) j = (uint16_t)(nr * TW + nc);
-                        else ex = true;
-                    }
-                }
-                if (FINAL && (lr == 0 || lr == TH - 1 || lc == 0 || lc == TW - 1)) {
-                    // exits of other tiles that drain into this cell
-#pragma unroll
-                    for (int dd = 0; dd < 8; dd++) {
-                        const int tr = lr + cdy(dd), tc = lc + cdx(dd);
-                        if (tr >= 0 && tr < TH && tc >= 0 && tc < TW) continue;   // inside the tile
-                        const int pn = p + cdy(dd) * PW + cdx(dd);
-                        if (!smk[pn] || sfd[pn] != donor_code(dd)) continue;
-                        const long y = (long)(r + cdy(dd)) * W + (col + cdx(dd));
-                        if (y == outlet) continue;                                // cut link
-                        v += a.ex_val[a.exit_id[y]];
-                    }
-                }
-            }
-            x[li] = v;
-            J[li] = j;
-            if (!FINAL) {
-                R[li] = j == FX_NONE ? (uint16_t)li : j;
-                isexit[li] = ex ? 1 : 0;
-            }
-            if (ex) {
+    for (int q = 0; q < FT::PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int lr = li / TW, lc = li % TW;
+        uint32_t j = FX_NONE;
+        unsigned long long v = 0;
+        if (T.smk[fx_pad<TW>(lr, lc)]) {
+            const long i = (long)(ty0 + lr) * W + tx0 + lc;
+            const int outlet = T.outlet[slot[q]];
+            cells |= 1u << q;
+            v = fx_quant(w[q], T.shift[slot[q]]);
+            if (fx_tagged(i, W, a.mask, outlet)) v += FX_TAG;
+            j = fx_link(T, lr, lc, i == outlet);
+            if (j == FX_EXIT) {
                 nexit++;
-                exitbits |= 1u << q;
+                exits |= 1u << q;
             }
         }
+        if (j >= FX_EXIT) j = FX_ROOT | (uint32_t)li;
+        T.x[li] = v;
+        T.J[li] = (uint16_t)j;
+        jr[q] = j;
+    }
+    for (;;) {
         __syncthreads();
-        // pointer doubling: after round t every cell holds the sum over the
-        // cells within 2^(t+1) - 1 links upstream in the tile
-        for (;;) {
-            unsigned long long v[PER];
-            uint16_t jj[PER], rr[PER];
-            int act = 0;
+        unsigned long long v[FT::PER];
+        uint32_t jj[FT::PER];
+        int act = 0;
 #pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int li = threadIdx.x + q * 256;
-                const uint16_t j = J[li];
-                if (j != FX_NONE) {
-                    act |= 1 << q;
-                    v[q] = x[li];
-                    jj[q] = J[j];
-                    if (!FINAL) rr[q] = R[R[li]];
-                }
+        for (int q = 0; q < FT::PER; q++) {
+            jj[q] = FX_ROOT;
+            if (!(jr[q] & FX_ROOT)) {
+                act = 1;
+                v[q] = T.x[threadIdx.x + q * 256];
+                jj[q] = T.J[jr[q]];
             }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                if (!((act >> q) & 1)) continue;
-                const int li = threadIdx.x + q * 256;
-                atomicAdd(&x[J[li]], v[q]);
-                J[li] = jj[q];
-                if (!FINAL) R[li] = rr[q];
-            }
-            if (!__syncthreads_or(act)) break;
         }
-        // outputs
-        if (!FINAL) {
-            int k = fx_block_append(a.ex_count, nexit, s_wave, &s_base);
+        if (!__syncthreads_or(act)) break;
 #pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int li = threadIdx.x + q * 256;
-                const int lr = li / TW, lc = li % TW;
-                const int r = ty0 + lr, col = tx0 + lc;
-                if (r >= H || col >= W) continue;
-                const long i = (long)r * W + col;
-                if ((exitbits >> q) & 1) {
-                    if (k < a.ex_cap) {
-                        const int d = fx_dir(sfd[fx_pad<TW>(lr, lc)]);
-                        a.exit_id[i] = k;
-                        a.ex_val[k] = x[li];
-                        a.ex_recv[k] = (int)((long)(r + cdy(d)) * W + (col + cdx(d)));
-                    }
-                    k++;
-                }
-                if (lr == 0 || lr == TH - 1 || lc == 0 || lc == TW - 1) {
-                    const int root = R[li];
-                    a.xroot[i] = isexit[root] ? (int)((long)(ty0 + root / TW) * W + (tx0 + root % TW)) : -1;
-                }
+        for (int q = 0; q < FT::PER; q++) {
+            if (jr[q] & FX_ROOT) continue;
+            atomicAdd(&T.x[jr[q]], v[q]);
+            jr[q] = jj[q];
+            T.J[threadIdx.x + q * 256] = (uint16_t)jj[q];
+        }
+    }
+    int k = fx_block_append(a.ex_count, nexit, s_wave, &s_base);
+#pragma unroll
+    for (int q = 0; q < FT::PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int lr = li / TW, lc = li % TW;
+        const int r = ty0 + lr, col = tx0 + lc;
+        if (!((cells >> q) & 1)) continue;
+        const long i = (long)r * W + col;
+        const unsigned long long s = T.x[li];
+        reinterpret_cast<unsigned long long *>(a.fa)[i] = s;
+        if (lr == 0 || lr == TH - 1 || lc == 0 || lc == TW - 1) {
+            // the root is an exit if its receiver is a mask cell (in
+            // another tile) and its link is not cut
+            const int root = jr[q] & (FX_ROOT - 1), rr = root / TW, rc = root % TW;
+            const long ri = (long)(ty0 + rr) * W + tx0 + rc;
+            const bool ex = fx_link(T, rr, rc, ri == T.outlet[slot[q]]) == FX_EXIT;
+            a.xroot[i] = ex ? (int)ri : -1;
+        }
+        if (!((exits >> q) & 1)) continue;
+        if (k < a.ex_cap) {
+            const int d = fx_dir(T.sfd[fx_pad<TW>(lr, lc)]);
+            a.exit_id[i] = k;
+            a.ex_val[k] = s;
+            a.ex_recv[k] = (int)((long)(r + cdy(d)) * W + (col + cdx(d)));
+        }
+        k++;
+    }
+}
+
+// Pass C.  Each border cell with donors in other tiles adds their final values
+// to every cell of its in-tile path, itself included.
+template <int TW, int TH>
+__global__ void __launch_bounds__(256, 5) k_fx_final(FxArgs a)
+{
+    typedef FxTile<TW, TH> FT;
+    __shared__ FT T;
+    const int W = a.W, H = a.H;
+    const int ntx = (W + TW - 1) / TW;
+    const int tx0 = (int)(blockIdx.x % ntx) * TW, ty0 = (int)(blockIdx.x / ntx) * TH;
+    fx_slots(a, T);
+    unsigned long long x[FT::PER];
+    int slot[FT::PER];
+    fx_load<TW, TH>(a, tx0, ty0, T, x, slot,
+                    [&](long c0, int n) { return (reinterpret_cast<const unsigned long long *>(a.fa) + c0)[n]; });
+    __syncthreads();
+    // donors in other tiles of this thread's border cell: their exit
+    // numbers in one wait, their values in another
+    unsigned long long in = 0;
+    int at = -1;
+    if (threadIdx.x < FT::NB) {
+        int lr, lc;
+        fx_border<TW, TH>(threadIdx.x, lr, lc);
+        const int p = fx_pad<TW>(lr, lc);
+        if (T.smk[p]) {
+            const long i = (long)(ty0 + lr) * W + tx0 + lc;
+            const int out = T.outlet[a.demid ? (int)a.demid[i] : 0];
+            int id[8];
+#pragma unroll
+            for (int d = 0; d < 8; d++) {
+                const int tr = lr + cdy(d), tc = lc + cdx(d);
+                const bool outside = tr < 0 || tr >= TH || tc < 0 || tc >= TW;
+                const int pn = p + cdy(d) * FT::PW + cdx(d);
+                const long y = i + (long)cdy(d) * W + cdx(d);
+                // (an outlet's link is cut)
+                id[d] = outside && T.smk[pn] && T.sfd[pn] == donor_code(d) && y != out ? a.exit_id[y] : -1;
+            }
+            unsigned long long e[8];
+#pragma unroll
+            for (int d = 0; d < 8; d++) e[d] = id[d] >= 0 ? a.ex_val[id[d]] : 0;
+#pragma unroll
+            for (int d = 0; d < 8; d++) in += e[d];
+            at = lr * TW + lc;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < FT::PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int lr = li / TW, lc = li % TW;
+        const bool m = T.smk[fx_pad<TW>(lr, lc)];
+        const long i = (long)(ty0 + lr) * W + tx0 + lc;
+        T.x[li] = m ? x[q] : 0;
+        T.J[li] = m ? fx_link(T, lr, lc, i == T.outlet[slot[q]]) : (uint16_t)FX_NONE;
+    }
+    __syncthreads();
+    if (in) {
+        for (int h = 0; at < (int)FX_EXIT && h < FT::NC; h++) {
+            atomicAdd(&T.x[at], in);
+            at = T.J[at];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < FT::PER; q++) {
+        const int li = threadIdx.x + q * 256;
+        const int lr = li / TW, lc = li % TW;
+        const int r = ty0 + lr, col = tx0 + lc;
+        if (r >= H || col >= W) continue;
+        const long i = (long)r * W + col;
+        if (!T.smk[fx_pad<TW>(lr, lc)]) {
+            a.fa[i] = make_float2(0.f, 0.f);
+            continue;
+        }
+        const unsigned long long s = T.x[li];
+        if (i == T.outlet[slot[q]]) a.dsw[slot[q]].fx_outlet_sum = s;
+        if (s >= FX_TAG) {
+            const int k = atomicAdd(a.tag_count, 1);
+            if (k < a.tag_cap) {
+                a.tag_cell[k] = (int)i;
+                a.tag_sum[k] = s;
             }
         } else {
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int li = threadIdx.x + q * 256;
-                const int lr = li / TW, lc = li % TW;
-                const int r = ty0 + lr, col = tx0 + lc;
-                if (r >= H || col >= W) continue;
-                const long i = (long)r * W + col;
-                if (!smk[fx_pad<TW>(lr, lc)]) {
-                    a.fa[i] = make_float2(0.f, 0.f);
-                    continue;
-                }
-                const unsigned long long s = x[li];
-                const int s2 = slot[q];
-                if (i == a.ds[s2].outlet) a.dsw[s2].fx_outlet_sum = s;
-                if (s >= FX_TAG) {
-                    const int k = atomicAdd(a.tag_count, 1);
-                    if (k < a.tag_cap) {
-                        a.tag_cell[k] = (int)i;
-                        a.tag_sum[k] = s;
-                    }
-                } else {
-                    a.fa[i] = fx_value(s, a.shift[s2]);
-                }
-            }
+            a.fa[i] = fx_value(s, T.shift[slot[q]]);
         }
     }
 }
@@ -411,6 +517,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     a.w = (const float *)c->w;
     a.ds = c->dsc;
     a.shift = c->fx_shift;
+    a.nslot = c->nslot;
     a.exit_id = reinterpret_cast<int *>(c->scan_tmp);
     a.xroot = c->ws;
     unsigned long long *tv = reinterpret_cast<unsigned long long *>(c->z2);
@@ -426,14 +533,9 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     a.dsw = c->dsc;
     constexpr int TW = 64, TH = 32;
     const long ntiles = (long)((c->W + TW - 1) / TW) * ((c->H + TH - 1) / TH);
-    int bpc = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_fx_tile<TW, TH, false>, 256, 0) != hipSuccess || bpc < 1)
-        bpc = 2;
-    int G = bpc * c->ncu;
-    if (G > ntiles) G = (int)ntiles;
     // A: in-tile sums, exits, in-tile roots of border cells
     LEM_CHECK(c, hipMemsetAsync(a.ex_count, 0, sizeof(int), c->s));
-    k_fx_tile<TW, TH, false><<<G, 256, 0, c->s>>>(a);
+    k_fx_sums<TW, TH><<<ntiles, 256, 0, c->s>>>(a);
     LEM_LAUNCHED(c);
     LEM_CHECK(c, hipMemcpyAsync(&c->hint[31], a.ex_count, sizeof(int), hipMemcpyDeviceToHost, c->s));
     LEM_CHECK(c, hipStreamSynchronize(c->s));
@@ -468,7 +570,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     }
     // C: final sums, fa, tagged cells
     LEM_CHECK(c, hipMemsetAsync(a.tag_count, 0, sizeof(int), c->s));
-    k_fx_tile<TW, TH, true><<<G, 256, 0, c->s>>>(a);
+    k_fx_final<TW, TH><<<ntiles, 256, 0, c->s>>>(a);
     LEM_LAUNCHED(c);
     LEM_CHECK(c, hipMemsetAsync(&c->scal->fa_uncomputed, 0, sizeof(int), c->s));
     k_fx_tags<<<64, 256, 0, c->s>>>(a.tag_count, a.tag_cap, a.tag_cell, a.tag_sum, c->demid, c->dsc, c->fx_shift,
