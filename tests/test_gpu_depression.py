@@ -60,3 +60,28 @@ def test_against_oracle(case, flow):
         for f in ("fa", "dem", "soilT"):
             assert np.array_equal(ctx.download(f), orc[f], equal_nan=True), f"step {k}: {f}"
     ctx.close()
+
+
+@pytest.mark.parametrize("h, w", [(15, 63), (16, 64), (17, 65), (33, 129), (64, 130)])
+def test_basin_pairs_at_block_edges(h, w):
+    """Many small basins with equal heights between them and holes in the mask,
+    on grids one cell around whole 64 x 16 blocks."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(h * 1000 + w)
+    z = 100.0 + rng.integers(0, 6, (h, w)).astype(np.float64)
+    z[rng.random((h, w)) < 0.03] = synth.NODATA
+    rain = np.full(z.shape, 800.0)
+    ctx = lemhip.LemContext(lemhip.default_params(w, h, 0), lemhip.FP64, 0)
+    ctx.init_state(z, rain, soilT_mode="nonneg")
+    orc = O.Oracle(z, rain, O.default_params(w, h, 0), soilT_mode="nonneg")
+    ctx.step(-1000)
+    orc.step(-1000)
+    s, o = ctx.summary(), orc.scalars()
+    for f in ("sinkcount", "nedges", "plateau_rounds1", "plateau_rounds2"):
+        if f in s and f in o:
+            assert s[f] == o[f], f
+    for f in ("fd", "SFD"):
+        assert np.array_equal(ctx.download(f), np.where(orc["mask"] != 0, orc[f], -9999)), f
+    for f in ("fa", "dem"):
+        assert np.array_equal(ctx.download(f), orc[f], equal_nan=True), f
+    ctx.close()
