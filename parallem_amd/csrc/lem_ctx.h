@@ -180,7 +180,7 @@ struct lemhip_ctx {
     int *hint = nullptr;          // pinned host ints for small readbacks (from 64: the plateau control block)
 
     // counters known on the host after each phase
-    int h_rounds1 = 0, h_rounds2 = 0, h_nlab = 0, h_nedges = 0, h_sinkcount = 0, h_sinks1 = 0;
+    int h_rounds1 = 0, h_rounds2 = 0, h_nlab = 0, h_nedges = 0;
     int h_fa_unc = 0, h_sed_unc = 0;
     int h_sed_open = 0;   // sediment cells the contraction took over (last pass)
 
@@ -241,7 +241,7 @@ int lem_runoff_phase(lemhip_ctx *c);
 int lem_calcwater(lemhip_ctx *c);
 int lem_fa32_sfd(lemhip_ctx *c, int *fallback);
 int lem_sed32(lemhip_ctx *c, int *fallback);
-int lem_sed_first(lemhip_ctx *c, int rounds);
+int lem_sed_first(lemhip_ctx *c, int rounds, const int *skip);
 int lem_fa_phase(lemhip_ctx *c, int iter);
 int lem_mod_phase(lemhip_ctx *c, int iter);
 int lem_sync_scalars(lemhip_ctx *c);

@@ -964,7 +964,8 @@ struct ResCtl {    // LEM_RES_CTL bytes
     int n;         // listed tiles
     int left;      // cells still pending in them after the launch
     int prog;      // some cell was resolved
-    int pad[13];
+    int pending;   // uncomputed cells of the grid
+    int pad[12];
     int beat[RES_BEATS * 16];   // one line each
 };
 static_assert(sizeof(ResCtl) <= LEM_RES_CTL && RES_EDGE == LEM_RES_EDGE && RES_T == LEM_RES_T, "resident buffers");
@@ -1416,10 +1417,12 @@ static int grid1d_dag(long n)
     return (int)g;
 }
 
-__global__ void k_iota(int n, int *a)
+// every tile on the list; none if *skip
+__global__ void k_iota(int n, int *a, int *count, const int *skip)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = i;
+    if (i == 0) *count = skip && *skip ? 0 : n;
 }
 
 // Finishes the pass with resident tiles if the unfinished ones fit the chip
@@ -1459,25 +1462,25 @@ static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, i
             k_dag_resident<Cell, SFD><<<n, 256, 0, c->s>>>(c->W, c->H, *round, cell, c->dmask, c->fd, st,
                                                            c->res_list, c->res_pos, c->res_ex, ctl);
         prof_end(c, prof_slot, 1);
-        LEM_CHECK(c, hipMemsetAsync(&c->scal->flag, 0, sizeof(int), c->s));
-        k_count_pending<<<grid1d_dag(c->N), 256, 0, c->s>>>(c->N, c->mask, st, &c->scal->flag);
+        k_count_pending<<<grid1d_dag(c->N), 256, 0, c->s>>>(c->N, c->mask, st, &ctl->pending);
         LEM_LAUNCHED(c);
-        LEM_CHECK(c, hipMemcpyAsync(&c->hint[40], ctl, 3 * sizeof(int), hipMemcpyDeviceToHost, c->s));
-        LEM_CHECK(c, hipMemcpyAsync(&c->hint[3], &c->scal->flag, sizeof(int), hipMemcpyDeviceToHost, c->s));
+        LEM_CHECK(c, hipMemcpyAsync(&c->hint[40], ctl, 4 * sizeof(int), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipStreamSynchronize(c->s));
         // every launch that resolved a cell is followed by another unless
         // nothing is left: at most one launch per cell
         if (c->hint[41] == 0 || c->hint[42] == 0) break;
     }
-    *uncomputed = c->hint[3];
+    *uncomputed = c->hint[43];
     *done = 1;
     return LEMHIP_OK;
 }
 
 // first_rounds > 0: only that many rounds (the first visits every tile),
-// with no wait for the device; *uncomputed is not set
+// with no wait for the device, and none of them if *skip turns out non-zero;
+// *uncomputed is not set
 template <int TW, int TH, class Cell, bool SFD>
-static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, int first_rounds = 0)
+static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, int first_rounds = 0,
+                      const int *skip = nullptr)
 {
     int ntiles = ((c->W + TW - 1) / TW) * ((c->H + TH - 1) / TH);
     int *st = reinterpret_cast<int *>(c->scan_tmp);
@@ -1499,11 +1502,9 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
     // wake stamps start below every round number of the pass
     LEM_CHECK(c, hipMemsetAsync(c->dag_wake, 0, sizeof(int) * ntiles, c->s));
     // the first round visits every tile
-    k_iota<<<(ntiles + 255) / 256, 256, 0, c->s>>>(ntiles, L[(r + 1) % 3]);
-    LEM_LAUNCHED(c);
     LEM_CHECK(c, hipMemsetAsync(ctl, 0, sizeof(DagCtl), c->s));
-    c->hint[16] = ntiles;
-    LEM_CHECK(c, hipMemcpyAsync(&ctl->cnt[(r + 1) % 3], &c->hint[16], sizeof(int), hipMemcpyHostToDevice, c->s));
+    k_iota<<<(ntiles + 255) / 256, 256, 0, c->s>>>(ntiles, L[(r + 1) % 3], &ctl->cnt[(r + 1) % 3], skip);
+    LEM_LAUNCHED(c);
     const int BATCH = c->dag_batch;
     int batch = BATCH;
     // as many workgroups as the CUs hold at once (the first rounds visit every tile)
@@ -1642,13 +1643,13 @@ int lem_sed_dag(lemhip_ctx *c)
 // crosses into them only from cells completed before (after round 2 about
 // 91%).  The rest stays pending for the contraction (lem_sed32.hip).  The tile shape is fixed, so
 // which cells complete here depends on the cell's position modulo 32 only.
-int lem_sed_first(lemhip_ctx *c, int rounds)
+int lem_sed_first(lemhip_ctx *c, int rounds, const int *skip)
 {
     SedCell<float, 32, 32> cell{reinterpret_cast<const float *>(c->ero), reinterpret_cast<const float *>(c->inci),
                                 reinterpret_cast<const float *>(c->geli), reinterpret_cast<const float *>(c->z2),
                                 reinterpret_cast<float *>(c->depo), reinterpret_cast<float *>(c->stone),
                                 reinterpret_cast<float *>(c->fines), c->soilT};
-    return run_rounds<32, 32, decltype(cell), true>(c, cell, nullptr, PROF_SED_K, rounds);
+    return run_rounds<32, 32, decltype(cell), true>(c, cell, nullptr, PROF_SED_K, rounds, skip);
 }
 
 // Times flow accumulation with every tile shape, then the best shape with

@@ -89,7 +89,7 @@ struct LemScalars {
     double FA_max;
     double totE, totI, totG, totD, totwC, totwP, totbio;
     int outlet;
-    int sinks_pass1;      // mask cells with SFD == 0 after pass-1 routing
+    int sinks_pass1;      // non-zero: some DEM has mask cells with SFD == 0 after pass-1 routing
     int sinkcount;        // distinct labels in the edge set (newflow.cu:1045) or sinks_pass1
     int nlabels;
     int nedges;
@@ -99,5 +99,6 @@ struct LemScalars {
     int kept[2];          // edges left after a spill-height phase, by phase parity
     int flag;             // generic change flag for host-driven loops
     int w_bad;            // a mask cell's runoff weight is negative or not finite
+    int sed_bad;          // a cell's stone-mixing parameters are not finite (FP32 sediment)
     unsigned long long lowest_enc;
 };

@@ -400,9 +400,23 @@ __global__ void __launch_bounds__(256, 5) k_fx_final(FxArgs a)
     }
 }
 
-// parent of each exit in the exit forest
-__global__ void k_fx_parent(int n, const int *ex_recv, const int *xroot, const int *exit_id, int *P)
+// exits listed, 0 if they are more than the list holds (the host then leaves the
+// pass before its values are used)
+__device__ __forceinline__ int fx_count(const int *count, int cap)
 {
+    const int n = *count;
+    return n <= cap ? n : 0;
+}
+
+// parent of each exit in the exit forest; clears the counters of pass C
+__global__ void k_fx_parent(const int *count, int cap, const int *ex_recv, const int *xroot, const int *exit_id, int *P,
+                            int *tag_count, int *uncomputed)
+{
+    const int n = fx_count(count, cap);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *tag_count = 0;
+        *uncomputed = 0;
+    }
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const int xr = xroot[ex_recv[k]];
         P[k] = xr >= 0 ? exit_id[xr] : -1;
@@ -410,8 +424,10 @@ __global__ void k_fx_parent(int n, const int *ex_recv, const int *xroot, const i
 }
 
 // one doubling round over the exit forest in two launches: snapshot, then add
-__global__ void k_fx_gather(int n, const unsigned long long *val, const int *P, unsigned long long *tv, int *tp)
+__global__ void k_fx_gather(const int *count, int cap, const unsigned long long *val, const int *P,
+                            unsigned long long *tv, int *tp)
 {
+    const int n = fx_count(count, cap);
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const int p = P[k];
         tv[k] = val[k];
@@ -424,10 +440,10 @@ __global__ void k_fx_gather(int n, const unsigned long long *val, const int *P, 
 // wave (a sum over the run's own lanes only, so every value counts once)
 // and added by the run's first lane with one atomic.  Integer sums: the
 // totals do not depend on the grouping.
-__global__ void __launch_bounds__(256) k_fx_scatter(int n, unsigned long long *val, int *P,
+__global__ void __launch_bounds__(256) k_fx_scatter(const int *count, int cap, unsigned long long *val, int *P,
                                                     const unsigned long long *tv, const int *tp, int *flag)
 {
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, n = fx_count(count, cap);
     bool more = false;
     // whole waves go round the loop together (the shuffles need every lane)
     for (int k0 = blockIdx.x * blockDim.x; k0 < n; k0 += gridDim.x * blockDim.x) {
@@ -537,50 +553,45 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     LEM_CHECK(c, hipMemsetAsync(a.ex_count, 0, sizeof(int), c->s));
     k_fx_sums<TW, TH><<<ntiles, 256, 0, c->s>>>(a);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[31], a.ex_count, sizeof(int), hipMemcpyDeviceToHost, c->s));
-    LEM_CHECK(c, hipStreamSynchronize(c->s));
-    const int nex = c->hint[31];
-    // the exit values and their snapshot share the 8-byte scratch of N cells;
-    // exits are tile border cells (9% of a full tile), so only grids of a few
-    // cells could have more
-    if ((long)nex > N / 2) { *fallback = 1; return LEMHIP_OK; }
-    // B: the exit forest
-    if (nex > 0) {
-        int *P = reinterpret_cast<int *>(c->sp0), *tp = reinterpret_cast<int *>(c->sp1);
-        k_fx_parent<<<fx_grid(nex), 256, 0, c->s>>>(nex, a.ex_recv, a.xroot, a.exit_id, P);
-        LEM_LAUNCHED(c);
-        // rounds before the first host read: enough to double along a path
-        // that crosses every tile row and column twice (a read leaves the
-        // device idle for about 15 us, a round over a short list takes less);
-        // only a batch's last round reports changes
-        int batch = 2;
-        while ((1 << batch) < 4 * ((c->W + TW - 1) / TW + (c->H + TH - 1) / TH)) batch++;
-        for (int round = 0;; round += batch, batch = 2) {
-            for (int q = 0; q < batch; q++) {
-                if (q == batch - 1) LEM_CHECK(c, hipMemsetAsync(&c->scal->nlabels, 0, sizeof(int), c->s));
-                k_fx_gather<<<fx_grid(nex), 256, 0, c->s>>>(nex, a.ex_val, P, tv, tp);
-                k_fx_scatter<<<fx_grid(nex), 256, 0, c->s>>>(nex, a.ex_val, P, tv, tp, &c->scal->nlabels);
-            }
-            LEM_LAUNCHED(c);
-            LEM_CHECK(c, hipMemcpyAsync(&c->hint[32], &c->scal->nlabels, sizeof(int), hipMemcpyDeviceToHost, c->s));
-            LEM_CHECK(c, hipStreamSynchronize(c->s));
-            if (!c->hint[32]) break;
-            if (round > 64) { c->err = "exit forest did not converge"; return LEMHIP_E_NOT_CONVERGED; }
+    // B: the exit forest.  The kernels take the number of exits from the device
+    // and their grid from what it can be.
+    const int ge = fx_grid(std::min(N, ntiles * FxTile<TW, TH>::NB));
+    int *P = reinterpret_cast<int *>(c->sp0), *tp = reinterpret_cast<int *>(c->sp1);
+    k_fx_parent<<<ge, 256, 0, c->s>>>(a.ex_count, a.ex_cap, a.ex_recv, a.xroot, a.exit_id, P, a.tag_count,
+                                      &c->scal->fa_uncomputed);
+    LEM_LAUNCHED(c);
+    // rounds before the first host read: enough to double along a path that
+    // crosses every tile row and column twice (a read leaves the device idle
+    // for about 15 us, a round over a short list takes less); only a batch's
+    // last round reports changes
+    int batch = 2;
+    while ((1 << batch) < 4 * ((c->W + TW - 1) / TW + (c->H + TH - 1) / TH)) batch++;
+    for (int round = 0;; round += batch, batch = 2) {
+        for (int q = 0; q < batch; q++) {
+            if (q == batch - 1) LEM_CHECK(c, hipMemsetAsync(&c->scal->nlabels, 0, sizeof(int), c->s));
+            k_fx_gather<<<ge, 256, 0, c->s>>>(a.ex_count, a.ex_cap, a.ex_val, P, tv, tp);
+            k_fx_scatter<<<ge, 256, 0, c->s>>>(a.ex_count, a.ex_cap, a.ex_val, P, tv, tp, &c->scal->nlabels);
         }
+        LEM_LAUNCHED(c);
+        LEM_CHECK(c, hipMemcpyAsync(c->hscal, c->scal, sizeof(LemScalars), hipMemcpyDeviceToHost, c->s));
+        LEM_CHECK(c, hipStreamSynchronize(c->s));
+        // the exit values and their snapshot share the 8-byte scratch of N
+        // cells; exits are tile border cells (9% of a full tile), so only grids
+        // of a few cells could have more
+        if (c->hscal->nedges > a.ex_cap) { *fallback = 1; return LEMHIP_OK; }
+        if (!c->hscal->nlabels) break;
+        if (round > 64) { c->err = "exit forest did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
     // C: final sums, fa, tagged cells
-    LEM_CHECK(c, hipMemsetAsync(a.tag_count, 0, sizeof(int), c->s));
     k_fx_final<TW, TH><<<ntiles, 256, 0, c->s>>>(a);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemsetAsync(&c->scal->fa_uncomputed, 0, sizeof(int), c->s));
     k_fx_tags<<<64, 256, 0, c->s>>>(a.tag_count, a.tag_cap, a.tag_cell, a.tag_sum, c->demid, c->dsc, c->fx_shift,
                                     a.w, a.fa, &c->scal->fa_uncomputed);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[33], a.tag_count, sizeof(int), hipMemcpyDeviceToHost, c->s));
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[34], &c->scal->fa_uncomputed, sizeof(int), hipMemcpyDeviceToHost, c->s));
+    LEM_CHECK(c, hipMemcpyAsync(c->hscal, c->scal, sizeof(LemScalars), hipMemcpyDeviceToHost, c->s));
     LEM_CHECK(c, hipStreamSynchronize(c->s));
-    if (c->hint[33] > a.tag_cap) { *fallback = 1; return LEMHIP_OK; }
-    c->h_fa_unc = c->hint[34];
+    if (c->hscal->flag > a.tag_cap) { *fallback = 1; return LEMHIP_OK; }
+    c->h_fa_unc = c->hscal->fa_uncomputed;
     c->dag_rounds_last = 0;
     return LEMHIP_OK;
 }

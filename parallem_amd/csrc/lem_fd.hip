@@ -710,23 +710,34 @@ __global__ void __launch_bounds__(PLAT_NT(K), K == 16 ? 4 : 6) k_plat_block(int 
     if (threadIdx.x == 0 && wg_last > 0) atomicMax(&ctl->last_change, wg_last);
 }
 
-__global__ void k_slots_sinks_init(int ns, DemScal *ds)
+// the sinks per DEM, and the counts and flag of the label phase
+__global__ void k_slots_sinks_init(int ns, DemScal *ds, LemScalars *sc)
 {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < ns) ds[j].sinks_pass1 = 0;
+    if (j == 0) {
+        sc->sinks_pass1 = 0;
+        sc->ncand = 0;
+        sc->flag = 0;
+    }
 }
 
 __global__ void __launch_bounds__(256) k_count_sinks(const int *cand, int n, const uint8_t *SFD,
-                                                     const uint8_t *demid, int ns, DemScal *ds)
+                                                     const uint8_t *demid, int ns, DemScal *ds, int *total)
 {
     __shared__ int hist[LEM_MAX_SLOTS + 1];
+    int mine = 0;
     for (int j = threadIdx.x; j < ns; j += blockDim.x) hist[j] = 0;
     __syncthreads();
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         long i = cand[k];
-        if (SFD[i] == 0) atomicAdd(&hist[slot_of(demid, i)], 1);
+        if (SFD[i] == 0) {
+            atomicAdd(&hist[slot_of(demid, i)], 1);
+            mine = 1;
+        }
     }
     slot_hist_flush(hist, ds, (int)offsetof(DemScal, sinks_pass1), ns);
+    if (mine) *total = 1;   // some DEM has sinks
 }
 
 // ------------------------------------------------ watershed labels
@@ -766,7 +777,7 @@ __global__ void k_sink_flags(int W, int H, const uint8_t *mask, const uint8_t *S
 
 // init_watershedMFD with labels = 1 + rank of the sink cell in atlas row-major order
 __global__ void k_init_ws(int W, int H, const uint8_t *mask, const uint8_t *SFD, const int *prefix,
-                          const uint8_t *demid, const DemDesc *dd, int *ws, uint8_t *labdem)
+                          const uint8_t *demid, const DemDesc *dd, int *ws, uint8_t *labdem, int *nlab)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= W) return;
@@ -785,6 +796,7 @@ __global__ void k_init_ws(int W, int H, const uint8_t *mask, const uint8_t *SFD,
             v = -((r + kDY[d]) * W + (c + kDX[d]) + 1);
         }
         ws[i] = v;
+        if (r == H - 1 && c == W - 1) *nlab = prefix[i] + (v > 0 ? 1 : 0);
     }
 }
 
@@ -792,27 +804,28 @@ __global__ void k_init_ws(int W, int H, const uint8_t *mask, const uint8_t *SFD,
 // label of an equal-height neighbour; iterated to the fixed point (the
 // component maximum, independent of the update order).  SFD==0 cells are a
 // subset of the pass-1 plateau candidates.
-__global__ void k_sink_merge(int W, int H, const int *cand, int n, const uint8_t *SFD, const double *z,
+__global__ void k_sink_merge(int W, int H, const int *cand, const int *count, const uint8_t *SFD, const double *z,
                              int *ws, int *flag)
 {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    long self = cand[k];
-    if (SFD[self] != 0) return;
-    int irow = (int)(self / W), icol = (int)(self % W);
-    double zc = z[self];
-    int cur = ws[self], best = cur;
-    for (int d = 0; d < 8; d++) {
-        int cx = icol + kDX[d], cy = irow + kDY[d];
-        if (cx >= 0 && cx < W && cy >= 0 && cy < H) {
-            long nb = (long)cy * W + cx;
-            if (z[nb] == zc) {
-                int v = ws[nb];
-                if (v > best) best = v;
+    const int n = *count;
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        long self = cand[k];
+        if (SFD[self] != 0) continue;
+        int irow = (int)(self / W), icol = (int)(self % W);
+        double zc = z[self];
+        int cur = ws[self], best = cur;
+        for (int d = 0; d < 8; d++) {
+            int cx = icol + kDX[d], cy = irow + kDY[d];
+            if (cx >= 0 && cx < W && cy >= 0 && cy < H) {
+                long nb = (long)cy * W + cx;
+                if (z[nb] == zc) {
+                    int v = ws[nb];
+                    if (v > best) best = v;
+                }
             }
         }
+        if (best > cur) { ws[self] = best; *flag = 1; }
     }
-    if (best > cur) { ws[self] = best; *flag = 1; }
 }
 
 // Only sinks with an equal-height neighbour can change in the merge above;
@@ -1603,7 +1616,8 @@ static int cutoff_components(lemhip_ctx *c, int nlab, int ne)
 // Spill heights of the labels into c->rmm (initialised: label 0 -inf, the
 // rest +inf) by Borůvka phases over the label-sorted edge list, whose length
 // is in scal->nedges (at most `bound`, read with the first counts).  Two phases
-// run between host reads: the kernels take the edge counts from the device and
+// run between host reads, three where an empty one costs no more than a read
+// (20 us on short label lists, 75 on the 8191x7003 DEM's): the kernels take the edge counts from the device and
 // their grids from the last count the host knows.  A read leaves the device
 // idle for about 15 us, as long as the phase itself on short lists (a step at
 // 512^2 with seven reads fewer, these among them: 1.80 instead of 1.88 ms).
@@ -1625,9 +1639,10 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
     const unsigned long long *w = c->ew;
     const int *cnt = &c->scal->nedges;
     LEM_TRY(clear_flag(c));   // raised only by a pointer walk that does not end
+    const int per = n <= (1 << 18) ? 3 : 2;
     // the profile slot times the kernels only, not the host reads between them
     for (int ph = 0, na = bound; na > 0;) {
-        for (int q = 0; q < 2; q++, ph++) {
+        for (int q = 0; q < per; q++, ph++) {
             const int p = ph & 1;
             const int ge = grid1d(na, 256, 1 << 30);
             uint32_t *lo2 = c->elo2[p], *hi2 = c->ehi2[p];
@@ -1658,7 +1673,7 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
         const int nk = c->hscal->kept[(ph - 1) & 1];
         // every component with an outgoing edge joins another each phase, so
         // the components with edges at least halve
-        if (nk >= na && ph > 2) { c->err = "spill-height phases made no progress"; return LEMHIP_E_NOT_CONVERGED; }
+        if (nk >= na && ph > per) { c->err = "spill-height phases made no progress"; return LEMHIP_E_NOT_CONVERGED; }
         na = nk;
         if (ph > 64) { c->err = "spill-height phases did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
@@ -1674,8 +1689,8 @@ static int raise_surface(lemhip_ctx *c)
 
 
 // floodingDriver (routeflow.cu:202-676) up to the raised surface in c->z2.
-// *sinks: the sinks pass 1 left, counted per DEM on the device and read with
-// the label count; with none of them nothing is flooded.
+// *sinks: whether pass 1 left any, read with the label count; if not, nothing is
+// flooded.
 static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
 {
     long N = c->N;
@@ -1694,35 +1709,29 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
     // prefix lands in ws, then k_init_ws rewrites ws in place from it: use z2 as the prefix buffer instead
     int *prefix = reinterpret_cast<int *>(c->z2);
     LEM_CHECK(c, hipcub::DeviceScan::ExclusiveSum(c->cub_tmp, need, c->scan_tmp, prefix, (int)N, c->s));
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[0], c->scan_tmp + (N - 1), sizeof(int), hipMemcpyDeviceToHost, c->s));
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[1], prefix + (N - 1), sizeof(int), hipMemcpyDeviceToHost, c->s));
-    k_init_ws<<<grid2d(W, H), 256, 0, c->s>>>(W, H, c->mask, c->SFD, prefix, c->demid, c->ddesc, c->ws, c->labdem);
+    k_init_ws<<<grid2d(W, H), 256, 0, c->s>>>(W, H, c->mask, c->SFD, prefix, c->demid, c->ddesc, c->ws, c->labdem,
+                                              &c->scal->nlabels);
     // sink merge over the sinks that have an equal-height neighbour (list in the
-    // prefix buffer, free after k_init_ws)
+    // prefix buffer, free after k_init_ws); the first rounds run before the
+    // host knows of any
     int *mlist = reinterpret_cast<int *>(c->z2);
-    LEM_CHECK(c, hipMemsetAsync(&c->scal->ncand, 0, sizeof(int), c->s));
     k_merge_list<<<grid1d(ncand1, 256, 4096), 256, 0, c->s>>>(c->cand, ncand1, c->SFD, c->dmask, mlist,
                                                              &c->scal->ncand);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemcpyAsync(c->hdsc, c->dsc, sizeof(DemScal) * c->nslot, hipMemcpyDeviceToHost, c->s));
-    LEM_TRY(read_scalars(c));
-    *sinks = 0;
-    for (int j = 0; j < c->nslot; j++) *sinks += c->hdesc[j].w > 0 ? c->hdsc[j].sinks_pass1 : 0;
-    if (*sinks == 0) return LEMHIP_OK;
-    const int nlab = c->hint[0] + c->hint[1];
-    c->h_nlab = nlab;
-    const int nm = c->hscal->ncand;
-    for (int it = 0; nm > 0; it += 4) {
-        LEM_TRY(clear_flag(c));
+    for (long it = 0;; it += 4) {
+        const int gm = it ? grid1d(c->hscal->ncand, 256, 1 << 30) : grid1d(ncand1, 256, 256);
+        if (it) LEM_TRY(clear_flag(c));
         for (int q = 0; q < 4; q++)
-            k_sink_merge<<<grid1d(nm, 256, 1 << 30), 256, 0, c->s>>>(W, H, mlist, nm, c->SFD, c->dem, c->ws,
-                                                                     &c->scal->flag);
+            k_sink_merge<<<gm, 256, 0, c->s>>>(W, H, mlist, &c->scal->ncand, c->SFD, c->dem, c->ws, &c->scal->flag);
         LEM_LAUNCHED(c);
-        int f = 0;
-        LEM_TRY(read_flag(c, &f));
-        if (!f) break;
-        if (it / 4 > nm + 2) { c->err = "sink merge did not converge"; return LEMHIP_E_NOT_CONVERGED; }
+        LEM_TRY(read_scalars(c));
+        *sinks = c->hscal->sinks_pass1;
+        if (*sinks == 0) return LEMHIP_OK;
+        if (!c->hscal->flag) break;
+        if (it / 4 > (long)c->hscal->ncand + 2) { c->err = "sink merge did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
+    const int nlab = c->hscal->nlabels;
+    c->h_nlab = nlab;
     // watershed labels: one jump over every cell, then each walks the rest
     // (none to four jumps first: within 2 % on every size)
     LEM_TRY(clear_flag(c));
@@ -1846,9 +1855,10 @@ static int fd_phase_t(lemhip_ctx *c, int iter)
     // pass 1 on the unraised surface; slopes keep these values
     int n1 = 0, r1 = 0;
     LEM_TRY(directions_and_plateaus<TS>(c, c->dem, reinterpret_cast<TS *>(c->slopes), &n1, &r1));
-    k_slots_sinks_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc);
+    k_slots_sinks_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc, c->scal);
     if (n1 > 0) {
-        k_count_sinks<<<grid1d(n1, 256, 2048), 256, 0, c->s>>>(c->cand, n1, c->SFD, c->demid, c->nslot, c->dsc);
+        k_count_sinks<<<grid1d(n1, 256, 2048), 256, 0, c->s>>>(c->cand, n1, c->SFD, c->demid, c->nslot, c->dsc,
+                                                                &c->scal->sinks_pass1);
         LEM_LAUNCHED(c);
     }
     c->h_rounds1 = r1;
@@ -1861,8 +1871,6 @@ static int fd_phase_t(lemhip_ctx *c, int iter)
     if (sinks > 0)
         k_slots_sinkcount_fin<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->ddesc, c->nslot, c->dsc);
     prof_end(c, PROF_FLOOD);
-    c->h_sinks1 = sinks;
-    c->h_sinkcount = sinks;
     if (sinks == 0) {
         c->h_nlab = 0;
         k_slots_sinkcount_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc);

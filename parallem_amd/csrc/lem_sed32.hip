@@ -176,9 +176,10 @@ __global__ void __launch_bounds__(256) k_cs_from_engine(long N, const uint8_t *_
                                                         const double *__restrict__ soilT,
                                                         const float *__restrict__ dps,
                                                         const float *__restrict__ stone, float *ca, float *cb,
-                                                        int *list, int *list0, CsCtl *ctl)
+                                                        int *list, int *list0, CsCtl *ctl, const int *bad)
 {
     __shared__ CsChunk<CS_ITEMS> C;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->bad = *bad;
     const long CH = 256L * CS_ITEMS;
     int unc = 0;
     for (long c0 = (long)blockIdx.x * CH; c0 < N; c0 += (long)gridDim.x * CH) {
@@ -429,17 +430,11 @@ int lem_sed32(lemhip_ctx *c, int *fallback)
     CsCtl *ctl = reinterpret_cast<CsCtl *>(c->dag_ctl);
     static_assert(sizeof(CsCtl) <= 512, "control block");
 
-    LEM_CHECK(c, hipMemsetAsync(ctl, 0, sizeof(CsCtl), c->s));
-    LEM_TRY(lem_sed_prep<float>(c, &ctl->bad));
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[25], &ctl->bad, sizeof(int), hipMemcpyDeviceToHost, c->s));
-    LEM_CHECK(c, hipStreamSynchronize(c->s));
-    // non-finite parameters: the engine's path handles them (nothing of the
-    // state has changed yet)
-    if (c->hint[25]) return LEMHIP_OK;
-    *fallback = 0;
+    LEM_CHECK(c, hipMemsetAsync(&c->scal->sed_bad, 0, sizeof(int), c->s));
+    LEM_TRY(lem_sed_prep<float>(c, &c->scal->sed_bad));
     // the engine's first rounds, the first over every tile (their control block
-    // shares the memory of this one)
-    LEM_TRY(lem_sed_first(c, c->cs_rounds));
+    // shares the memory of this one); none if a parameter is not finite
+    LEM_TRY(lem_sed_first(c, c->cs_rounds, &c->scal->sed_bad));
     const long CH = 256L * CS_ITEMS;
     auto chunks = [&](long n) { return (int)std::max(1L, std::min((n + CH - 1) / CH, 4096L)); };
     auto chunks_r = [&](long n, int items) {
@@ -451,11 +446,16 @@ int lem_sed32(lemhip_ctx *c, int *fallback)
     // holds the lower half as floats)
     int *list0 = reinterpret_cast<int *>(c->z2) + NP;
     k_cs_from_engine<<<chunks(N), 256, 0, c->s>>>(N, c->mask, c->scan_tmp, c->soilT, dps, (const float *)c->stone,
-                                                  ca, cb, lists[0], list0, ctl);
+                                                  ca, cb, lists[0], list0, ctl, &c->scal->sed_bad);
     LEM_LAUNCHED(c);
-    LEM_CHECK(c, hipMemcpyAsync(&c->hint[24], &ctl->cnt[2], sizeof(int), hipMemcpyDeviceToHost, c->s));
+    const CsCtl *h = reinterpret_cast<const CsCtl *>(c->hint + 64);
+    LEM_CHECK(c, hipMemcpyAsync(c->hint + 64, ctl, offsetof(CsCtl, unc), hipMemcpyDeviceToHost, c->s));
     LEM_CHECK(c, hipStreamSynchronize(c->s));
-    long open = c->hint[24];
+    // non-finite parameters: the engine's path handles them (nothing of the
+    // state has changed yet)
+    if (h->bad) return LEMHIP_OK;
+    *fallback = 0;
+    long open = h->cnt[2];
     const long open0 = open;
     c->h_sed_open = (int)open;
     uint32_t r = 1;
