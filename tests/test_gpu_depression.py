@@ -1,6 +1,7 @@
 """Depression routing: basins that NaN heights cut off from the border (found
-only after the surface was raised once), and watershed pointers as long as a
-serpentine valley.  Bit-identical with the oracle."""
+only after the surface was raised once), watershed pointers as long as a
+serpentine valley, and a row of basins that join in one long path.
+Bit-identical with the oracle."""
 import numpy as np
 import pytest
 
@@ -39,11 +40,23 @@ def _serpentine(h, w):
     return z
 
 
+def _stairs(h, w):
+    """A channel of pits whose sills rise one after the other: every basin's lowest
+    sill is the last one's, so all of them join along one path."""
+    z = np.full((h, w), 5000.0)
+    c = np.arange(1, w - 1)
+    z[h // 2, 1:-1] = 500.0 + c + np.where(c % 2 == 0, 0.0, -3.0)
+    z[0] = z[-1] = synth.NODATA
+    z[:, 0] = z[:, -1] = synth.NODATA
+    return z
+
+
 @pytest.mark.parametrize("flow", [0, 1])
-@pytest.mark.parametrize("case", ["nan_ring", "serpentine"])
+@pytest.mark.parametrize("case", ["nan_ring", "serpentine", "stairs"])
 def test_against_oracle(case, flow):
     from oracle import oracle as O
-    z = _nan_ring(70, 90) if case == "nan_ring" else _serpentine(131, 140)
+    z = {"nan_ring": lambda: _nan_ring(70, 90), "serpentine": lambda: _serpentine(131, 140),
+         "stairs": lambda: _stairs(7, 1500)}[case]()
     h, w = z.shape
     rain = np.full(z.shape, 800.0)
     ctx = lemhip.LemContext(lemhip.default_params(w, h, flow), lemhip.FP64, 0)
