@@ -193,7 +193,9 @@ int lemhip_step_group(lemhip_ctx *const *ctxs, int n, const int *iters, const in
 /* Launch tuning (no reference counterpart).  The dependency engine of the
  * two accumulation passes runs in tiles of dag_tile_w x dag_tile_h cells
  * (64x16, 32x32, 16x64, 128x8, 64x32 or 32x64) and checks convergence on the
- * host every dag_batch round launches; plateau routing advances
+ * host every dag_batch round launches, as long as more tiles are unfinished
+ * than the chip holds (32x32 each); those finish in one launch, on small
+ * grids from the start.  Plateau routing advances
  * plateau_rounds_per_launch (4, 8 or 16) synchronous rounds per launch (8,
  * the default: 16 once few tiles still move).
  * Results never depend on these choices.  lemhip_set_tuning cancels a
