@@ -425,9 +425,10 @@ __global__ void k_fx_parent(const int *count, int cap, const int *ex_recv, const
 
 // one doubling round over the exit forest in two launches: snapshot, then add
 __global__ void k_fx_gather(const int *count, int cap, const unsigned long long *val, const int *P,
-                            unsigned long long *tv, int *tp)
+                            unsigned long long *tv, int *tp, int *flag)
 {
     const int n = fx_count(count, cap);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;   // raised by the scatter that follows
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const int p = P[k];
         tv[k] = val[k];
@@ -568,8 +569,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     while ((1 << batch) < 4 * ((c->W + TW - 1) / TW + (c->H + TH - 1) / TH)) batch++;
     for (int round = 0;; round += batch, batch = 2) {
         for (int q = 0; q < batch; q++) {
-            if (q == batch - 1) LEM_CHECK(c, hipMemsetAsync(&c->scal->nlabels, 0, sizeof(int), c->s));
-            k_fx_gather<<<ge, 256, 0, c->s>>>(a.ex_count, a.ex_cap, a.ex_val, P, tv, tp);
+            k_fx_gather<<<ge, 256, 0, c->s>>>(a.ex_count, a.ex_cap, a.ex_val, P, tv, tp, &c->scal->nlabels);
             k_fx_scatter<<<ge, 256, 0, c->s>>>(a.ex_count, a.ex_cap, a.ex_val, P, tv, tp, &c->scal->nlabels);
         }
         LEM_LAUNCHED(c);

@@ -175,21 +175,14 @@ __device__ __forceinline__ T block_reduce_sum(T v, T *sh)
 
 // routeflow.cu:739-741: the outlet is lowered below the lowest cell after the
 // directions were computed on the unadjusted surface (one thread per slot)
-__global__ void k_slots_outlet_adjust(double *dem, const DemDesc *dd, int ns, DemScal *ds)
+__global__ void k_slots_outlet_adjust(double *dem, uint8_t *fd, const DemDesc *dd, int ns, DemScal *ds)
 {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= ns || dd[j].w == 0) return;
     double lowest = ord_dec(ds[j].lowest_enc);
     ds[j].lowest = lowest;
     if (lowest < dem[ds[j].outlet]) dem[ds[j].outlet] = lowest - 0.0001;
-}
-
-// routeflow.cu:953: fd[outlet] = WEST
-__global__ void k_slots_fd_outlet(uint8_t *fd, const DemDesc *dd, int ns, const DemScal *ds)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ns || dd[j].w == 0) return;
-    fd[ds[j].outlet] = 16;
+    fd[ds[j].outlet] = 16;   // routeflow.cu:953: WEST
 }
 
 // per-slot counter adds from a block: LDS histogram over slots, then one atomic per slot touched
@@ -847,8 +840,10 @@ __global__ void __launch_bounds__(256) k_merge_list(const int *cand, int n, cons
 
 // identify_watershedMFD (newflow.cu:469-487): pointer jumping, four links;
 // in-place reads of already-jumped targets only shorten chains
-__global__ void k_jump(long N, const uint8_t *mask, int *ws)
+// (clears the error flag of the walks and the count of the edge list)
+__global__ void k_jump(long N, const uint8_t *mask, int *ws, int *flag, int *nedges)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = *nedges = 0;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
         const uint8_t m = mask[i];   // loads in flight together
         int v = ws[i];
@@ -1024,17 +1019,6 @@ __global__ void k_edges_decode(const int *cnt, const unsigned long long *ukeys, 
 }
 
 // distinct labels of each slot in the edge set (newflow.cu:1045: data->sinkcount)
-__global__ void __launch_bounds__(256) k_count_labels(long n, const uint8_t *seen, const uint8_t *labdem, int ns,
-                                                      DemScal *ds)
-{
-    __shared__ int hist[LEM_MAX_SLOTS + 1];
-    for (int j = threadIdx.x; j < ns; j += blockDim.x) hist[j] = 0;
-    __syncthreads();
-    for (long l = 1 + blockIdx.x * (long)blockDim.x + threadIdx.x; l < n; l += (long)gridDim.x * blockDim.x)
-        if (seen[l]) atomicAdd(&hist[labdem[l]], 1);
-    slot_hist_flush(hist, ds, (int)offsetof(DemScal, sinkcount), ns);
-}
-
 __global__ void k_slots_sinkcount_init(int ns, DemScal *ds)
 {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1053,8 +1037,16 @@ __global__ void k_slots_sinkcount_fin(const DemDesc *dd, int ns, DemScal *ds)
     else ds[j].sinkcount += ds[j].zero_seen;
 }
 
-__global__ void k_minimax_init(long n, unsigned long long *r, uint8_t *seen)
+// spill heights and label marks; the DEMs' sink counts, the error flag of the
+// walks and the cut-off flag
+__global__ void k_minimax_init(long n, unsigned long long *r, uint8_t *seen, int ns, DemScal *ds, int *flag, int *cut)
 {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < ns) {
+        ds[j].sinkcount = 0;
+        ds[j].zero_seen = 0;
+    }
+    if (j == 0) *flag = *cut = 0;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         r[i] = (i == 0) ? ord_enc(-lm_inf()) : ord_enc(lm_inf());
         seen[i] = 0;
@@ -1105,16 +1097,24 @@ __global__ void k_minimax_relax(int ne, const uint32_t *elo, const uint32_t *ehi
 // by phase parity; nxt: the component each root joins):
 // st[0], st[1]: label 0's running maximum and its component (st[2], st[3] in
 // odd phases)
-__global__ void k_bv_init(long n, uint32_t *comp, unsigned long long *mv, unsigned long long *bw0,
-                          unsigned long long *bw1, uint32_t *be0, uint32_t *be1, unsigned long long *st)
+// (the labels of the edge set are counted per DEM on the way)
+__global__ void __launch_bounds__(256) k_bv_init(long n, uint32_t *comp, unsigned long long *mv,
+                                                 unsigned long long *bw0, unsigned long long *bw1, uint32_t *be0,
+                                                 uint32_t *be1, unsigned long long *st, const uint8_t *seen,
+                                                 const uint8_t *labdem, int ns, DemScal *ds)
 {
+    __shared__ int hist[LEM_MAX_SLOTS + 1];
+    for (int j = threadIdx.x; j < ns; j += blockDim.x) hist[j] = 0;
+    __syncthreads();
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         comp[i] = (uint32_t)i;
         mv[i] = 0ULL;
         bw0[i] = bw1[i] = ~0ULL;
         be0[i] = be1[i] = ~0u;
         if (i == 0) st[0] = st[1] = 0ULL;
+        else if (seen[i]) atomicAdd(&hist[labdem[i]], 1);
     }
+    slot_hist_flush(hist, ds, (int)offsetof(DemScal, sinkcount), ns);
 }
 
 // the lightest outgoing weight of each component.  The edge list is sorted
@@ -1633,12 +1633,12 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
     unsigned long long *mv = c->hvals, *bw[2] = {c->cmax, c->hvals + n}, *st = c->hvals + 2 * n;
     uint32_t *be[2] = {reinterpret_cast<uint32_t *>(c->hkeys), reinterpret_cast<uint32_t *>(c->hkeys) + n};
     uint32_t *nxt = reinterpret_cast<uint32_t *>(c->hkeys) + 2 * n;
-    k_bv_init<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, mv, bw[0], bw[1], be[0], be[1], st);
+    k_bv_init<<<grid1d(n, 256, 2048), 256, 0, c->s>>>(n, c->comp, mv, bw[0], bw[1], be[0], be[1], st, c->seen,
+                                                      c->labdem, c->nslot, c->dsc);
     LEM_LAUNCHED(c);
     const uint32_t *lo = c->elo, *hi = c->ehi;
     const unsigned long long *w = c->ew;
     const int *cnt = &c->scal->nedges;
-    LEM_TRY(clear_flag(c));   // raised only by a pointer walk that does not end
     const int per = n <= (1 << 18) ? 3 : 2;
     // the profile slot times the kernels only, not the host reads between them
     for (int ph = 0, na = bound; na > 0;) {
@@ -1734,9 +1734,8 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
     // (few basins) one jump leaves depression routing at 0.72 ms, two at 0.41,
     // three at 0.37 (1.35 with one link and no progress left); on 8191x7003 (250 cells a
     // basin) a second costs 0.08 of 4.11 ms
-    LEM_TRY(clear_flag(c));
     for (int q = N / (nlab + 1L) > 4096 ? 3 : 1; q > 0; q--)
-        k_jump<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws);
+        k_jump<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag, &c->scal->nedges);
     k_jump_walk<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag);
     LEM_LAUNCHED(c);
     // edges: block-distinct pairs appended, sorted by pair, reduced to the
@@ -1751,7 +1750,7 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
     long np = 0;
     for (int attempt = 0;; ++attempt) {
         LEM_TRY(ensure_hash(c, want));
-        LEM_CHECK(c, hipMemsetAsync(&c->scal->nedges, 0, sizeof(int), c->s));
+        if (attempt) LEM_CHECK(c, hipMemsetAsync(&c->scal->nedges, 0, sizeof(int), c->s));
         dim3 blk(64, 4), grd((W + 63) / 64, (H + 4 * EDGE_RG - 1) / (4 * EDGE_RG));
         k_edges_emit<<<grd, blk, 0, c->s>>>(W, H, c->mask, c->ws, c->dem, c->demid, c->hkeys, c->hvals, c->hcap,
                                             &c->scal->nedges, B);
@@ -1763,8 +1762,11 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
         want = np + np / 4;
         if (attempt > 8) { c->err = "edge list overflow"; return LEMHIP_E_NOMEM; }
     }
-    k_minimax_init<<<grid1d(nlab + 1), 256, 0, c->s>>>(nlab + 1, c->rmm, c->seen);
-    k_slots_sinkcount_init<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->nslot, c->dsc);
+    // labels cut off from label 0 (NaN heights only) raise the flag `cut`, read
+    // with the next pass's first counts: the surface is raised before it is known
+    int *cut = &reinterpret_cast<PlatCtl *>(c->pl_ctl)->cut;
+    k_minimax_init<<<grid1d(std::max(nlab + 1, c->nslot)), 256, 0, c->s>>>(nlab + 1, c->rmm, c->seen, c->nslot, c->dsc,
+                                                                          &c->scal->flag, cut);
     LEM_LAUNCHED(c);
     if (np > 0) {
         unsigned long long *skeys = c->ew2[0], *svals = c->ew2[1];
@@ -1790,14 +1792,8 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
                                                                 c->ew, c->seen, c->labdem, c->dsc);
         LEM_LAUNCHED(c);
     }
-    k_count_labels<<<grid1d(nlab + 1, 256, 1024), 256, 0, c->s>>>(nlab + 1, c->seen, c->labdem, c->nslot, c->dsc);
-    LEM_LAUNCHED(c);
 
     LEM_TRY(spill_heights(c, nlab, (int)np));
-    // labels cut off from label 0 (NaN heights only) raise the flag read with
-    // the next pass's first counts: the surface is raised before it is known
-    int *cut = &reinterpret_cast<PlatCtl *>(c->pl_ctl)->cut;
-    LEM_CHECK(c, hipMemsetAsync(cut, 0, sizeof(int), c->s));
     const int ne = c->h_nedges;
     if (ne > 0) k_fb_unreached<<<grid1d(ne, 256, 1 << 30), 256, 0, c->s>>>(ne, c->elo, c->ehi, c->rmm, cut);
     return raise_surface(c);
@@ -1888,8 +1884,7 @@ static int fd_phase_t(lemhip_ctx *c, int iter)
         c->h_rounds2 = r2;
     }
     k_merge<<<grid1d(N), 256, 0, c->s>>>(N, c->p.flowdirectiontype, c->mask, c->fd, c->SFD);
-    k_slots_fd_outlet<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->fd, c->ddesc, c->nslot, c->dsc);
-    k_slots_outlet_adjust<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->dem, c->ddesc, c->nslot, c->dsc);
+    k_slots_outlet_adjust<<<(c->nslot + 255) / 256, 256, 0, c->s>>>(c->dem, c->fd, c->ddesc, c->nslot, c->dsc);
     LEM_LAUNCHED(c);
     prof_end(c, PROF_FD);
     return LEMHIP_OK;
