@@ -503,6 +503,16 @@ static int fx_grid(long n)
     return (int)g;
 }
 
+// fa as the runoff kernel left it.  Pass A keeps its sums there, and the
+// engine writes only the cells that complete: those on a cycle through an
+// outlet have to find fa = w.  (Bound by HBM; runs only before that engine.)
+__global__ void __launch_bounds__(256) k_fx_undo(long N, const uint8_t *__restrict__ mask, const float *__restrict__ w,
+                                                 float2 *__restrict__ fa)
+{
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x)
+        fa[i] = make_float2(mask[i] ? w[i] : 0.f, 0.f);
+}
+
 // 0: done; 1: inputs the integer form cannot represent exactly (a negative
 // or non-finite runoff weight, or too many tagged cells) — the caller runs
 // the dependency engine instead
@@ -548,6 +558,12 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     a.tag_count = &c->scal->flag;
     a.tag_cap = (int)c->fx_tag_cap;
     a.dsw = c->dsc;
+    auto leave = [&]() -> int {   // after pass A
+        k_fx_undo<<<fx_grid(N), 256, 0, c->s>>>(N, a.mask, a.w, a.fa);
+        LEM_LAUNCHED(c);
+        *fallback = 1;
+        return LEMHIP_OK;
+    };
     constexpr int TW = 64, TH = 32;
     const long ntiles = (long)((c->W + TW - 1) / TW) * ((c->H + TH - 1) / TH);
     // A: in-tile sums, exits, in-tile roots of border cells
@@ -578,7 +594,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
         // the exit values and their snapshot share the 8-byte scratch of N
         // cells; exits are tile border cells (9% of a full tile), so only grids
         // of a few cells could have more
-        if (c->hscal->nedges > a.ex_cap) { *fallback = 1; return LEMHIP_OK; }
+        if (c->hscal->nedges > a.ex_cap) return leave();
         if (!c->hscal->nlabels) break;
         if (round > 64) { c->err = "exit forest did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
@@ -590,7 +606,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
     LEM_LAUNCHED(c);
     LEM_CHECK(c, hipMemcpyAsync(c->hscal, c->scal, sizeof(LemScalars), hipMemcpyDeviceToHost, c->s));
     LEM_CHECK(c, hipStreamSynchronize(c->s));
-    if (c->hscal->flag > a.tag_cap) { *fallback = 1; return LEMHIP_OK; }
+    if (c->hscal->flag > a.tag_cap) return leave();
     c->h_fa_unc = c->hscal->fa_uncomputed;
     c->dag_rounds_last = 0;
     return LEMHIP_OK;
