@@ -37,6 +37,7 @@
 #define FX_NONE 0xFFFFu   // no receiver
 #define FX_EXIT 0xFFFEu   // the receiver is in another tile
 #define FX_ROOT 0x8000u   // pass A: the pointer has reached the path's root
+#define FX_CYCLE (1 << 30)   // in the exit count, more than any list holds: a tile's links close a cycle
 
 // direction index of a single ESRI code, -1 for 0 or a multi-bit code
 __device__ __forceinline__ int fx_dir(uint8_t code)
@@ -261,7 +262,7 @@ __global__ void __launch_bounds__(256, 5) k_fx_sums(FxArgs a)
         T.J[li] = (uint16_t)j;
         jr[q] = j;
     }
-    for (;;) {
+    for (int t = 0;; t++) {
         __syncthreads();
         unsigned long long v[FT::PER];
         uint32_t jj[FT::PER];
@@ -276,6 +277,10 @@ __global__ void __launch_bounds__(256, 5) k_fx_sums(FxArgs a)
             }
         }
         if (!__syncthreads_or(act)) break;
+        if ((1 << t) >= FT::NC) {   // no path in the tile is that long: a cycle
+            if (threadIdx.x == 0) atomicOr(a.ex_count, FX_CYCLE);
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < FT::PER; q++) {
             if (jr[q] & FX_ROOT) continue;
@@ -514,8 +519,9 @@ __global__ void __launch_bounds__(256) k_fx_undo(long N, const uint8_t *__restri
 }
 
 // 0: done; 1: inputs the integer form cannot represent exactly (a negative
-// or non-finite runoff weight, or too many tagged cells) — the caller runs
-// the dependency engine instead
+// or non-finite runoff weight, too many tagged cells, or a cycle that does not
+// pass the outlet: directions from the caller, or an outlet moved after the
+// direction phase) — the caller runs the dependency engine instead
 int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
 {
     *fallback = 0;
@@ -596,7 +602,7 @@ int lem_fa32_sfd(lemhip_ctx *c, int *fallback)
         // of a few cells could have more
         if (c->hscal->nedges > a.ex_cap) return leave();
         if (!c->hscal->nlabels) break;
-        if (round > 64) { c->err = "exit forest did not converge"; return LEMHIP_E_NOT_CONVERGED; }
+        if (round > 64) return leave();   // a cycle across tiles
     }
     // C: final sums, fa, tagged cells
     k_fx_final<TW, TH><<<ntiles, 256, 0, c->s>>>(a);

@@ -102,3 +102,47 @@ def test_cycle_longer_than_the_list():
     assert float(np.max(np.abs(fa - ref) / ref)) <= 1e-6
     for c in ctx:
         c.close()
+
+
+def _accumulate(fd, outlet):
+    """Accumulation of uploaded directions in the FP32 and the FP64 form, and
+    the engine launches of the first."""
+    h, w = fd.shape
+    z = synth.fbm_surface(max(h, w), np.random.default_rng(4))[:h, :w] + 10.0
+    out = []
+    for precision in (lemhip.FP32_KAHAN, lemhip.FP64):
+        c = lemhip.LemContext(lemhip.default_params(w, h), precision, 0)
+        c.init_state(z, np.full(z.shape, 900.0), soilT_mode="nonneg")
+        c.flow_direction(-999)
+        c.runoff()
+        c.upload("fd", fd)
+        c.outlet = outlet
+        c.profile(True)
+        c.flow_accum(-999)
+        out.append((c.download("fa").reshape(h, w), c.summary()["fa_uncomputed"], c.profile_read()["fa_rounds"][1],
+                    c.download("runoff").reshape(h, w)))
+        c.close()
+    assert float(np.max(np.abs(out[0][0] - out[1][0]) / out[1][0])) <= 1e-6
+    assert out[0][1] == out[1][1]
+    return out[0]
+
+
+@pytest.mark.parametrize("col", [20, 63])
+def test_cycle_apart_from_the_outlet(col):
+    """Two cells that point at each other, in one 64 x 32 tile and across two:
+    the integer form hands over to the engine, which leaves them at fa = w."""
+    fd = np.full((40, 130), 16, np.int32)
+    fd[5, col] = 1
+    fa, uncomputed, engine, w = _accumulate(fd, 130 + 10)
+    assert uncomputed == 2 and engine > 0
+    assert np.array_equal(fa[5, col:col + 2], w[5, col:col + 2])
+
+
+def test_longest_path_of_a_tile():
+    """A path through all 2048 cells of a tile is no cycle."""
+    fd = np.full((32, 64), 1, np.int32)
+    fd[1::2] = 16
+    fd[0::2, -1] = fd[1::2, 0] = 4
+    fa, uncomputed, engine, w = _accumulate(fd, 31 * 64)
+    assert uncomputed == 0 and engine == 0
+    assert abs(fa[31, 0] / w.sum() - 1.0) <= 1e-6
