@@ -1097,22 +1097,25 @@ __global__ void k_minimax_relax(int ne, const uint32_t *elo, const uint32_t *ehi
 // by phase parity; nxt: the component each root joins):
 // st[0], st[1]: label 0's running maximum and its component (st[2], st[3] in
 // odd phases)
-// (the labels of the edge set are counted per DEM on the way)
+// (the labels of the edge set are counted per DEM on the way, ns = 0: they have
+// been; heights: the spill heights an earlier start of the phases left, reset)
 __global__ void __launch_bounds__(256) k_bv_init(long n, uint32_t *comp, unsigned long long *mv,
                                                  unsigned long long *bw0, unsigned long long *bw1, uint32_t *be0,
                                                  uint32_t *be1, unsigned long long *st, const uint8_t *seen,
-                                                 const uint8_t *labdem, int ns, DemScal *ds)
+                                                 const uint8_t *labdem, int ns, DemScal *ds,
+                                                 unsigned long long *heights)
 {
     __shared__ int hist[LEM_MAX_SLOTS + 1];
     for (int j = threadIdx.x; j < ns; j += blockDim.x) hist[j] = 0;
     __syncthreads();
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        if (heights) heights[i] = ord_enc(i == 0 ? -lm_inf() : lm_inf());
         comp[i] = (uint32_t)i;
         mv[i] = 0ULL;
         bw0[i] = bw1[i] = ~0ULL;
         be0[i] = be1[i] = ~0u;
         if (i == 0) st[0] = st[1] = 0ULL;
-        else if (seen[i]) atomicAdd(&hist[labdem[i]], 1);
+        else if (ns && seen[i]) atomicAdd(&hist[labdem[i]], 1);
     }
     slot_hist_flush(hist, ds, (int)offsetof(DemScal, sinkcount), ns);
 }
@@ -1195,16 +1198,30 @@ __global__ void k_bv_hook(long n, const uint32_t *__restrict__ lo, const uint32_
     }
 }
 
+// pointer jumping towards the roots, launched only once a walk below gave up
+__global__ void k_bv_jump(long n, uint32_t *nxt)
+{
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const uint32_t t = nxt[i];
+        const uint32_t tt = nxt[t];
+        if (tt != t) nxt[i] = tt;
+    }
+}
+
 // The root of component c's joined component: the pointers form trees whose
 // roots point at themselves (the only cycles Borůvka's choices make under a
 // strict order are pairs, and k_bv_hook turns those into roots).  Most paths
 // have a few links (pointer jumping launched before the walks cost more than it
 // saved: 0.22 instead of 0.19 ms for the phases on 1201^2).  In a longer path,
 // a row of basins with rising sills, each walker leaves its progress at its own
-// component every eight links, so walkers behind it skip ahead.  A walk longer
-// than any tree could be raises the error flag instead of running on.
-#define BV_WALK_MAX (1u << 20)
-__device__ __forceinline__ uint32_t bv_root(uint32_t *nxt, uint32_t c, int *err)
+// component every eight links, so walkers behind it skip ahead.  A path can
+// have as many links as there are labels, and label 0's walk runs in every
+// block before any other has shortened its path, so a walk of more than
+// BV_WALK_MAX links raises the flag instead: the host then starts the phases
+// again with jumps before the walks (260 K basins joining along one path: a
+// step of 4.7 ms, 390 to 630 with walks to the end).
+#define BV_WALK_MAX 512
+__device__ __forceinline__ uint32_t bv_root(uint32_t *nxt, uint32_t c, int *over)
 {
     uint32_t x = nxt[c];
     for (int h = 0; h < 8; h++) {
@@ -1212,13 +1229,13 @@ __device__ __forceinline__ uint32_t bv_root(uint32_t *nxt, uint32_t c, int *err)
         if (y == x) return x;
         x = y;
     }
-    for (uint32_t h = 0; h < BV_WALK_MAX; h++) {
+    for (int h = 0; h < BV_WALK_MAX; h++) {
         if ((h & 7) == 0) __hip_atomic_store(&nxt[c], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const uint32_t y = __hip_atomic_load(&nxt[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (y == x) return x;
         x = y;
     }
-    *err = 1;
+    *over = 1;
     return x;
 }
 
@@ -1229,7 +1246,7 @@ __device__ __forceinline__ uint32_t bv_root(uint32_t *nxt, uint32_t c, int *err)
 __global__ void k_bv_labels(long n, uint32_t *comp, const unsigned long long *__restrict__ bw,
                             const uint32_t *__restrict__ be, uint32_t *nxt,
                             unsigned long long *mv, unsigned long long *r, const unsigned long long *st,
-                            unsigned long long *stn, unsigned long long *bwn, uint32_t *ben, int *err)
+                            unsigned long long *stn, unsigned long long *bwn, uint32_t *ben, int *over)
 {
     const unsigned long long INF = ord_enc(lm_inf()), NEG = ord_enc(-lm_inf());
     __shared__ unsigned long long s_m0;
@@ -1239,7 +1256,7 @@ __global__ void k_bv_labels(long n, uint32_t *comp, const unsigned long long *__
         unsigned long long m = st[0];
         if (be[c0] != ~0u && bw[c0] > m) m = bw[c0];
         s_m0 = m;
-        s_root0 = bv_root(nxt, c0, err);
+        s_root0 = bv_root(nxt, c0, over);
         if (blockIdx.x == 0) {
             stn[0] = m;
             stn[1] = s_root0;
@@ -1253,7 +1270,7 @@ __global__ void k_bv_labels(long n, uint32_t *comp, const unsigned long long *__
         unsigned long long m = mv[i];
         if (be[c] != ~0u && bw[c] > m) m = bw[c];
         mv[i] = m;
-        const uint32_t nc = bv_root(nxt, c, err);
+        const uint32_t nc = bv_root(nxt, c, over);
         comp[i] = nc;
         bwn[i] = ~0ULL;
         ben[i] = ~0u;
@@ -1621,11 +1638,10 @@ static int cutoff_components(lemhip_ctx *c, int nlab, int ne)
 // their grids from the last count the host knows.  A read leaves the device
 // idle for about 15 us, as long as the phase itself on short lists (a step at
 // 512^2 with seven reads fewer, these among them: 1.80 instead of 1.88 ms).
-static int spill_heights(lemhip_ctx *c, int nlab, int bound)
+// jumps: pointer-jumping launches before each phase's walks; *over: a walk gave
+// up, and the heights are of no use.
+static int bv_phases(lemhip_ctx *c, long n, int bound, int jumps, bool *over)
 {
-    const long n = (long)nlab + 1;
-    c->h_nedges = 0;
-    if (bound <= 0) return LEMHIP_OK;
     // per-label scratch: running maxima, chosen weights (parity 1) and label
     // 0's scalars in the hash value table, chosen edges and roots in the hash
     // key table (both >= 8 * (nlab + 1) entries of 8 bytes), chosen weights
@@ -1634,7 +1650,8 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
     uint32_t *be[2] = {reinterpret_cast<uint32_t *>(c->hkeys), reinterpret_cast<uint32_t *>(c->hkeys) + n};
     uint32_t *nxt = reinterpret_cast<uint32_t *>(c->hkeys) + 2 * n;
     k_bv_init<<<grid1d(n, 256, 2048), 256, 0, c->s>>>(n, c->comp, mv, bw[0], bw[1], be[0], be[1], st, c->seen,
-                                                      c->labdem, c->nslot, c->dsc);
+                                                      c->labdem, jumps ? 0 : c->nslot, c->dsc,
+                                                      jumps ? c->rmm : nullptr);
     LEM_LAUNCHED(c);
     const uint32_t *lo = c->elo, *hi = c->ehi;
     const unsigned long long *w = c->ew;
@@ -1652,6 +1669,7 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
             k_bv_min_w<<<ge, 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, bw[p]);
             k_bv_min_e<<<ge, 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, bw[p], be[p]);
             k_bv_hook<<<grid1d(n), 256, 0, c->s>>>(n, lo, hi, c->comp, be[p], nxt, kept);
+            for (int j = 0; j < jumps; j++) k_bv_jump<<<grid1d(n), 256, 0, c->s>>>(n, nxt);
             k_bv_labels<<<grid1d(n), 256, 0, c->s>>>(n, c->comp, bw[p], be[p], nxt, mv, c->rmm, st + 2 * p,
                                                       st + 2 * (p ^ 1), bw[p ^ 1], be[p ^ 1], &c->scal->flag);
             if (na <= BV_KEEP_SHORT)
@@ -1659,14 +1677,15 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
             else
                 k_bv_keep<COMPACT_ITEMS><<<grid_chunks(na), 256, 0, c->s>>>(cnt, lo, hi, w, c->comp, lo2, hi2, w2,
                                                                             kept);
-            prof_end(c, PROF_MM_K, 5);
+            prof_end(c, PROF_MM_K, 5 + jumps);
             LEM_LAUNCHED(c);
             lo = lo2; hi = hi2; w = w2;
             cnt = kept;
         }
         LEM_TRY(read_scalars(c));
         c->h_nedges = c->hscal->nedges;
-        if (c->hscal->flag) { c->err = "spill-height component pointers form a cycle"; return LEMHIP_E_NOT_CONVERGED; }
+        *over = c->hscal->flag != 0;
+        if (*over) return LEMHIP_OK;
         const int nk = c->hscal->kept[(ph - 1) & 1];
         // every component with an outgoing edge joins another each phase, so
         // the components with edges at least halve
@@ -1674,6 +1693,24 @@ static int spill_heights(lemhip_ctx *c, int nlab, int bound)
         na = nk;
         if (ph > 64) { c->err = "spill-height phases did not converge"; return LEMHIP_E_NOT_CONVERGED; }
     }
+    return LEMHIP_OK;
+}
+
+// The phases with walks alone, and if a path was too long for them, once more
+// with as many jumps as the longest path can need.
+static int spill_heights(lemhip_ctx *c, int nlab, int bound)
+{
+    const long n = (long)nlab + 1;
+    c->h_nedges = 0;
+    if (bound <= 0) return LEMHIP_OK;
+    bool over = false;
+    LEM_TRY(bv_phases(c, n, bound, 0, &over));
+    if (!over) return LEMHIP_OK;
+    int jumps = 1;
+    while ((1L << jumps) < n) jumps++;
+    LEM_TRY(clear_flag(c));
+    LEM_TRY(bv_phases(c, n, bound, jumps, &over));
+    if (over) { c->err = "spill-height component pointers form a cycle"; return LEMHIP_E_NOT_CONVERGED; }
     return LEMHIP_OK;
 }
 

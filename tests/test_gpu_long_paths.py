@@ -1,0 +1,48 @@
+"""Depression routing where paths are longer than the walks that follow them:
+basins that join along one path.  Bit-identical with the oracle."""
+import numpy as np
+import pytest
+
+from parallem_amd import lemhip, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _falling_sills(h, w, outlet):
+    """A channel of pits winding through every second row, its sills falling one
+    after the other: every basin, and label 0 before them all, joins the next one
+    along it.  outlet: a valid cell on the DEM's edge beside the first pit."""
+    z = np.full((h, w), 1e7)
+    n = w - 4
+    for k, r in enumerate(range(2, h - 2, 2)):
+        p = k * (n + 1) + np.arange(n + 1)
+        v = 4e6 - p - 3.0 * (p % 2)
+        z[r, 2:w - 2] = v[:n] if k % 2 == 0 else v[n - 1::-1]
+        if r + 2 < h - 2:
+            z[r + 1, w - 3 if k % 2 == 0 else 2] = v[n]
+    z[0] = z[-1] = synth.NODATA
+    z[:, 0] = z[:, -1] = synth.NODATA
+    if outlet:
+        z[1, 2], z[0, 2] = 4e6, 4e6 - 10
+    return z
+
+
+# 1307 and 2997 basins: more than a walk follows; 1103026: more than 2^20
+@pytest.mark.parametrize("h, w, outlet, flow", [(40, 150, True, 0), (40, 150, True, 1), (7, 3000, True, 0),
+                                                (2105, 2104, False, 0)])
+def test_basins_joining_along_one_path(h, w, outlet, flow):
+    from oracle import oracle as O
+    z = _falling_sills(h, w, outlet)
+    rain = np.full(z.shape, 800.0)
+    ctx = lemhip.LemContext(lemhip.default_params(w, h, flow), lemhip.FP64, 0)
+    ctx.init_state(z, rain, soilT_mode="nonneg")
+    orc = O.Oracle(z, rain, O.default_params(w, h, flow), soilT_mode="nonneg", openmp=True)
+    ctx.step(-1000)
+    orc.step(-1000)
+    s, o = ctx.summary(), orc.scalars()
+    for f in ("sinkcount", "plateau_rounds1", "plateau_rounds2"):
+        assert s[f] == o[f], f
+    for f in ("fd", "SFD"):   # downloads carry -9999 on nodata
+        assert np.array_equal(ctx.download(f), np.where(orc["mask"] != 0, orc[f], -9999)), f
+    assert np.array_equal(ctx.download("fa"), orc["fa"], equal_nan=True)
+    ctx.close()
