@@ -838,9 +838,10 @@ __global__ void __launch_bounds__(256) k_merge_list(const int *cand, int n, cons
     }
 }
 
-// identify_watershedMFD (newflow.cu:469-487): pointer jumping, four links;
+// identify_watershedMFD (newflow.cu:469-487): pointer jumping, LINKS links;
 // in-place reads of already-jumped targets only shorten chains
-// (clears the error flag of the walks and the count of the edge list)
+// (clears the flag of the walks and the count of the edge list)
+template <int LINKS>
 __global__ void k_jump(long N, const uint8_t *mask, int *ws, int *flag, int *nedges)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) *flag = *nedges = 0;
@@ -848,7 +849,7 @@ __global__ void k_jump(long N, const uint8_t *mask, int *ws, int *flag, int *ned
         const uint8_t m = mask[i];   // loads in flight together
         int v = ws[i];
         if (v >= 0 || !m) continue;
-        for (int q = 0; q < 4 && v < 0; q++) v = ws[-v - 1];
+        for (int q = 0; q < LINKS && v < 0; q++) v = ws[-v - 1];
         ws[i] = v;
     }
 }
@@ -858,19 +859,20 @@ __global__ void k_jump(long N, const uint8_t *mask, int *ws, int *flag, int *ned
 // ahead.  (Walks that left only their label took 1.10 ms on a smooth 2000x1500
 // DEM, paths of up to some 3000 cells; a list of the cells still pointing and
 // launches over it until none was left cost two host reads and nine launches
-// more: 0.12 ms of a 512^2 DEM's step.)  A walk longer than any chain raises
-// the error flag.
-__global__ void k_jump_walk(long N, const uint8_t *mask, int *ws, int *err)
+// more: 0.12 ms of a 512^2 DEM's step.)  A walk ends after `limit` links and
+// says so: the cells downstream of a long path may not have started yet, and
+// then a winding valley is walked link by link (see WS_JUMPS).
+__global__ void k_jump_walk(long N, const uint8_t *mask, int *ws, int limit, int *more)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
         int v = ws[i];
         if (v >= 0 || !mask[i]) continue;
-        long hops = 0;
+        int hops = 0;
         do {
             v = __hip_atomic_load(&ws[-v - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (v < 0 && (++hops & 7) == 0) __hip_atomic_store(&ws[i], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } while (v < 0 && hops <= N);
-        if (v < 0) *err = 1;
+        } while (v < 0 && hops < limit);
+        if (v < 0) *more = 1;
         ws[i] = v;
     }
 }
@@ -906,8 +908,10 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long k)
 __global__ void __launch_bounds__(256) k_edges_emit(int W, int H, const uint8_t *__restrict__ mask,
                                                     const int *__restrict__ ws, const double *__restrict__ z,
                                                     const uint8_t *__restrict__ demid, unsigned long long *keys,
-                                                    unsigned long long *vals, long cap, int *count, int B)
+                                                    unsigned long long *vals, long cap, int *count, int B,
+                                                    const int *unfinished)
 {
+    if (*unfinished) return;   // some cell has no label yet: the host runs this again
     __shared__ unsigned long long lk[EDGE_LDS], lv[EDGE_LDS];
     __shared__ int s_wave[4];
     __shared__ int s_base;
@@ -1766,14 +1770,24 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
     }
     const int nlab = c->hscal->nlabels;
     c->h_nlab = nlab;
-    // watershed labels: one jump over every cell, three where basins are large
-    // and so paths long, then each walks the rest.  On the smooth 2000x1500 DEM
-    // (few basins) one jump leaves depression routing at 0.72 ms, two at 0.41,
-    // three at 0.37 (1.35 with one link and no progress left); on 8191x7003 (250 cells a
-    // basin) a second costs 0.08 of 4.11 ms
-    for (int q = N / (nlab + 1L) > 4096 ? 3 : 1; q > 0; q--)
-        k_jump<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag, &c->scal->nedges);
-    k_jump_walk<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag);
+    // watershed labels: one jump over every cell, two or three where basins are
+    // large and so paths long, then each walks the rest.  On the smooth 2000x1500
+    // DEM (few basins) one jump leaves depression routing at 0.72 ms, two at 0.41,
+    // three at 0.37 (1.35 with one link and no progress left); on a straight
+    // valley of 4096 rows (2900 cells a basin) one leaves it at 1.49 ms, two at
+    // 1.05; on 8191x7003 (250 cells a basin) a second costs 0.08 of 4.11 ms.
+    // A walk takes at most 256 links, after three jumps 128.  Where that is not
+    // enough, WS_JUMPS jumps of one link each, which double what a pointer
+    // spans, and more walks follow until every cell has its label: a valley
+    // winding over 4096^2 2.9 ms, 4.6 with many small basins beside it (89 and
+    // 1740 with walks to the end; 2.0 at 64 links, but then 0.1 more on the
+    // straight valley)
+#define WS_JUMPS 8
+    const long basin = N / (nlab + 1L);   // cells of one, on average
+    const int limit = basin > 4096 ? 128 : 256;
+    for (int q = basin > 4096 ? 3 : basin > 1024 ? 2 : 1; q > 0; q--)
+        k_jump<4><<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag, &c->scal->nedges);
+    k_jump_walk<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, limit, &c->scal->flag);
     LEM_LAUNCHED(c);
     // edges: block-distinct pairs appended, sorted by pair, reduced to the
     // minimum weight per pair; the list comes out sorted by label (the
@@ -1785,15 +1799,25 @@ static int flooding(lemhip_ctx *c, int ncand1, int *sinks)
     long want = 8L * (nlab + 1);
     if (want < 1024) want = 1024;
     long np = 0;
-    for (int attempt = 0;; ++attempt) {
+    for (int attempt = 0, walks = 0;; ++attempt) {
         LEM_TRY(ensure_hash(c, want));
         if (attempt) LEM_CHECK(c, hipMemsetAsync(&c->scal->nedges, 0, sizeof(int), c->s));
         dim3 blk(64, 4), grd((W + 63) / 64, (H + 4 * EDGE_RG - 1) / (4 * EDGE_RG));
         k_edges_emit<<<grd, blk, 0, c->s>>>(W, H, c->mask, c->ws, c->dem, c->demid, c->hkeys, c->hvals, c->hcap,
-                                            &c->scal->nedges, B);
+                                            &c->scal->nedges, B, &c->scal->flag);
         LEM_LAUNCHED(c);
         LEM_TRY(read_scalars(c));
-        if (c->hscal->flag) { c->err = "watershed pointer jumping did not converge"; return LEMHIP_E_NOT_CONVERGED; }
+        if (c->hscal->flag) {   // paths longer than one launch's walks
+            for (int more = 1; more;) {
+                if (++walks > 8) { c->err = "watershed pointer jumping did not converge"; return LEMHIP_E_NOT_CONVERGED; }
+                for (int q = 0; q < WS_JUMPS; q++)
+                    k_jump<1><<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, &c->scal->flag, &c->scal->nedges);
+                k_jump_walk<<<grid1d(N), 256, 0, c->s>>>(N, c->mask, c->ws, limit, &c->scal->flag);
+                LEM_LAUNCHED(c);
+                LEM_TRY(read_flag(c, &more));
+            }
+            continue;
+        }
         np = c->hscal->nedges;
         if (np <= c->hcap) break;
         want = np + np / 4;
