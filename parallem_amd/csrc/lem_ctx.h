@@ -144,6 +144,7 @@ struct lemhip_ctx {
     int res_cap = 0;                                  // tiles the buffers hold
     int dag_round = 0;
     int dag_rounds_last = 0;
+    bool dag_shaped = false;    // a pass launched rounds in the tuned tile shape since the tuner cleared this
     int plat_k = 8;             // plateau rounds per launch (4, 8 or 16; 8: 16 once few tiles move)
     int plat_grid[2][2] = {};   // workgroups of the plateau kernels (plat_grids)
     // lemhip_autotune sets both; each tuner clears its own flag once it has run

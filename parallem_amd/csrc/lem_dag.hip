@@ -1527,6 +1527,7 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
         return LEMHIP_OK;
     }
     long guard = 0;
+    c->dag_shaped = true;
     for (;;) {
         LEM_CHECK(c, hipMemsetAsync(&ctl->flag, 0, sizeof(int), c->s));
         prof_begin(c, prof_slot);
@@ -1654,8 +1655,10 @@ int lem_sed_first(lemhip_ctx *c, int rounds, const int *skip)
 
 // Times flow accumulation with every tile shape, then the best shape with
 // several launch batches, on the current directions and runoff weights (the
-// pass is idempotent), and keeps the fastest.  Results do not depend on the
-// choice.
+// pass is idempotent), and keeps the fastest, or what the context had if
+// resident tiles took the whole pass every time (then the times say nothing of
+// shape and batch, which the sediment pass may still use: fewer of its tiles
+// fit the chip).  Results do not depend on the choice.
 int lem_tune_dag(lemhip_ctx *c)
 {
     hipEvent_t e0, e1;
@@ -1671,7 +1674,9 @@ int lem_tune_dag(lemhip_ctx *c)
     };
     float best = 1e30f;
     int bs = c->dag_shape;
+    const int shape0 = bs, batch0 = c->dag_batch;
     c->dag_batch = 16;
+    c->dag_shaped = false;
     for (int k = 0; k < lem_dag_shape_count(); k++) {
         c->dag_shape = k;
         float ms = 0.f;
@@ -1690,6 +1695,7 @@ int lem_tune_dag(lemhip_ctx *c)
         if (ms < best) { best = ms; bb = BATCHES[q]; }
     }
     c->dag_batch = bb;
+    if (!c->dag_shaped) { c->dag_shape = shape0; c->dag_batch = batch0; }   // resident tiles alone were timed
     c->tune_dag_pending = false;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -1734,7 +1740,9 @@ int lem_tune_sed(lemhip_ctx *c)
     LEM_TRY(copy_all(true));
     float best = 1e30f;
     int bs = c->dag_shape;
+    const int shape0 = bs, batch0 = c->dag_batch;
     c->dag_batch = 16;
+    c->dag_shaped = false;
     for (int k = 0; k < lem_dag_shape_count(); k++) {
         c->dag_shape = k;
         float ms = 0.f;
@@ -1753,6 +1761,7 @@ int lem_tune_sed(lemhip_ctx *c)
         if (ms < best) { best = ms; bb = BATCHES[q]; }
     }
     c->dag_batch = bb;
+    if (!c->dag_shaped) { c->dag_shape = shape0; c->dag_batch = batch0; }   // resident tiles alone were timed
     LEM_TRY(copy_all(false));
     LEM_CHECK(c, hipStreamSynchronize(c->s));
     c->tune_dag_pending = false;
