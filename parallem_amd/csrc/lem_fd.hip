@@ -1937,8 +1937,10 @@ static int fd_phase_t(lemhip_ctx *c, int iter)
         bool cut = false;
         LEM_TRY(directions_and_plateaus<TS>(c, c->z2, (TS *)nullptr, &n2, &r2, &cut));
         if (cut) {
+            prof_begin(c, PROF_FLOOD);
             LEM_TRY(cutoff_components(c, c->h_nlab, c->h_nedges));
             LEM_TRY(raise_surface(c));
+            prof_end(c, PROF_FLOOD, 0);
         }
         if (c->tune_plat_pending) LEM_TRY(tune_plateau<TS>(c, c->z2, (TS *)nullptr));
         if (cut) LEM_TRY(directions_and_plateaus<TS>(c, c->z2, (TS *)nullptr, &n2, &r2));

@@ -90,3 +90,24 @@ def test_time_of_a_winding_valley():
     ms = ctx.profile_read()["depression"][0]
     ctx.close()
     assert 0 < ms < 30
+
+
+def test_cut_off_basins_are_timed_as_depression_routing():
+    """A row of basins inside a NaN ring: their spill heights take hundreds of
+    relaxation passes, found necessary only once the surface was raised."""
+    z = np.full((11, 800), 5000.0)
+    c = np.arange(3, 797)
+    z[5, 3:-3] = 500.0 + c + np.where(c % 2 == 0, 0.0, -3.0)
+    z[1:-1, 1] = z[1:-1, -2] = z[1, 1:-1] = z[-2, 1:-1] = np.nan
+    z[0] = z[-1] = synth.NODATA
+    z[:, 0] = z[:, -1] = synth.NODATA
+    ctx = lemhip.LemContext(lemhip.default_params(800, 11), lemhip.FP64, 0)
+    ctx.init_state(z, np.full(z.shape, 800.0), soilT_mode="nonneg")
+    ctx.flow_direction(-1000)
+    ctx.profile(True)
+    ctx.flow_direction(-999)
+    p = ctx.profile_read()
+    ctx.close()
+    # hundreds of passes at some 10 us each, against a millisecond of other phases
+    assert p["depression"][0] > 0.5 * p["fd"][0]
+    assert p["depression"][1] == 1
