@@ -8,8 +8,10 @@
 // each workgroup owns a tile of cells, runs the tile's local dependency chains
 // to completion in LDS-synchronised iterations, and only chains that cross a
 // tile edge wait for the next round.  A cell's status word records the round
-// in which it completed, so a workgroup trusts another tile's value only when
-// it was written in an earlier launch (kernel boundary = visibility point).
+// in which it completed, so in these launch rounds a workgroup trusts another
+// tile's value only when it was written in an earlier launch (kernel boundary =
+// visibility point).  The resident tiles that finish a pass exchange edge
+// values within one launch instead, each a word that is final by itself.
 #include "lem_ctx.h"
 #include <string.h>
 #include <type_traits>

@@ -214,7 +214,7 @@ __device__ __forceinline__ void fx_load(const FxArgs &a, int tx0, int ty0, FxTil
 //
 // Both passes are bound by the latency of what a tile waits for (loads, seven
 // rounds here, a path of the tile's height or so there) and hide it with five
-// and seven tiles per compute unit.  One workgroup per tile: in a loop over
+// and six tiles per compute unit.  One workgroup per tile: in a loop over
 // tiles the compiler keeps every cell's offsets in registers across the loop
 // (155 of them, three tiles per compute unit).  4096^2: 285 -> 176 us here
 // (a second pointer array for the roots and a wait per cell's weight before)

@@ -1022,7 +1022,8 @@ __global__ void k_edges_decode(const int *cnt, const unsigned long long *ukeys, 
     if (lo == 0 && !ds[labdem[hi]].zero_seen) ds[labdem[hi]].zero_seen = 1;
 }
 
-// distinct labels of each slot in the edge set (newflow.cu:1045: data->sinkcount)
+// nothing to flood: every slot's sink count (newflow.cu:1045: data->sinkcount, the
+// distinct labels in the edge set, counted by k_bv_init) is 0
 __global__ void k_slots_sinkcount_init(int ns, DemScal *ds)
 {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1041,7 +1042,7 @@ __global__ void k_slots_sinkcount_fin(const DemDesc *dd, int ns, DemScal *ds)
     else ds[j].sinkcount += ds[j].zero_seen;
 }
 
-// spill heights and label marks; the DEMs' sink counts, the error flag of the
+// spill heights and label marks; the DEMs' sink counts, the flag of the
 // walks and the cut-off flag
 __global__ void k_minimax_init(long n, unsigned long long *r, uint8_t *seen, int ns, DemScal *ds, int *flag, int *cut)
 {
