@@ -600,8 +600,9 @@ __global__ void __launch_bounds__(256) k_sed_prep(int W, int H, const uint8_t *_
 struct DagCtl {
     int cnt[3];
     int pad0[29];
-    int flag;
-    int pad1[31];
+    int flag;   // some tile made progress in the batch
+    int left;   // tiles with a pending cell after the batch (k_dag_left)
+    int pad1[30];
 };
 
 
@@ -974,8 +975,12 @@ static_assert(sizeof(ResCtl) <= LEM_RES_CTL && RES_EDGE == LEM_RES_EDGE && RES_T
 
 // Tiles with a pending cell, in list; pos[tile]: its place there, or -1.  The
 // exchange entries of the first `cap` listed tiles are cleared.
+// wake: the wake stamps of the launch rounds in tiles of tw x th cells, or null
+// before any: the status words of a tile that lies in finished ones alone are
+// not read (on 16384^2 that is 1 GB, 0.6 ms a listing).
 #define RES_LIST_TILES 4
-__global__ void __launch_bounds__(256) k_res_list(int W, int H, const int *__restrict__ st, int cap, int *list,
+__global__ void __launch_bounds__(256) k_res_list(int W, int H, const int *__restrict__ st,
+                                                  const int *__restrict__ wake, int tw, int th, int cap, int *list,
                                                   int *pos, unsigned long long *ex, ResCtl *ctl)
 {
     __shared__ int s_pend[RES_LIST_TILES], s_base;
@@ -986,11 +991,18 @@ __global__ void __launch_bounds__(256) k_res_list(int W, int H, const int *__res
 #pragma unroll
     for (int j = 0; j < RES_LIST_TILES; j++) {
         const int t = t0 + j, tx0 = (t % ntx) * RES_T, ty0 = (t / ntx) * RES_T;
+        bool open = t < ntiles;
+        if (open && wake) {
+            open = false;
+            const int x1 = tx0 + RES_T < W ? tx0 + RES_T : W, y1 = ty0 + RES_T < H ? ty0 + RES_T : H;
+            for (int y = ty0 / th; y * th < y1; y++)
+                for (int x = tx0 / tw; x * tw < x1; x++) open |= wake[y * ((W + tw - 1) / tw) + x] != DAG_TILE_DONE;
+        }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const int li = threadIdx.x + q * 256;
             const int r = ty0 + li / RES_T, c = tx0 + li % RES_T;
-            v[j][q] = t < ntiles && r < H && c < W ? st[(long)r * W + c] : 0;
+            v[j][q] = open && r < H && c < W ? st[(long)r * W + c] : 0;
         }
     }
     __syncthreads();
@@ -1419,6 +1431,16 @@ static int grid1d_dag(long n)
     return (int)g;
 }
 
+// tiles of the launch rounds that still hold a pending cell
+__global__ void __launch_bounds__(256) k_dag_left(int n, const int *__restrict__ wake, int *left)
+{
+    int mine = 0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        mine += wake[i] != DAG_TILE_DONE;
+    for (int d = 32; d; d >>= 1) mine += __shfl_xor(mine, d);
+    if ((threadIdx.x & 63) == 0 && mine) atomicAdd(left, mine);
+}
+
 // every tile on the list; none if *skip
 __global__ void k_iota(int n, int *a, int *count, const int *skip)
 {
@@ -1430,10 +1452,19 @@ __global__ void k_iota(int n, int *a, int *count, const int *skip)
 // Finishes the pass with resident tiles if the unfinished ones fit the chip
 // (*done = 1, the uncomputed cells in *uncomputed).  If all of the grid's tiles
 // do, the launch takes the device's count and the host reads nothing before
-// it.  over: by how many the unfinished tiles are too many, if by less than half.
+// it.  After launch rounds their number is estimated first, and nothing is
+// listed while it is too large: on 16384^2 in the FP64 form a listing after each
+// batch of 16 rounds, with its host read, made flow accumulation 66 ms
+// instead of 41.
+struct ResAfter {
+    int tw, th;    // tile shape of the rounds
+    int left;      // of those tiles, how many are unfinished
+    float per;     // resident tiles to each: the least there can be, then as last listed
+    int over;      // by how many the unfinished resident tiles are too many, if by less than half
+};
 template <class Cell, bool SFD>
 static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, int *done, int prof_slot,
-                        int *over = nullptr)
+                        ResAfter *after = nullptr)
 {
     *done = 0;
     const int ntiles = ((c->W + RES_T - 1) / RES_T) * ((c->H + RES_T - 1) / RES_T);
@@ -1441,22 +1472,26 @@ static int run_resident(lemhip_ctx *c, Cell cell, int *round, int *uncomputed, i
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_dag_resident<Cell, SFD>, 256, 0) != hipSuccess || bpc < 1)
         return LEMHIP_OK;
     const int cap = bpc * c->ncu < c->res_cap ? bpc * c->ncu : c->res_cap;
+    auto too_many = [&](int n) {
+        if (after) after->over = n > cap && n < cap + cap / 2 ? n - cap : 0;
+        return n > cap;
+    };
+    if (after && too_many((int)(after->per * after->left))) return LEMHIP_OK;
     int *st = reinterpret_cast<int *>(c->scan_tmp);
     ResCtl *ctl = reinterpret_cast<ResCtl *>(c->res_ctl);
     for (;;) {
         LEM_CHECK(c, hipMemsetAsync(ctl, 0, 4 * sizeof(int), c->s));
-        k_res_list<<<(ntiles + RES_LIST_TILES - 1) / RES_LIST_TILES, 256, 0, c->s>>>(c->W, c->H, st, cap, c->res_list,
-                                                                                    c->res_pos, c->res_ex, ctl);
+        k_res_list<<<(ntiles + RES_LIST_TILES - 1) / RES_LIST_TILES, 256, 0, c->s>>>(
+            c->W, c->H, st, after ? c->dag_wake : nullptr, after ? after->tw : 0, after ? after->th : 0, cap,
+            c->res_list, c->res_pos, c->res_ex, ctl);
         LEM_LAUNCHED(c);
         int n = ntiles;
         if (n > cap) {
             LEM_CHECK(c, hipMemcpyAsync(&c->hint[40], &ctl->n, sizeof(int), hipMemcpyDeviceToHost, c->s));
             LEM_CHECK(c, hipStreamSynchronize(c->s));
             n = c->hint[40];
-            if (n > cap) {
-                if (over && n < cap + cap / 2) *over = n - cap;
-                return LEMHIP_OK;
-            }
+            if (after && after->left > 0) after->per = (float)n / after->left;
+            if (too_many(n)) return LEMHIP_OK;
         }
         ++*round;
         prof_begin(c, prof_slot);
@@ -1530,8 +1565,11 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
     }
     long guard = 0;
     c->dag_shaped = true;
+    // at most `cover` of these tiles meet in one resident tile
+    constexpr int cover = (TW < RT ? RT / TW : 1) * (TH < RT ? RT / TH : 1);
+    ResAfter after{TW, TH, 0, 1.f / cover, 0};
     for (;;) {
-        LEM_CHECK(c, hipMemsetAsync(&ctl->flag, 0, sizeof(int), c->s));
+        LEM_CHECK(c, hipMemsetAsync(&ctl->flag, 0, 2 * sizeof(int), c->s));   // and left
         prof_begin(c, prof_slot);
         for (int q = 0; q < batch; q++) {
             ++r;
@@ -1539,14 +1577,16 @@ static int run_rounds(lemhip_ctx *c, Cell cell, int *uncomputed, int prof_slot, 
                                                            L[(r + 1) % 3], c->dag_wake, ctl);
         }
         prof_end(c, prof_slot, batch);
+        k_dag_left<<<grid1d_dag(ntiles / 16), 256, 0, c->s>>>(ntiles, c->dag_wake, &ctl->left);
         LEM_LAUNCHED(c);
-        LEM_CHECK(c, hipMemcpyAsync(&c->hint[20], &ctl->flag, sizeof(int), hipMemcpyDeviceToHost, c->s));
+        LEM_CHECK(c, hipMemcpyAsync(&c->hint[20], &ctl->flag, 2 * sizeof(int), hipMemcpyDeviceToHost, c->s));
         LEM_CHECK(c, hipStreamSynchronize(c->s));
         if (!c->hint[20]) break;
-        int over = 0;
-        LEM_TRY((run_resident<std::remove_const_t<decltype(rcell)>, SFD>(c, rcell, &r, uncomputed, &done, prof_slot, &over)));
+        after.left = c->hint[21];
+        LEM_TRY((run_resident<std::remove_const_t<decltype(rcell)>, SFD>(c, rcell, &r, uncomputed, &done, prof_slot,
+                                                                         &after)));
         // not many more tiles than fit: look again soon
-        if (over > 0 && BATCH > 4) batch = 4;
+        if (after.over > 0 && BATCH > 4) batch = 4;
         if (done) {
             c->dag_rounds_last = r - c->dag_round;
             c->dag_round = r;

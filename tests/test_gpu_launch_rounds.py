@@ -129,3 +129,25 @@ def test_fp32_contexts_that_do_not_fit_at_once():
         alone.close()
     for c in together:
         c.close()
+
+
+def test_time_of_looking_for_the_end_of_the_rounds():
+    """8192^2: looking every 4 launches whether the unfinished tiles fit the chip costs
+    little more than every 16 (3%; with a listing of the whole grid each time, 19%)."""
+    z = synth.fbm_surface(2048, np.random.default_rng(9))
+    z = np.block([[z, z[:, ::-1]], [z[::-1], z[::-1, ::-1]]])
+    z = np.block([[z, z], [z, z]])
+    synth.add_tilt(z)
+    z[0] = z[-1] = synth.NODATA
+    z[:, 0] = z[:, -1] = synth.NODATA
+    c = _context(z, 0, dag_tile=(64, 16))
+    c.flow_direction(-1000)
+    c.runoff()
+    ms = {}
+    for batch in (16, 4, 16, 4, 16, 4):
+        c.set_tuning(dag_batch=batch)
+        c.profile(True)
+        c.flow_accum(-1000)
+        ms[batch] = min(ms.get(batch, 1e9), c.profile_read()["flow_accum"][0])
+    c.close()
+    assert 0 < ms[4] < 1.1 * ms[16], ms
