@@ -9,6 +9,7 @@
 #include <vector>
 #include <type_traits>
 #include <thread>
+#include <type_traits>
 #include <mutex>
 
 static int grid1d(long n, int block = 256, int cap = 8192)
@@ -621,29 +622,44 @@ static int rect_copy(lemhip_ctx *c, void *buf, void *base, int plane, size_t es,
     return LEMHIP_OK;
 }
 
-// Rows r0.. of rectangle D of a field, as the host receives them: row-major,
-// `ne` values per cell (8 for Slopes, direction-minor), widened to double, or
-// to int for codes and the mask (nodata cells carry -9999 in the reference's
-// fd/SFD, newflow.cu:74-78).
-// Bound by HBM (a cell's element read, its host element written).  Packing on
-// the device makes every download one contiguous copy: rows of an odd pitch
+// Rows r0.. of rectangle D of a field in the order the host receives them:
+// row-major, `ne` values per cell (8 for Slopes, direction-minor), as narrow as
+// they are: directions in 16 bits, since nodata cells carry -9999 in the
+// reference's fd/SFD (newflow.cu:74-78), float pairs as their sum.
+// Bound by the host link where it writes to pinned memory, else by HBM.  Packing
+// on the device makes every download one contiguous copy: rows of an odd pitch
 // went through the strided copy's slow path (the directions of a 1201^2 DEM:
-// 18.8 ms, now 0.5 ms), and the conversions ran on one host thread.
-template <typename S, typename O>
+// 18.8 ms, now 0.2 ms).
+template <typename S, typename P>
 __global__ void __launch_bounds__(256) k_pack(int W, DemDesc D, int r0, long n, const S *__restrict__ src, long plane,
-                                              int ne, const uint8_t *__restrict__ mask, O *__restrict__ out)
+                                              int ne, const uint8_t *__restrict__ mask, P *__restrict__ out)
 {
     for (long k = blockIdx.x * (long)blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
         const int row = (int)(k / D.w), col = (int)(k % D.w);
         const long i = (long)(D.y0 + r0 + row) * W + D.x0 + col;
-        if constexpr (sizeof(O) == sizeof(int)) {
-            out[k] = !mask || mask[i] ? (O)src[i] : (O)-9999;
-        } else if constexpr (sizeof(S) == sizeof(float2) && !__is_same(S, double)) {
+        if constexpr (std::is_same_v<P, int16_t>) {
+            out[k] = mask[i] ? (P)src[i] : (P)-9999;
+        } else if constexpr (std::is_same_v<S, float2>) {
             const float2 v = src[i];
             out[k] = (double)v.x + (double)v.y;
         } else {
-            for (int d = 0; d < ne; d++) out[ne * k + d] = (O)src[d * plane + i];
+            for (int d = 0; d < ne; d++) out[ne * k + d] = src[d * plane + i];
         }
+    }
+}
+
+// n packed values into the caller's memory, widened to the host's type.  On the
+// host, where each value is read and written in any case: widening on the device
+// sent two to four times the bytes over the link (the mask of a 1024^2 DEM 0.22
+// instead of 0.08 ms, the directions 0.22 instead of 0.13).
+template <typename P, typename O> static void widen(const char *from, char *to, size_t n)
+{
+    if constexpr (std::is_same_v<P, O>) {
+        memcpy(to, from, n * sizeof(O));
+    } else {
+        const P *p = reinterpret_cast<const P *>(from);
+        O *o = reinterpret_cast<O *>(to);
+        for (size_t i = 0; i < n; i++) o[i] = (O)p[i];
     }
 }
 
@@ -657,7 +673,7 @@ __global__ void __launch_bounds__(256) k_pack(int W, DemDesc D, int r0, long n, 
 #define DL_DIRECT ((size_t)4 << 20)
 #define DL_THREADS 4
 static_assert(2 * DL_THREADS <= sizeof(lemhip_ctx::dl_ev) / sizeof(hipEvent_t), "one event per pinned chunk");
-static int copy_out(lemhip_ctx *c, const char *dev, char *host, size_t bytes)
+template <typename P, typename O> static int copy_out(lemhip_ctx *c, const char *dev, char *host, size_t bytes)
 {
     LEM_TRY(stage_reserve(c, 2 * (size_t)DL_THREADS * DL_CHUNK));
     for (hipEvent_t &e : c->dl_ev)
@@ -677,7 +693,8 @@ static int copy_out(lemhip_ctx *c, const char *dev, char *host, size_t bytes)
             if (e == hipSuccess) e = hipEventSynchronize(c->dl_ev[2 * t + j]);
             const size_t off = k * DL_CHUNK;
             if (e == hipSuccess)
-                memcpy(host + off, (char *)c->stage + (2 * t + j) * DL_CHUNK, std::min((size_t)DL_CHUNK, bytes - off));
+                widen<P, O>((char *)c->stage + (2 * t + j) * DL_CHUNK, host + off / sizeof(P) * sizeof(O),
+                            std::min((size_t)DL_CHUNK, bytes - off) / sizeof(P));
         }
         return e;
     };
@@ -700,24 +717,18 @@ static int copy_out(lemhip_ctx *c, const char *dev, char *host, size_t bytes)
     return LEMHIP_OK;
 }
 
-static int slot_download(lemhip_ctx *c, int slot, int field, void *host)
+// field src of S, `ne` values per cell, packed as P and widened to O
+template <typename S, typename P, typename O>
+static int pack_out(lemhip_ctx *c, const DemDesc &D, const void *src, int ne, const uint8_t *mask, void *host)
 {
-    int kind = -1;
-    void *src = field_ptr(c, field, &kind);
-    if (!src) { c->err = "unknown field"; return LEMHIP_E_ARG; }
-    DemDesc D;
-    LEM_TRY(slot_rect(c, slot, 2, &D));
-    LEM_CHECK(c, hipSetDevice(c->dev));
-    const bool whole = kind == 2 || kind == 3, f64 = c->prec == LEMHIP_FP64;
-    const int ne = kind == 4 ? 8 : 1;
-    const size_t cell = whole ? sizeof(int) : ne * sizeof(double);
-    // up to DL_DIRECT bytes are packed straight into pinned host memory (a copy
-    // behind the kernel makes a 96^2 field's 17 us 28, a 512^2 one's 125 us 140).
-    // Otherwise the staging
-    // that initialised the slot holds 8 bytes per cell of its DEM, and Slopes
-    // go in bands of rows.
-    const size_t total = cell * D.w * D.h;
-    const bool direct = total <= DL_DIRECT;
+    // up to DL_DIRECT bytes, widened to twice that at most, are packed straight
+    // into pinned host memory (a copy behind the kernel makes a 96^2 field's 17 us
+    // 28, a 512^2 one's 125 us 140; a float field of 1024^2 0.25 ms, 0.52 on
+    // several threads; the mask of 2048^2, 16 MB widened, 0.46 and 0.31).
+    // Otherwise the staging that initialised the slot holds 8 bytes per cell of
+    // its DEM, and Slopes go in bands of rows.
+    const size_t cell = ne * sizeof(P), total = cell * D.w * D.h;
+    const bool direct = total <= DL_DIRECT && total / sizeof(P) * sizeof(O) <= 2 * DL_DIRECT;
     int band = D.h;
     if (direct) {
         LEM_TRY(stage_reserve(c, total));
@@ -729,26 +740,35 @@ static int slot_download(lemhip_ctx *c, int slot, int field, void *host)
     for (int r0 = 0; r0 < D.h; r0 += band) {
         const int rows = std::min(band, D.h - r0);
         const long n = (long)D.w * rows;
-        const int g = grid1d(n);
-        void *to = direct ? c->stage : c->dstage;
-        int *oi = (int *)to;
-        double *od = (double *)to;
-        if (whole) k_pack<uint8_t, int><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const uint8_t *)src, 0, 1,
-                                                            kind == 2 ? c->mask : nullptr, oi);
-        else if (kind == 5 && !f64) k_pack<float2, double><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const float2 *)src, 0,
-                                                                              1, nullptr, od);
-        else if (kind == 1 || f64) k_pack<double, double><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const double *)src,
-                                                                             c->NP, ne, nullptr, od);
-        else k_pack<float, double><<<g, 256, 0, c->s>>>(c->W, D, r0, n, (const float *)src, c->NP, ne, nullptr, od);
+        k_pack<S, P><<<grid1d(n), 256, 0, c->s>>>(c->W, D, r0, n, (const S *)src, c->NP, ne, mask,
+                                                  (P *)(direct ? c->stage : c->dstage));
         LEM_LAUNCHED(c);
+        char *to = (char *)host + (size_t)D.w * r0 * ne * sizeof(O);
         if (!direct) {
-            LEM_TRY(copy_out(c, (const char *)c->dstage, (char *)host + (size_t)D.w * r0 * cell, n * cell));
+            LEM_TRY((copy_out<P, O>(c, (const char *)c->dstage, to, n * cell)));
             continue;
         }
         LEM_CHECK(c, hipStreamSynchronize(c->s));
-        memcpy(host, c->stage, total);
+        widen<P, O>((const char *)c->stage, to, n * ne);
     }
     return LEMHIP_OK;
+}
+
+static int slot_download(lemhip_ctx *c, int slot, int field, void *host)
+{
+    int kind = -1;
+    const void *src = field_ptr(c, field, &kind);
+    if (!src) { c->err = "unknown field"; return LEMHIP_E_ARG; }
+    DemDesc D;
+    LEM_TRY(slot_rect(c, slot, 2, &D));
+    LEM_CHECK(c, hipSetDevice(c->dev));
+    const bool f64 = c->prec == LEMHIP_FP64;
+    const int ne = kind == 4 ? 8 : 1;
+    if (kind == 2) return pack_out<uint8_t, int16_t, int>(c, D, src, ne, c->mask, host);
+    if (kind == 3) return pack_out<uint8_t, uint8_t, int>(c, D, src, ne, nullptr, host);
+    if (kind == 5 && !f64) return pack_out<float2, double, double>(c, D, src, ne, nullptr, host);
+    if (kind == 1 || f64) return pack_out<double, double, double>(c, D, src, ne, nullptr, host);
+    return pack_out<float, float, double>(c, D, src, ne, nullptr, host);
 }
 
 static int slot_upload(lemhip_ctx *c, int slot, int field, const void *host)
