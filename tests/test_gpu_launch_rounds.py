@@ -144,7 +144,7 @@ def test_time_of_looking_for_the_end_of_the_rounds():
     c.flow_direction(-1000)
     c.runoff()
     ms = {}
-    for batch in (16, 4, 16, 4, 16, 4):
+    for batch in (16, 4) * 6:
         c.set_tuning(dag_batch=batch)
         c.profile(True)
         c.flow_accum(-1000)
