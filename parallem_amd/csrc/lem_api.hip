@@ -622,28 +622,31 @@ static int rect_copy(lemhip_ctx *c, void *buf, void *base, int plane, size_t es,
     return LEMHIP_OK;
 }
 
-// Rows r0.. of rectangle D of a field in the order the host receives them:
-// row-major, `ne` values per cell (8 for Slopes, direction-minor), as narrow as
+// Values v0.. of rectangle D of a field in the order the host receives them:
+// row-major, NE values per cell (8 for Slopes, direction-minor), as narrow as
 // they are: directions in 16 bits, since nodata cells carry -9999 in the
 // reference's fd/SFD (newflow.cu:74-78), float pairs as their sum.
-// Bound by the host link where it writes to pinned memory, else by HBM.  Packing
-// on the device makes every download one contiguous copy: rows of an odd pitch
-// went through the strided copy's slow path (the directions of a 1201^2 DEM:
-// 18.8 ms, now 0.2 ms).
-template <typename S, typename P>
-__global__ void __launch_bounds__(256) k_pack(int W, DemDesc D, int r0, long n, const S *__restrict__ src, long plane,
-                                              int ne, const uint8_t *__restrict__ mask, P *__restrict__ out)
+// Bound by the host link: `out` is pinned host memory, whole lines to a wave.
+// No copy engine is involved: rows of an odd pitch went through the strided
+// copy's slow path (the directions of a 1201^2 DEM: 18.8 ms, now 0.2 ms), and
+// contiguous copies behind a packing kernel through an engine that the runtime
+// picks for a stream's first copy, 42 GB/s or 12 (an f64 field of 1024^2 0.36 or
+// 0.78 ms, now 0.33).
+template <int NE, typename S, typename P>
+__global__ void __launch_bounds__(256) k_pack(int W, DemDesc D, size_t v0, size_t n, const S *__restrict__ src,
+                                              long plane, const uint8_t *__restrict__ mask, P *__restrict__ out)
 {
-    for (long k = blockIdx.x * (long)blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
-        const int row = (int)(k / D.w), col = (int)(k % D.w);
-        const long i = (long)(D.y0 + r0 + row) * W + D.x0 + col;
+    for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t cell = (uint32_t)((v0 + v) / NE), d = (uint32_t)((v0 + v) % NE);
+        const uint32_t row = cell / (uint32_t)D.w, col = cell % (uint32_t)D.w;
+        const long i = (long)(D.y0 + row) * W + D.x0 + col;
         if constexpr (std::is_same_v<P, int16_t>) {
-            out[k] = mask[i] ? (P)src[i] : (P)-9999;
+            out[v] = mask[i] ? (P)src[i] : (P)-9999;
         } else if constexpr (std::is_same_v<S, float2>) {
-            const float2 v = src[i];
-            out[k] = (double)v.x + (double)v.y;
+            const float2 p = src[i];
+            out[v] = (double)p.x + (double)p.y;
         } else {
-            for (int d = 0; d < ne; d++) out[ne * k + d] = src[d * plane + i];
+            out[v] = src[d * plane + i];
         }
     }
 }
@@ -663,38 +666,52 @@ template <typename P, typename O> static void widen(const char *from, char *to, 
     }
 }
 
-// Device staging to caller memory, on DL_THREADS threads, each taking every DL_THREADS-th chunk through its own two pinned
-// chunks: the next chunk's transfer overlaps the copy into the caller's pages
-// (one thread's page faults and copy took 10 of the 12.2 ms of a 134 MB field
-// and the transfer 2.5; now 4.0 ms, 12.1 ms for 459 MB; 1 to 4 MB chunks are
-// alike, 8 threads slower: 4.6 ms).  The pinned staging stays at 16 MB however
-// large the DEM.
+// A field of a DEM to caller memory, packed as P from S and widened to O.
+// Up to DL_DIRECT bytes, widened to twice that at most, in one piece.  More on
+// DL_THREADS threads, each taking every DL_THREADS-th chunk through its own two
+// pinned chunks: the next chunk's packing overlaps the copy into the caller's
+// pages (one thread's page faults and copy took 10 of the 12.2 ms of a 134 MB
+// field and the transfer 2.5; now 3.9 ms, 12.1 ms for 459 MB; 1 to 4 MB chunks
+// are alike, 8 threads slower).  A float field of 1024^2 takes 0.25 ms in
+// one piece, 0.52 on several threads; the mask of 2048^2, 16 MB widened, 0.46 and
+// 0.31.  The pinned staging stays at 16 MB however large the DEM.
 #define DL_CHUNK ((size_t)2 << 20)
 #define DL_DIRECT ((size_t)4 << 20)
 #define DL_THREADS 4
 static_assert(2 * DL_THREADS <= sizeof(lemhip_ctx::dl_ev) / sizeof(hipEvent_t), "one event per pinned chunk");
-template <typename P, typename O> static int copy_out(lemhip_ctx *c, const char *dev, char *host, size_t bytes)
+template <int NE, typename S, typename P, typename O>
+static int pack_out(lemhip_ctx *c, const DemDesc &D, const void *src, const uint8_t *mask, void *host)
 {
+    const size_t values = (size_t)NE * D.w * D.h;
+    auto pack = [=](size_t v0, size_t n, void *to) -> hipError_t {
+        k_pack<NE, S, P><<<grid1d((long)n), 256, 0, c->s>>>(c->W, D, v0, n, (const S *)src, c->NP, mask, (P *)to);
+        return hipGetLastError();
+    };
+    if (values * sizeof(P) <= DL_DIRECT && values * sizeof(O) <= 2 * DL_DIRECT) {
+        LEM_TRY(stage_reserve(c, values * sizeof(P)));
+        LEM_CHECK(c, pack(0, values, c->stage));
+        LEM_CHECK(c, hipStreamSynchronize(c->s));
+        widen<P, O>((const char *)c->stage, (char *)host, values);
+        return LEMHIP_OK;
+    }
     LEM_TRY(stage_reserve(c, 2 * (size_t)DL_THREADS * DL_CHUNK));
     for (hipEvent_t &e : c->dl_ev)
         if (!e) LEM_CHECK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    const size_t nch = (bytes + DL_CHUNK - 1) / DL_CHUNK, nt = std::min(nch, (size_t)DL_THREADS);
+    const size_t per = DL_CHUNK / sizeof(P), nch = (values + per - 1) / per, nt = std::min(nch, (size_t)DL_THREADS);
     auto part = [=](size_t t) -> hipError_t {
         hipError_t e = hipSetDevice(c->dev);
         auto fetch = [&](size_t k, size_t buf) {   // chunk k into this thread's pinned chunk
             if (e != hipSuccess || k >= nch) return;
-            const size_t off = k * DL_CHUNK, len = std::min((size_t)DL_CHUNK, bytes - off);
-            e = hipMemcpyAsync((char *)c->stage + buf * DL_CHUNK, dev + off, len, hipMemcpyDeviceToHost, c->s);
+            e = pack(k * per, std::min(per, values - k * per), (char *)c->stage + buf * DL_CHUNK);
             if (e == hipSuccess) e = hipEventRecord(c->dl_ev[buf], c->s);
         };
         fetch(t, 2 * t);
         for (size_t k = t, j = 0; k < nch && e == hipSuccess; k += nt, j ^= 1) {
             fetch(k + nt, 2 * t + (j ^ 1));
             if (e == hipSuccess) e = hipEventSynchronize(c->dl_ev[2 * t + j]);
-            const size_t off = k * DL_CHUNK;
             if (e == hipSuccess)
-                widen<P, O>((char *)c->stage + (2 * t + j) * DL_CHUNK, host + off / sizeof(P) * sizeof(O),
-                            std::min((size_t)DL_CHUNK, bytes - off) / sizeof(P));
+                widen<P, O>((const char *)c->stage + (2 * t + j) * DL_CHUNK, (char *)host + k * per * sizeof(O),
+                            std::min(per, values - k * per));
         }
         return e;
     };
@@ -712,45 +729,8 @@ template <typename P, typename O> static int copy_out(lemhip_ctx *c, const char 
         if (inl[t]) rc[t] = part(t);
     for (std::thread &t : th)
         if (t.joinable()) t.join();
-    LEM_CHECK(c, hipStreamSynchronize(c->s));   // no transfer is left writing the pinned chunks
+    LEM_CHECK(c, hipStreamSynchronize(c->s));   // no kernel is left writing the pinned chunks
     for (hipError_t e : rc) LEM_CHECK(c, e);
-    return LEMHIP_OK;
-}
-
-// field src of S, `ne` values per cell, packed as P and widened to O
-template <typename S, typename P, typename O>
-static int pack_out(lemhip_ctx *c, const DemDesc &D, const void *src, int ne, const uint8_t *mask, void *host)
-{
-    // up to DL_DIRECT bytes, widened to twice that at most, are packed straight
-    // into pinned host memory (a copy behind the kernel makes a 96^2 field's 17 us
-    // 28, a 512^2 one's 125 us 140; a float field of 1024^2 0.25 ms, 0.52 on
-    // several threads; the mask of 2048^2, 16 MB widened, 0.46 and 0.31).
-    // Otherwise the staging that initialised the slot holds 8 bytes per cell of
-    // its DEM, and Slopes go in bands of rows.
-    const size_t cell = ne * sizeof(P), total = cell * D.w * D.h;
-    const bool direct = total <= DL_DIRECT && total / sizeof(P) * sizeof(O) <= 2 * DL_DIRECT;
-    int band = D.h;
-    if (direct) {
-        LEM_TRY(stage_reserve(c, total));
-    } else {
-        LEM_TRY(dstage_reserve(c, (size_t)D.w * D.h * 8));
-        band = (int)std::max((size_t)1, std::min((size_t)D.h, c->dstage_bytes / (cell * D.w)));
-        LEM_TRY(dstage_reserve(c, cell * D.w * band));
-    }
-    for (int r0 = 0; r0 < D.h; r0 += band) {
-        const int rows = std::min(band, D.h - r0);
-        const long n = (long)D.w * rows;
-        k_pack<S, P><<<grid1d(n), 256, 0, c->s>>>(c->W, D, r0, n, (const S *)src, c->NP, ne, mask,
-                                                  (P *)(direct ? c->stage : c->dstage));
-        LEM_LAUNCHED(c);
-        char *to = (char *)host + (size_t)D.w * r0 * ne * sizeof(O);
-        if (!direct) {
-            LEM_TRY((copy_out<P, O>(c, (const char *)c->dstage, to, n * cell)));
-            continue;
-        }
-        LEM_CHECK(c, hipStreamSynchronize(c->s));
-        widen<P, O>((const char *)c->stage, to, n * ne);
-    }
     return LEMHIP_OK;
 }
 
@@ -763,12 +743,13 @@ static int slot_download(lemhip_ctx *c, int slot, int field, void *host)
     LEM_TRY(slot_rect(c, slot, 2, &D));
     LEM_CHECK(c, hipSetDevice(c->dev));
     const bool f64 = c->prec == LEMHIP_FP64;
-    const int ne = kind == 4 ? 8 : 1;
-    if (kind == 2) return pack_out<uint8_t, int16_t, int>(c, D, src, ne, c->mask, host);
-    if (kind == 3) return pack_out<uint8_t, uint8_t, int>(c, D, src, ne, nullptr, host);
-    if (kind == 5 && !f64) return pack_out<float2, double, double>(c, D, src, ne, nullptr, host);
-    if (kind == 1 || f64) return pack_out<double, double, double>(c, D, src, ne, nullptr, host);
-    return pack_out<float, float, double>(c, D, src, ne, nullptr, host);
+    if (kind == 2) return pack_out<1, uint8_t, int16_t, int>(c, D, src, c->mask, host);
+    if (kind == 3) return pack_out<1, uint8_t, uint8_t, int>(c, D, src, nullptr, host);
+    if (kind == 4 && f64) return pack_out<8, double, double, double>(c, D, src, nullptr, host);
+    if (kind == 4) return pack_out<8, float, float, double>(c, D, src, nullptr, host);
+    if (kind == 5 && !f64) return pack_out<1, float2, double, double>(c, D, src, nullptr, host);
+    if (kind == 1 || f64) return pack_out<1, double, double, double>(c, D, src, nullptr, host);
+    return pack_out<1, float, float, double>(c, D, src, nullptr, host);
 }
 
 static int slot_upload(lemhip_ctx *c, int slot, int field, const void *host)
